@@ -23,8 +23,11 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", f"--offload-arch={A
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           f"-I{os.path.join(HERE, '..', 'include')}"]
 
-SOURCES = ["p3_kernel_fp64.hip", "p3_kernel_mixed.hip", "p3x_api.hip", "p3x_server.hip",
-           "p3x_process.hip", "p3_tables.cpp", "p3_table_gen.hip"]
+# Translation units: (source, lanes per column of its sedimentation launches or 0).
+# The sedimentation launches take most of the time: a unit per precision and
+# lanes count, the longest first.
+SOURCES = [(f"p3_kernel_{prec}.hip", lpc) for prec in ("fp64", "mixed") for lpc in (64, 32, 16, 0)] + [
+    (src, 0) for src in ("p3x_api.hip", "p3x_server.hip", "p3x_process.hip", "p3_tables.cpp", "p3_table_gen.hip")]
 
 # Extra flags per translation unit.  The mixed-precision form may use the
 # hardware-backed FP32 division, square root and transcendental sequences
@@ -35,9 +38,11 @@ FILE_FLAGS: dict[str, list[str]] = {
 }
 
 
-def _compile(src: str) -> str:
-    out = os.path.join(OBJ, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC] + COMMON + FILE_FLAGS.get(src, []) + ["-c", os.path.join(CSRC, src), "-o", out]
+def _compile(unit: tuple[str, int]) -> str:
+    src, lpc = unit
+    out = os.path.join(OBJ, os.path.splitext(src)[0] + (f"_sed{lpc}" if lpc else "") + ".o")
+    cmd = [HIPCC] + COMMON + FILE_FLAGS.get(src, []) + ([f"-DP3_SED_LPC={lpc}"] if lpc else []) + [
+        "-c", os.path.join(CSRC, src), "-o", out]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed on {src}:\n{r.stderr[-4000:]}")

@@ -91,7 +91,12 @@ struct KParams {
 };
 
 __host__ __device__ __forceinline__ double exner_function(double pres) {  // PhysicsFunctions, p^(Rd/cp)
-  return p3m_pow(pres / P0, Rair * INV_CP);
+  return p3m_pow(p3m_div(pres, P0), Rair * INV_CP);
+}
+
+// Air density of a layer (dpres / dz / g), as every kernel forms it.
+__device__ __forceinline__ double air_density(double dpres, double dz) {
+  return p3m_div(p3m_div(dpres, dz), gravit);
 }
 
 constexpr int kMaxSubsteps = 100000;
@@ -116,17 +121,20 @@ __device__ __forceinline__ int part1_level(const KParams& p, int k, int i, unsig
     const double dp = a.dp_wet[x], dp_dry = p.dpres[x];
     const double c1 = -1.0 + 1.0 / ep_2;  // calculate_dz with the wet qv's virtual temperature
     const double T_virtual = T * (1.0 + c1 * p.qv[x]);
-    dz = (Rair / gravit) * dp * T_virtual / pmid;
+    dz = p3m_div((Rair / gravit) * dp * T_virtual, pmid);
     a.dz[x] = dz;
     // wet -> dry mixing ratios (calculate_drymmr_from_wetmmr_dp_based)
-    qc = p.qc[x] * dp / dp_dry; nc = p.nc[x] * dp / dp_dry; qr = p.qr[x] * dp / dp_dry;
-    nr = p.nr[x] * dp / dp_dry; qi = p.qi[x] * dp / dp_dry; ni = p.ni[x] * dp / dp_dry;
-    qm = p.qm[x] * dp / dp_dry; bm = p.bm[x] * dp / dp_dry;
-    qv = p.qv[x] * dp / dp_dry;
-    a.qv_prev[x] = a.qv_prev[x] * dp / dp_dry;
-    inv_exner = 1.0 / exner_function(pmid);
+    const double rdry = p3m_recip(dp_dry);
+    auto to_dry = [&](double q) { return p3m_div_y(q * dp, dp_dry, rdry); };
+    qc = to_dry(p.qc[x]); nc = to_dry(p.nc[x]); qr = to_dry(p.qr[x]);
+    nr = to_dry(p.nr[x]); qi = to_dry(p.qi[x]); ni = to_dry(p.ni[x]);
+    qm = to_dry(p.qm[x]); bm = to_dry(p.bm[x]);
+    qv = to_dry(p.qv[x]);
+    a.qv_prev[x] = to_dry(a.qv_prev[x]);
+    const double ex = exner_function(pmid), rex = p3m_recip(ex);
+    inv_exner = p3m_div_y(1.0, ex, rex);
     a.inv_exner[x] = inv_exner;
-    th = T / exner_function(pmid);
+    th = p3m_div_y(T, ex, rex);
     // cloud fractions with the 1e-4 floor and the maximum-overlap rain fraction
     cfl = cft > 0.0001 ? cft : 0.0001;
     a.cld_frac_l[x] = cfl;
@@ -150,21 +158,21 @@ __device__ __forceinline__ int part1_level(const KParams& p, int k, int i, unsig
   // is not stored again (with the pre-amble every field changes to dry)
   const double in[10] = {qc, nc, qr, nr, qi, ni, qm, bm, qv, th};
   qv = vmax(qv, 0.0);
-  const double exner = 1 / inv_exner;
+  const double exner = p3m_div(1.0, inv_exner);
   const double pres = p.pres[x];
   double T_atm = th * exner;
-  const double rho = p.dpres[x] / dz / gravit;
-  const double inv_rho = 1 / rho;
-  const double qv_sat_l = qv_sat_dry(T_atm, pres, false, err);
-  const double qv_sat_i = qv_sat_dry(T_atm, pres, true, err);
-  const double qv_supersat_i = qv / qv_sat_i - 1;
+  const double rho = air_density(p.dpres[x], dz);
+  const double inv_rho = p3m_div(1.0, rho);
+  double qv_sat_l, qv_sat_i;
+  qv_sat_dry_both(T_atm, pres, qv_sat_l, qv_sat_i, err);
+  const double qv_supersat_i = p3m_div(qv, qv_sat_i) - 1;
   double rhofacr, rhofaci, acn;
   {
     const R ir = R(inv_rho), Tr = R(T_atm);
     rhofacr = double(m_pow(R(RHO_1000MB) * ir, R(.54)));
     rhofaci = double(m_pow(R(RHO_600MB) * ir, R(.54)));
-    const R dum = R(1.496e-6) * m_pow(Tr, R(1.5)) / (Tr + R(120));
-    acn = double(R(gravit) * R(RHO_H2O) / (R(18) * dum));
+    const R dum = m_div(R(1.496e-6) * m_pow(Tr, R(1.5)), Tr + R(120));
+    acn = double(m_div(R(gravit) * R(RHO_H2O), R(18) * dum));
   }
   if (T_atm < T_zerodegc && qv_supersat_i >= -0.05) flags |= 1;
 
@@ -392,14 +400,14 @@ __device__ __forceinline__ void part2_tile(const KParams& p, int tile) {
       s.nc = p.nc[x]; s.nr = p.nr[x]; s.qm = p.qm[x]; s.ni = p.ni[x]; s.bm = p.bm[x];
       s.qv = p.qv[x]; s.th = p.th[x];
       s.pres = p.pres[x];
-      s.rho = p.dpres[x] / p.dz[x] / gravit;
-      s.inv_rho = 1 / s.rho;
+      s.rho = air_density(p.dpres[x], p.dz[x]);
+      s.inv_rho = p3m_div(1.0, s.rho);
       s.qv_sat_l = scr(SC_QVSL);
       s.qv_sat_i = scr(SC_QVSI);
       s.rhofaci = scr(SC_RHOFACI);
       s.acn = scr(SC_ACN);
       s.cfl = p.cld_frac_l[x]; s.cfr = p.cld_frac_r[x]; s.cfi = p.cld_frac_i[x];
-      s.icfl = 1 / s.cfl; s.icfr = 1 / s.cfr; s.icfi = 1 / s.cfi;
+      s.icfl = p3m_div(1.0, s.cfl); s.icfr = p3m_div(1.0, s.cfr); s.icfi = p3m_div(1.0, s.cfi);
       s.inv_exner = p.inv_exner[x];
       s.qv_prev = p.qv_prev[x]; s.t_prev = p.t_prev[x];
       s.ni_activated = p.ni_activated[x];

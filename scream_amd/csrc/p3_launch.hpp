@@ -66,6 +66,13 @@ struct SedClass {
   int nsets;
   int grid;             // blocks (one per virtual block, or a persistent grid)
 };
+// The sedimentation launches on one lanes-per-column count.
+struct SedLaunch {
+  hipError_t (*single)(const KParams& p, int group, int L, hipStream_t s);  // one species group
+  hipError_t (*fused)(const KParams& p, int L, hipStream_t s);              // both groups, one launch
+  hipError_t (*batch)(const SedClass& c, hipStream_t s);
+  hipError_t (*occupancy)(int L, int* blocks);  // resident blocks per CU of the batched kernels
+};
 struct BatchPlan {
   Shape shape;
   const KParams* sets;  // device array, all sets (part 1 and part 2 launches)

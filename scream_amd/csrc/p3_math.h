@@ -41,20 +41,61 @@ P3M_FN double p3m_from_bits(uint64_t u) { double x; __builtin_memcpy(&x, &u, 8);
 P3M_FN double p3m_inf(void) { return p3m_from_bits(0x7ff0000000000000ULL); }
 P3M_FN double p3m_nan(void) { return p3m_from_bits(0x7ff8000000000000ULL); }
 
-/* x * 2^k for x in [0.5, 2) and any k that keeps the result finite or subnormal */
+#if defined(__HIP_DEVICE_COMPILE__)
+#define P3M_DEVICE 1
+#else
+#define P3M_DEVICE 0
+#endif
+
+/* Division.  hipcc's FP64 a / b is eleven VALU instructions of which two
+ * (v_div_scale) and the condition code they leave only serve operands near the
+ * ends of the exponent range.  Without that scaling the same steps -- v_rcp,
+ * two Newton steps y <- y + y (1 - b y), q = a y, q + y (a - b q) -- give the
+ * same bits whenever b, a / b and 1 / b are normal, |a| >= 2^-969 and
+ * |a / b| < 2^768: the scaling is then the identity.  A quarter-rate v_rcp
+ * included, a division measured 65 cycles per wavefront on MI355X against 52
+ * here and 20 for one more division by the same b (p3m_div_y).
+ * v_div_fixup keeps the results for zero, infinite and NaN operands; the _n form
+ * leaves it out where the operands are finite and b is not zero.  On the CPU
+ * all of these are a / b. */
+#if P3M_DEVICE
+P3M_FN double p3m_recip(double b) { /* the refined 1/b of the division, for p3m_div_y */
+  double y = __builtin_amdgcn_rcp(b);
+  y = fma(y, fma(-b, y, 1.0), y);
+  return fma(y, fma(-b, y, 1.0), y);
+}
+P3M_FN double p3m_div_yn(double a, double b, double y) {
+  const double q = a * y;
+  return fma(fma(-b, q, a), y, q);
+}
+P3M_FN double p3m_div_y(double a, double b, double y) {
+  return __builtin_amdgcn_div_fixup(p3m_div_yn(a, b, y), b, a);
+}
+#else
+P3M_FN double p3m_recip(double b) { return 1.0 / b; }
+P3M_FN double p3m_div_yn(double a, double b, double y) { (void)y; return a / b; }
+P3M_FN double p3m_div_y(double a, double b, double y) { (void)y; return a / b; }
+#endif
+P3M_FN double p3m_div(double a, double b) { return p3m_div_y(a, b, p3m_recip(b)); }
+P3M_FN double p3m_div_n(double a, double b) { return p3m_div_yn(a, b, p3m_recip(b)); }
+
+/* x * 2^k for x in [0.5, 2), one rounding where the result is subnormal (the
+ * device's v_ldexp rounds the same) */
 P3M_FN double p3m_scale2(double x, int k) {
+#if P3M_DEVICE
+  return __builtin_amdgcn_ldexp(x, k);
+#else
   if (k > 1023) { x *= p3m_from_bits((uint64_t)(1023 + 1023) << 52); k -= 1023; }
   if (k < -1022) { x *= p3m_from_bits((uint64_t)(-1000 + 1023) << 52); k += 1000;
                    if (k < -1022) { x *= p3m_from_bits((uint64_t)(-1000 + 1023) << 52); k += 1000; } }
   return x * p3m_from_bits((uint64_t)(k + 1023) << 52);
+#endif
 }
 
-/* exp: Cody-Waite reduction x = k ln2 + r, |r| <= ln2/2, then the Taylor
- * series of e^r to r^13 (truncation < 1e-17), evaluated with fma. */
-P3M_FN double p3m_exp(double x) {
-  if (!(x == x)) return x;
-  if (x > 709.782712893384) return p3m_inf();
-  if (x < -745.1332191019412) return 0.0;
+/* exp of a finite x in about [-746, 710] (NaN gives NaN): Cody-Waite reduction
+ * x = k ln2 + r, |r| <= ln2/2, then the Taylor series of e^r to r^13
+ * (truncation < 1e-17), evaluated with fma. */
+P3M_FN double p3m_exp_core(double x) {
   const double t = x * P3M_INVLN2;
   const int k = (int)(t + (t >= 0 ? 0.5 : -0.5));
   const double kd = (double)k;
@@ -77,26 +118,58 @@ P3M_FN double p3m_exp(double x) {
   return p3m_scale2(p, k);
 }
 
-/* log as an unevaluated sum hi + lo.  Reduction x = 2^e m, m in (sqrt(1/2), sqrt(2)],
+P3M_FN double p3m_exp(double x) {
+#if P3M_DEVICE
+  /* the range ends by selects: branches would end the basic blocks that the
+   * compiler schedules across (the float to int conversion saturates) */
+  double e = p3m_exp_core(x);
+  e = x > 709.782712893384 ? p3m_inf() : e;
+  return x < -745.1332191019412 ? 0.0 : e;
+#else
+  if (!(x == x)) return x;
+  if (x > 709.782712893384) return p3m_inf();
+  if (x < -745.1332191019412) return 0.0;
+  return p3m_exp_core(x);
+#endif
+}
+
+/* True for positive, normal or subnormal, finite x. */
+P3M_FN int p3m_positive(double x) {
+#if P3M_DEVICE
+  return __builtin_amdgcn_class(x, 0x180);
+#else
+  return x > 0 && x < p3m_inf();
+#endif
+}
+
+/* x = 2^e m with m in (sqrt(1/2), sqrt(2)], for positive finite x */
+P3M_FN double p3m_split(double x, int* e) {
+#if P3M_DEVICE
+  const double m = __builtin_amdgcn_frexp_mant(x); /* [1/2, 1), subnormal x too */
+  const int up = m > 0.5 * P3M_SQRT2 ? 0 : 1;
+  *e = __builtin_amdgcn_frexp_exp(x) - up;
+  return __builtin_amdgcn_ldexp(m, up);
+#else
+  uint64_t u = p3m_bits(x);
+  int k = 0;
+  if (u < 0x0010000000000000ULL) { x *= 18014398509481984.0; u = p3m_bits(x); k = -54; } /* subnormal */
+  k += (int)(u >> 52) - 1023;
+  double m = p3m_from_bits((u & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
+  if (m > P3M_SQRT2) { m *= 0.5; k += 1; }
+  *e = k;
+  return m;
+#endif
+}
+
+/* log of a positive finite x as an unevaluated sum hi + lo.  x = 2^e m,
  * f = m - 1, s = f/(2+f), log m = 2 atanh s = f - f^2/2 + s (f^2/2 + R) with
  * R = sum_{k>=1} 2 s^(2k)/(2k+1) (the formulation of Sun's fdlibm __ieee754_log,
  * here with the exact series coefficients up to s^22). */
-P3M_FN void p3m_log_dd(double x, double* hi, double* lo) {
-  uint64_t u = p3m_bits(x);
-  int e = 0;
-  /* One unsigned compare separates the positive normal finite arguments (the
-   * only ones P3 passes) from zero, subnormals, negatives, infinities and NaN. */
-  if (u - 0x0010000000000000ULL >= 0x7fe0000000000000ULL) {
-    if (!(x == x) || x < 0) { *hi = p3m_nan(); *lo = 0; return; }
-    if (x == 0) { *hi = -p3m_inf(); *lo = 0; return; }
-    if (u >= 0x7ff0000000000000ULL) { *hi = x; *lo = 0; return; }
-    x *= 18014398509481984.0; u = p3m_bits(x); e = -54;  /* subnormal */
-  }
-  e += (int)(u >> 52) - 1023;
-  double m = p3m_from_bits((u & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
-  if (m > P3M_SQRT2) { m *= 0.5; e += 1; }
+P3M_FN void p3m_log_core(double x, double* hi, double* lo) {
+  int e;
+  const double m = p3m_split(x, &e);
   const double f = m - 1.0;
-  const double s = f / (2.0 + f);
+  const double s = p3m_div_n(f, 2.0 + f);
   const double z = s * s;
   double R = 2.0 / 23.0;
   R = fma(R, z, 2.0 / 21.0);
@@ -118,59 +191,85 @@ P3M_FN void p3m_log_dd(double x, double* hi, double* lo) {
   *hi = h;
   *lo = (A - h) + B;  /* |A| >= |B| whenever A != 0 */
 }
+/* log of zero, an infinity, NaN or a negative number */
+P3M_FN double p3m_log_special(double x) {
+  if (!(x == x) || x < 0) return p3m_nan();
+  return x == 0 ? -p3m_inf() : x;
+}
 
 P3M_FN double p3m_log(double x) {
   double h, l;
-  p3m_log_dd(x, &h, &l);
+  if (!p3m_positive(x)) return p3m_log_special(x);
+  p3m_log_core(x, &h, &l);
   return h + l;
 }
 
 P3M_FN double p3m_log10(double x) {
   double h, l;
-  p3m_log_dd(x, &h, &l);
-  if (!(h == h) || h == p3m_inf() || h == -p3m_inf()) return h;
+  if (!p3m_positive(x)) return p3m_log_special(x);
+  p3m_log_core(x, &h, &l);
   return fma(h, P3M_INVLN10_HI, fma(h, P3M_INVLN10_LO, l * P3M_INVLN10_HI));
 }
 
-/* pow for the arguments P3 uses (x >= 0): exp(y log x) with log x in
- * double-double and the product's rounding error carried into exp.  A negative
- * base with an integral exponent is |x|^y with the sign of (-1)^y.  (No
- * recursion, so that the device compiler can inline it everywhere.) */
-P3M_FN double p3m_pow(double x, double y) {
-  if (y == 0.0) return 1.0;
-  if (!(x == x) || !(y == y)) return x + y;
-  if (x == 1.0) return 1.0;
-  if (y == 1.0) return x;
-  if (y == 2.0) return x * x;
-  double sgn = 1.0;
-  if (x < 0) {
-    const double yi = (double)(int64_t)y;
-    if (yi != y || y > 9007199254740992.0 || y < -9007199254740992.0) return p3m_nan();
-    sgn = ((int64_t)y & 1) ? -1.0 : 1.0;
-    x = -x;
-    if (x == 1.0) return sgn;
-  }
-  if (x == 0.0) return y > 0 ? 0.0 : p3m_inf();
-  if (p3m_bits(x) == 0x7ff0000000000000ULL) return sgn * (y > 0 ? x : 0.0);
-  double lh, ll;
-  p3m_log_dd(x, &lh, &ll);
+/* x^y from log x = lh + ll of a positive finite x: exp(y log x), the rounding
+ * error of the product carried into exp. */
+P3M_FN double p3m_pow_log(double lh, double ll, double y) {
   const double z = y * lh;
   const double zl = fma(y, lh, -z) + y * ll;
-  if (z > 709.8) return sgn * p3m_inf();
-  if (z < -745.2) return sgn * 0.0;
+#if P3M_DEVICE
+  const double e = p3m_exp_core(z);
+  double r = fma(e, zl, e);
+  r = z > 709.8 ? p3m_inf() : r;
+  return z < -745.2 ? 0.0 : r;
+#else
+  if (z > 709.8) return p3m_inf();
+  if (z < -745.2) return 0.0;
   const double e = p3m_exp(z);
-  return sgn * fma(e, zl, e);
+  return fma(e, zl, e);
+#endif
+}
+
+/* pow for the arguments P3 uses (x >= 0): exp(y log x) with log x in
+ * double-double.  A negative base with an integral exponent is |x|^y with the
+ * sign of (-1)^y.  (No recursion, so that the device compiler can inline it
+ * everywhere; one branch covers every argument that P3 does not pass.) */
+P3M_FN double p3m_pow(double x, double y) {
+  int neg = 0;
+  if (y == 0.0) return 1.0;
+  if (y == 1.0) return x;
+  if (y == 2.0) return x * x;
+  if (!p3m_positive(x) || !(y == y) || x == 1.0) {
+    if (!(x == x) || !(y == y)) return x + y;
+    if (x == 1.0) return 1.0;
+    if (x < 0) {
+      const double yi = (y > 9007199254740992.0 || y < -9007199254740992.0) ? 0.0 : (double)(int64_t)y;
+      if (yi != y) return p3m_nan();
+      neg = (int)((int64_t)y & 1);
+      x = -x;
+    }
+    if (x == 0.0) return y > 0 ? 0.0 : p3m_inf();
+    if (p3m_bits(x) == 0x7ff0000000000000ULL) {
+      const double r = y > 0 ? x : 0.0;
+      return neg ? -r : r;
+    }
+  }
+  double lh, ll;
+  p3m_log_core(x, &lh, &ll);
+  const double r = p3m_pow_log(lh, ll, y);
+  return neg ? -r : r;
 }
 
 /* cbrt: inverse cube root y ~ a^(-1/3) from the exponent bits, refined by the
  * division-free Newton iteration y <- y + y (1 - a y^3)/3, then one Newton step
  * on c^3 = a for c = a y^2 with the residual c^3 - a formed exactly with fma. */
 P3M_FN double p3m_cbrt(double x) {
-  if (x == 0.0 || !(x == x) || p3m_bits(x < 0 ? -x : x) >= 0x7ff0000000000000ULL) return x;
-  const double sgn = x < 0 ? -1.0 : 1.0;
-  double a = x < 0 ? -x : x;
-  double post = 1.0;
-  if (a < 2.2250738585072014e-308) { a *= 18014398509481984.0; post = 1.0 / 262144.0; }
+  double sgn = 1.0, a = x, post = 1.0;
+  if (!(x >= 2.2250738585072014e-308 && x < p3m_inf())) { /* not positive, normal and finite */
+    if (x == 0.0 || !(x == x) || p3m_bits(x < 0 ? -x : x) >= 0x7ff0000000000000ULL) return x;
+    sgn = x < 0 ? -1.0 : 1.0;
+    a = x < 0 ? -x : x;
+    if (a < 2.2250738585072014e-308) { a *= 18014398509481984.0; post = 1.0 / 262144.0; }
+  }
   double y = p3m_from_bits(0x553ef0ff289dd796ULL - p3m_bits(a) / 3);
   for (int it = 0; it < 5; ++it) {
     const double y3 = y * y * y;
@@ -182,7 +281,7 @@ P3M_FN double p3m_cbrt(double x) {
   const double c3 = c2 * c;
   const double e3 = fma(c2, c, -c3) + e2 * c;
   const double r = (c3 - a) + e3;
-  c = c - r / (3.0 * c2);
+  c = c - p3m_div_n(r, 3.0 * c2);
   return sgn * c * post;
 }
 
@@ -219,7 +318,7 @@ P3M_FN double p3m_tanh(double x) {
   if (ax > 22.0) return x < 0 ? -1.0 : 1.0;
   if (ax < 3.725290298461914e-09) return x;
   const double e = p3m_expm1(2.0 * ax);
-  const double t = e / (e + 2.0);
+  const double t = p3m_div_n(e, e + 2.0);
   return x < 0 ? -t : t;
 }
 
@@ -229,14 +328,7 @@ P3M_FN double p3m_tanh(double x) {
  * Press et al. / Godfrey), Gamma(z+1) = sqrt(2 pi) t^(z+1/2) e^(-t) A(z),
  * t = z + 7.5, with the partial-fraction sum A taken over one common
  * denominator so that a single division is needed. */
-P3M_FN double p3m_tgamma(double x) {
-  if (!(x == x)) return x;
-  if (x <= 0.0) return p3m_nan();
-  if (x > 171.6) return p3m_inf();
-  double prod = 1.0, div = 1.0;
-  if (x < 1.0) { div = x; x = x + 1.0; }
-  while (x >= 2.0) { x = x - 1.0; prod *= x; }
-  const double z = x - 1.0;
+P3M_FN double p3m_gamma_1_2(double z) { /* Gamma(1 + z), z in [0, 1) */
   const double p0 = 0.99999999999980993, p1 = 676.5203681218851, p2 = -1259.1392167224028,
                p3 = 771.32342877765313, p4 = -176.61502916214059, p5 = 12.507343278686905,
                p6 = -0.13857109526572012, p7 = 9.9843695780195716e-6, p8 = 1.5056327351493116e-7;
@@ -253,10 +345,10 @@ P3M_FN double p3m_tgamma(double x) {
   num = fma(p6, q1234 * d5 * q78, num);
   num = fma(p7, q1234 * q56 * d8, num);
   num = fma(p8, q1234 * q56 * d7, num);
-  const double A = p0 + num / (q1234 * q5678);
+  const double A = p0 + p3m_div_n(num, q1234 * q5678);
   const double t = z + 7.5;
   double lh, ll;
-  p3m_log_dd(t, &lh, &ll);
+  p3m_log_core(t, &lh, &ll);
   const double zh = z + 0.5;
   /* w + wl = zh*(lh+ll) - t: exact product error by fma, exact sum error by
    * Fast2Sum (|t| > |zh*lh| on [1, 2)) */
@@ -264,9 +356,32 @@ P3M_FN double p3m_tgamma(double x) {
   const double pl = fma(zh, lh, -ph);
   const double w = ph - t;
   const double wl = (ph - (w + t)) + pl + zh * ll;
-  const double e = p3m_exp(w);
-  const double g = P3M_SQRT2PI * fma(e, wl, e) * A;
-  return g * prod / div;
+  const double e = p3m_exp_core(w);
+  return P3M_SQRT2PI * fma(e, wl, e) * A;
+}
+P3M_FN double p3m_tgamma(double x) {
+  double div = 1.0;
+  if (!(x >= 1.0 && x <= 171.6)) {
+    if (!(x == x)) return x;
+    if (x <= 0.0) return p3m_nan();
+    if (x > 171.6) return p3m_inf();
+    div = x;
+    x = x + 1.0;
+  }
+  /* x - 1, x - 2, ... are exact, so the reduced argument is known at once and
+   * the chain of products runs beside the Lanczos sum.  Four factors a turn,
+   * those past the lane's last one being 1 (a product with 1 is exact). */
+  const int n = (int)x - 1;
+  double prod = 1.0;
+  for (int k = 1; k <= n; k += 4) {
+    const double y = x - (double)k;
+    prod *= y;
+    prod *= k + 1 <= n ? y - 1.0 : 1.0;
+    prod *= k + 2 <= n ? y - 2.0 : 1.0;
+    prod *= k + 3 <= n ? y - 3.0 : 1.0;
+  }
+  const double g = p3m_gamma_1_2(x - (double)n - 1.0) * prod;
+  return div == 1.0 ? g : g / div;
 }
 
 #endif /* P3_MATH_H */

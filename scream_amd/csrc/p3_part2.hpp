@@ -54,10 +54,12 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     const R Tr = R(T_atm), rhor = R(rho), rhofaci = R(s.rhofaci);
     const R dT_melt = R(T_atm - Tmelt);  // FP64 difference (exact in the FP64 form)
     // get_time_space_phys_variables, P3I/p3_get_time_space_phys_variables_impl.hpp:10-46
-    const R mu = R(1.496e-6) * m_pow(Tr, R(1.5)) / (Tr + R(120));
-    const R dv = R(8.794e-5) * m_pow(Tr, R(1.81)) / R(pres);
-    const R sc = mu / (rhor * dv);
-    const R dum_t = R(1) / (R(RV) * (Tr * Tr));
+    R T15, T181;  // T^1.5, T^1.81
+    pow_15_181(Tr, T15, T181);
+    const R mu = m_div(R(1.496e-6) * T15, Tr + R(120));
+    const R dv = m_div(R(8.794e-5) * T181, R(pres));
+    const R sc = m_div(mu, rhor * dv);
+    const R dum_t = m_div(R(1), R(RV) * (Tr * Tr));
     const R dqsdt = R(latvap) * R(s.qv_sat_l) * dum_t;
     const R dqsidt = R(latvap + latice) * R(s.qv_sat_i) * dum_t;
     const R ab = R(1) + dqsdt * R(latvap) * R(INV_CP);
@@ -74,7 +76,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     get_rain_dsd2<R>(rt, qr_incld, nr_incld, mu_r, lamr);
     // get_cdistr_logn0r, P3I/p3_dsd2_impl.hpp:128-148
     if (qr_incld >= R(QSMALL)) {
-      cdistr = nr_incld / m_tgamma(mu_r + R(1));
+      cdistr = m_div(nr_incld, m_tgamma(mu_r + R(1)));
       logn0r = m_log10(cdistr) + (mu_r + R(1)) * m_log10(lamr);
     }
     s.nr = double(nr_incld) * cld_frac_r;
@@ -131,7 +133,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     // ventilation factor shared by melting, wet growth and the relaxation timescale
     // (every use below requires qi_incld >= QSMALL)
     const R vent = (qi_incld >= R(QSMALL))
-                       ? tv_qi2qr_melting + tv_vent_melt * m_cbrt(sc) * m_sqrt(rhofaci * rhor / mu)
+                       ? tv_qi2qr_melting + tv_vent_melt * m_cbrt(sc) * m_sqrt(m_div(rhofaci * rhor, mu))
                        : R(0);
 
     if (rt.do_ice_production) {
@@ -165,7 +167,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
       if (qi_incld >= R(QSMALL)) {
         const bool qm_pos = qm_incld > R(0.0);
         R tmp1 = R(0.0), Eii_fact = R(0.0);
-        if (qm_pos) tmp1 = qm_incld / qi_incld;
+        if (qm_pos) tmp1 = m_div(qm_incld, qi_incld);
         if (tmp1 < R(0.6) && qm_pos) Eii_fact = R(1);
         if (tmp1 >= R(0.6) && tmp1 < R(0.9) && qm_pos) Eii_fact = R(1) - (tmp1 - R(0.6)) / R(0.3);
         if (tmp1 >= R(0.9) && qm_pos) Eii_fact = R(0);
@@ -180,7 +182,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
       const R dqs = R(qsat0 - s.qv);
       qi2qr_melt_tend = (vent * (dT_melt * kap - rhor * R(latvap) * dv * dqs) * R(2) * R(Pi) / R(latice)) * ni_incld;
       qi2qr_melt_tend = vmax(qi2qr_melt_tend, R(0));
-      ni2nr_melt_tend = qi2qr_melt_tend * (ni_incld / qi_incld);
+      ni2nr_melt_tend = qi2qr_melt_tend * m_div(ni_incld, qi_incld);
     }
 
     if (rt.do_ice_production) {
@@ -198,7 +200,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
         const bool dum_ge_small = dum >= R(1.0e-10);
         if (dum_ge_small) {
           nr_ice_shed_tend = nr_ice_shed_tend + dum * R(1.923e+6);
-          const R dum1 = R(1.0) / (qc2qi_collect_tend + qr2qi_collect_tend);
+          const R dum1 = m_div(R(1.0), qc2qi_collect_tend + qr2qi_collect_tend);
           if (any_if_col) {
             qc2qr_ice_shed_tend = qc2qr_ice_shed_tend + dum * qc2qi_collect_tend * dum1;
             qc2qi_collect_tend = vmax(R(0), qc2qi_collect_tend - dum * qc2qi_collect_tend * dum1);
@@ -220,10 +222,10 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     if (qc2qi_collect_tend >= R(QSMALL) && T_atm < T_zerodegc) {
       const R vtrmi1 = tv_qi_fallspd * rhofaci;
       if (qc_incld >= R(QSMALL)) {
-        const R Vt_qc = R(s.acn) * m_tgamma(R(4 + bcn) + mu_c) / (m_pow(lamc, R(bcn)) * m_tgamma(R(4) + mu_c));
-        const R D_c = (R(4) + mu_c) / lamc;
+        const R Vt_qc = m_div(R(s.acn) * m_tgamma(R(4 + bcn) + mu_c), m_pow(lamc, R(bcn)) * m_tgamma(R(4) + mu_c));
+        const R D_c = m_div(R(4) + mu_c, lamc);
         const R V_impact = m_fabs(vtrmi1 - Vt_qc);
-        const R inv_Tc = R(1) / vmin(R(-0.001), R(T_atm - T_zerodegc));
+        const R inv_Tc = m_div(R(1), vmin(R(-0.001), R(T_atm - T_zerodegc)));
         const R Ri = vmax(R(1), vmin(R(-0.5e+6) * D_c * V_impact * inv_Tc, R(12)));
         if (Ri <= R(8.0)) rho_qm_cloud = double((R(0.051) + R(0.114) * Ri - R(0.0055) * (Ri * Ri)) * R(1000));
         else rho_qm_cloud = double(R(611.) + R(72.25) * (Ri - R(8)));
@@ -236,7 +238,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
       // cldliq_immersion_freezing, P3I/p3_cldliq_imm_freezing_impl.hpp:15-52
       if (qc_incld >= R(QSMALL) && T_atm <= T_rainfrz) {
         const R expAimmDt = m_exp(aimm * dT_frz);
-        const R x = R(1) / lamc;
+        const R x = m_div(R(1), lamc);
         const R inv_lamc3 = x * x * x;
         if constexpr (sizeof(R) == sizeof(double)) {
           qc2qi_hetero_freeze_tend = R(1.0) * R(CONS6) * cdist1 * m_tgamma(R(7) + mu_c) * expAimmDt * (inv_lamc3 * inv_lamc3);
@@ -260,7 +262,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     if (qr_incld >= R(QSMALL)) {
       const Tab3<R> t3 = lookup3<R>(mu_r, lamr);
       epsr = R(2) * R(Pi) * cdistr * rhor * dv *
-             (R(f1r) * m_tgamma(mu_r + R(2)) / lamr + R(f2r) * m_sqrt(rhor / mu) * m_cbrt(sc) * apply_table3<R>(TabOf<R>::get(tb).revap, t3));
+             (m_div(R(f1r) * m_tgamma(mu_r + R(2)), lamr) + R(f2r) * m_sqrt(m_div(rhor, mu)) * m_cbrt(sc) * apply_table3<R>(TabOf<R>::get(tb).revap, t3));
     }
 
     // evaporate_rain, P3I/p3_evaporate_rain_impl.hpp:83-201
@@ -271,56 +273,58 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
       const R cfr = R(cld_frac_r);
       if (qr_incld >= R(QSMALL) && ssat_r_d < 0 && cfr > cld_frac) {
         const R inv_dt_r = R(1 / dt);
-        const R tau_r = R(1) / epsr;
+        const R tau_r = m_div(R(1), epsr);
         const R dqv_dt = R((s.qv - s.qv_prev) * (1 / dt));
         const R dT = R(T_atm - s.t_prev);
         R eps_eff, A_c;
         if (T_atm < Tmelt) {
           const R fac = R(1) + R(latvap + latice) * R(1 / Cpair) * dqsdt;
-          eps_eff = epsr + epsi_tot * fac / abi;
-          A_c = dqv_dt - dqsdt * dT * inv_dt_r - R(s.qv_sat_l - s.qv_sat_i) * fac / abi * epsi_tot;
+          eps_eff = epsr + m_div(epsi_tot * fac, abi);
+          A_c = dqv_dt - dqsdt * dT * inv_dt_r - m_div(R(s.qv_sat_l - s.qv_sat_i) * fac, abi) * epsi_tot;
         } else {
           eps_eff = epsr;
           A_c = dqv_dt - dqsdt * dT * inv_dt_r;
         }
         if (eps_eff < R(1e-20)) eps_eff = R(1e-20);
-        const R tau_eff = R(1) / eps_eff;
+        const R tau_eff = m_div(R(1), eps_eff);
         // The limits below can remove all rain; they run in FP64 on the FP64
         // in-cloud mass (qr_incld is unchanged since entry) so that complete
         // evaporation leaves the same clipped residual in both forms.
         const double qr_incld_d = in0.qr;
         const double inv_dt_d = 1 / dt;
         double ev;
-        if (qr_incld < R(1e-12) && s.qv / s.qv_sat_l < 0.999) {
+        if (qr_incld < R(1e-12) && p3m_div(s.qv, s.qv_sat_l) < 0.999) {
           ev = qr_incld_d * inv_dt_d;
         } else {
-          const R dt_over_tau = R(dt) / tau_eff;
-          const R tscale_weight = -m_expm1(-dt_over_tau) / dt_over_tau;
-          const R equilib_tend = -A_c / ab * tau_eff / tau_r;
-          const R instant_tend = -ssat_r / (ab * tau_r);
+          const R dt_over_tau = m_div(R(dt), tau_eff);
+          const R tscale_weight = m_div(-m_expm1(-dt_over_tau), dt_over_tau);
+          const R equilib_tend = m_div(m_div(-A_c, ab) * tau_eff, tau_r);
+          const R instant_tend = m_div(-ssat_r, ab * tau_r);
           ev = double(instant_tend * tscale_weight + equilib_tend * (R(1) - tscale_weight));
         }
         const double abd = ab, cfd = cld_frac;
-        if (ev > -ssat_r_d * inv_dt_d / abd) ev = -ssat_r_d * inv_dt_d / abd;
+        const double ev_max = p3m_div(-ssat_r_d * inv_dt_d, abd);
+        if (ev > ev_max) ev = ev_max;
         if (ev < 0) ev = 0;
         if (ev > qr_incld_d * inv_dt_d) ev = qr_incld_d * inv_dt_d;
-        ev = ev * (cld_frac_r - cfd) / cld_frac_r;
+        ev = p3m_div(ev * (cld_frac_r - cfd), cld_frac_r);
         evap_d = ev;
-        nr_evap_d = ev * (double(nr_incld) / qr_incld_d);
+        nr_evap_d = ev * p3m_div(double(nr_incld), qr_incld_d);
       }
     }
 
     if (rt.do_ice_production) {
       // ice_deposition_sublimation, P3I/p3_ice_deposition_sublimation_impl.hpp:10-65
       if (qi_incld > R(QSMALL)) {
-        const R qi_tend = vmin(epsi / abi, R(inv_dt)) * R(s.qv - s.qv_sat_i);
+        const R epsi_abi = m_div(epsi, abi);
+        const R qi_tend = vmin(epsi_abi, R(inv_dt)) * R(s.qv - s.qv_sat_i);
         const bool neg = qi_tend < R(0);
         if (neg) {
           qi2qv_sublim_tend = -qi_tend;
-          ni_sublim_tend = qi2qv_sublim_tend * (ni_incld / qi_incld);
+          ni_sublim_tend = qi2qv_sublim_tend * m_div(ni_incld, qi_incld);
         }
         if (T_atm < T_zerodegc && !neg) qv2qi_vapdep_tend = qi_tend;
-        if (T_atm < T_zerodegc) qc2qi_berg_tend = vmax(epsi / abi * R(s.qv_sat_l - s.qv_sat_i), R(0));
+        if (T_atm < T_zerodegc) qc2qi_berg_tend = vmax(epsi_abi * R(s.qv_sat_l - s.qv_sat_i), R(0));
       }
     }
   }  // !skip_micro
@@ -357,7 +361,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
       qc2qr_autoconv_tend = R(1.0) * R(rt.autoconversion_prefactor) * m_pow(qc_incld, R(rt.autoconversion_qc_exponent)) *
                             m_pow(nc_incld * R(1.e-6) * R(rho), R(-rt.autoconversion_nc_exponent));
       ncautr = qc2qr_autoconv_tend * cons3;
-      nc2nr_autoconv_tend = qc2qr_autoconv_tend * nc_incld / qc_incld;
+      nc2nr_autoconv_tend = m_div(qc2qr_autoconv_tend * nc_incld, qc_incld);
     }
     if (qc2qr_autoconv_tend == R(0)) nc2nr_autoconv_tend = R(0);
     if (nc2nr_autoconv_tend == R(0)) qc2qr_autoconv_tend = R(0);
@@ -370,14 +374,14 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     else
       qc2qr_accret_tend = R(1.0) * R(rt.accretion_prefactor) * m_pow(qc_incld, R(rt.accretion_qc_exponent)) *
                           m_pow(qr_incld, R(rt.accretion_qr_exponent));
-    nc_accret_tend = qc2qr_accret_tend * nc_incld / qc_incld;
+    nc_accret_tend = m_div(qc2qr_accret_tend * nc_incld, qc_incld);
     if (nc_accret_tend == R(0)) qc2qr_accret_tend = R(0);
     if (qc2qr_accret_tend == R(0)) nc_accret_tend = R(0);
   }
   // rain_self_collection, P3I/p3_rain_self_collection_impl.hpp:9-55
   if (qr_incld >= R(QSMALL)) {
     const R bd = R(rt.rain_selfcollection_breakup_diameter);
-    const R dum2 = m_cbrt((qr_incld) / (R(Pi) * R(RHO_H2O) * nr_incld));
+    const R dum2 = m_cbrt(m_div(qr_incld, R(Pi) * R(RHO_H2O) * nr_incld));
     R dum;
     if (dum2 < bd) dum = R(1);
     else dum = R(2) - m_exp(R(2300) * (dum2 - bd));
@@ -441,7 +445,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     const double sources = s.qc;
     double ratio;
     if (sinks > sources && sinks >= QTENDSMALL) {
-      ratio = sources / sinks;
+      ratio = p3m_div(sources, sinks);
       t_qc2qr_autoconv *= ratio;
       t_qc2qr_accret *= ratio;
       t_qc2qi_collect *= ratio;
@@ -461,7 +465,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     const double sinks = (t_qr2qv_evap + t_qr2qi_collect + t_qr2qi_immers) * dt;
     const double sources = s.qr + (t_qc2qr_autoconv + t_qc2qr_accret + t_qi2qr_melt + t_qc2qr_ice_shed) * dt;
     if (sinks > sources && sinks >= QTENDSMALL) {
-      const double ratio = sources / sinks;
+      const double ratio = p3m_div(sources, sinks);
       t_qr2qv_evap *= ratio;
       t_qr2qi_collect *= ratio;
       t_qr2qi_immers *= ratio;
@@ -473,7 +477,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     const double sources = s.qi + (t_qv2qi_vapdep + t_qv2qi_nucleat + t_qr2qi_collect + t_qc2qi_collect + t_qr2qi_immers +
                                    t_qc2qi_hetero + t_qc2qi_berg) * dt;
     if (sinks > sources && sinks >= QTENDSMALL) {
-      const double ratio = sources / sinks;
+      const double ratio = p3m_div(sources, sinks);
       t_qi2qv_sublim *= ratio;
       t_qi2qr_melt *= ratio;
     }
@@ -515,15 +519,15 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
   }
   // ice_supersat_conservation, P3I/p3_ice_supersat_conservation_impl.hpp:14-43
   {
-    const double t_atm = s.th / s.inv_exner;
+    const double t_atm = p3m_div(s.th, s.inv_exner);
     const double latsublim2 = (latvap + latice) * (latvap + latice);
     const double qv_sink = t_qv2qi_vapdep + t_qv2qi_nucleat;
     if (qv_sink > QSMALL && cld_frac_i > 1e-20) {
-      double qv_avail = (s.qv + (t_qi2qv_sublim + t_qr2qv_evap) * dt - s.qv_sat_i) /
-                        (1 + latsublim2 * s.qv_sat_i / (CP * RH2O * (t_atm * t_atm))) / dt;
+      double qv_avail = p3m_div(p3m_div(s.qv + (t_qi2qv_sublim + t_qr2qv_evap) * dt - s.qv_sat_i,
+                                        1 + p3m_div(latsublim2 * s.qv_sat_i, CP * RH2O * (t_atm * t_atm))), dt);
       qv_avail = vmax(qv_avail, 0.0);
       if (qv_sink > qv_avail) {
-        const double fract = qv_avail / qv_sink;
+        const double fract = p3m_div(qv_avail, qv_sink);
         t_qv2qi_nucleat = t_qv2qi_nucleat * fract;
         t_qv2qi_vapdep = t_qv2qi_vapdep * fract;
       }
@@ -536,10 +540,10 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
       const double qv_sinks = t_qv2qi_vapdep + t_qv2qi_nucleat;
       const double T_endstep = T_atm + ((qv_sinks - t_qi2qv_sublim) * (latvap + latice) * inv_cp -
                                         t_qr2qv_evap * latvap * inv_cp) * dt;
-      const double qsl = qv_sat_dry(T_endstep, pres, false, err);
-      const double A = latvap * qsl * dt * inv_cp / (RV * T_endstep * T_endstep) *
+      const double qsl = qv_sat_dry_liquid(T_endstep, pres, err);
+      const double A = p3m_div(latvap * qsl * dt * inv_cp, RV * T_endstep * T_endstep) *
                        ((latvap + latice) * t_qi2qv_sublim + latvap * t_qr2qv_evap);
-      double frac = (qsl - s.qv + qv_sinks * dt + A) / (qv_sources * dt + A);
+      double frac = p3m_div(qsl - s.qv + qv_sinks * dt + A, qv_sources * dt + A);
       frac = vmax(0.0, frac);
       frac = vmin(1.0, frac);
       t_qi2qv_sublim = frac * t_qi2qv_sublim;
@@ -555,14 +559,15 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     s.qr = s.qr + (-t_qr2qi_collect + t_qi2qr_melt - t_qr2qi_immers + t_qc2qr_ice_shed) * dt;
     s.nr = s.nr + (-t_nr_collect - t_nr2ni_immers + nmltratio * t_ni2nr_melt + t_nr_ice_shed + t_ncshdc) * dt;
     if (s.qi >= QSMALL) {
-      s.bm = s.bm - ((t_qi2qv_sublim + t_qi2qr_melt) / s.qi) * dt * s.bm;
-      s.qm = s.qm - ((t_qi2qv_sublim + t_qi2qr_melt) * s.qm / s.qi) * dt;
+      const double rqi = p3m_recip(s.qi);
+      s.bm = s.bm - p3m_div_y(t_qi2qv_sublim + t_qi2qr_melt, s.qi, rqi) * dt * s.bm;
+      s.qm = s.qm - p3m_div_y((t_qi2qv_sublim + t_qi2qr_melt) * s.qm, s.qi, rqi) * dt;
       s.qi = s.qi - (t_qi2qv_sublim + t_qi2qr_melt) * dt;
     }
     const double dum = (t_qr2qi_collect + t_qc2qi_collect + t_qr2qi_immers + t_qc2qi_hetero) * dt;
     s.qi = s.qi + (t_qv2qi_vapdep + t_qv2qi_nucleat + t_qc2qi_berg) * dt + dum;
     s.qm = s.qm + dum;
-    s.bm = s.bm + (t_qr2qi_collect * INV_RHO_RIMEMAX + t_qc2qi_collect / rho_qm_cloud +
+    s.bm = s.bm + (t_qr2qi_collect * INV_RHO_RIMEMAX + p3m_div(t_qc2qi_collect, rho_qm_cloud) +
                    (t_qr2qi_immers + t_qc2qi_hetero) * INV_RHO_RIMEMAX) * dt;
     s.ni = s.ni + (t_ni_nucleat - t_ni2nr_melt - t_ni_sublim - t_ni_selfcollect + t_nr2ni_immers + t_nc2ni_immers) * dt;
     if (s.qm < 0) { s.qm = 0; s.bm = 0; }
@@ -608,7 +613,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     } else present = true;
 
     // P3I/p3_main_impl_part2.hpp:514-517
-    double ni_incld_d = s.ni / cld_frac_i;
+    double ni_incld_d = p3m_div(s.ni, cld_frac_i);
     impose_max_total_ni<double>(ni_incld_d, rt.max_total_ni, inv_rho);
     s.ni = ni_incld_d * cld_frac_i;
     return present;

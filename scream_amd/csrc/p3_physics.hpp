@@ -46,6 +46,24 @@ __device__ __forceinline__ float m_expm1(float x) { return ::expm1f(x); }
 __device__ __forceinline__ double m_fabs(double x) { return ::fabs(x); }
 __device__ __forceinline__ float m_fabs(float x) { return ::fabsf(x); }
 
+// Division whose operands and quotient stay inside the exponent range that
+// needs no scaling (p3_math.h); the mixed form divides as it always did.
+__device__ __forceinline__ double m_div(double a, double b) { return p3m_div(a, b); }
+__device__ __forceinline__ float m_div(float a, float b) { return a / b; }
+
+// t^1.5 and t^1.81 of a temperature (FP64: from one logarithm; NaN where t is
+// not positive and finite)
+__device__ __forceinline__ void pow_15_181(double t, double& a, double& b) {
+  double h, l;
+  p3m_log_core(p3m_positive(t) ? t : p3m_nan(), &h, &l);
+  a = p3m_pow_log(h, l, 1.5);
+  b = p3m_pow_log(h, l, 1.81);
+}
+__device__ __forceinline__ void pow_15_181(float t, float& a, float& b) {
+  a = m_pow(t, 1.5f);
+  b = m_pow(t, 1.81f);
+}
+
 // ekat::impl::min/max on scalars (ternary form, argument order preserved)
 template <class T> __device__ __forceinline__ T vmin(T a, T b) { return a < b ? a : b; }
 template <class T> __device__ __forceinline__ T vmax(T a, T b) { return a > b ? a : b; }
@@ -54,21 +72,33 @@ template <class T> __device__ __forceinline__ T vmax(T a, T b) { return a > b ? 
 enum : unsigned { ERR_BAD_TEMPERATURE = 1u, ERR_SUBSTEP_LIMIT = 2u, ERR_CHECK_VALUES = 4u };
 
 // ---------------------------------------------------------------- saturation (FP64 always)
-// MurphyKoop_svp, PSH:38-77 (with check_temperature, PSH:14-36, as a flag)
-__host__ __device__ __forceinline__ double mk_svp(double t, bool ice, unsigned& err) {
-  if (t <= 0 || t != t) err |= ERR_BAD_TEMPERATURE;  // t != t: NaN
-  if (ice && t < Tmelt) {
-    return p3m_exp(9.550426 - (5723.265 / t) + (3.53068 * p3m_log(t)) - (0.00728332 * t));
-  }
-  const double logt = p3m_log(t);
-  return p3m_exp(54.842763 - (6763.22 / t) - (4.210 * logt) + (0.000367 * t) +
-               (p3m_tanh(0.0415 * (t - 218.8)) *
-                (53.878 - (1331.22 / t) - (9.44523 * logt) + 0.014025 * t)));
+// MurphyKoop_svp, PSH:38-77 (check_temperature, PSH:14-36, as a flag), from
+// log(t) and the reciprocal of t that its divisions by t share
+__host__ __device__ __forceinline__ double mk_svp_ice(double t, double logt, double rt) {
+  return p3m_exp(9.550426 - p3m_div_y(5723.265, t, rt) + (3.53068 * logt) - (0.00728332 * t));
 }
-// qv_sat_dry, PSH:127-157
-__device__ __forceinline__ double qv_sat_dry(double t, double p, bool ice, unsigned& err) {
-  const double e = mk_svp(t, ice, err);
-  return ep_2 * e / vmax(p, 1.e-3);
+__host__ __device__ __forceinline__ double mk_svp_liquid(double t, double logt, double rt) {
+  return p3m_exp(54.842763 - p3m_div_y(6763.22, t, rt) - (4.210 * logt) + (0.000367 * t) +
+               (p3m_tanh(0.0415 * (t - 218.8)) *
+                (53.878 - p3m_div_y(1331.22, t, rt) - (9.44523 * logt) + 0.014025 * t)));
+}
+__host__ __device__ __forceinline__ void check_temperature(double t, unsigned& err) {
+  if (t <= 0 || t != t) err |= ERR_BAD_TEMPERATURE;  // t != t: NaN
+}
+// qv_sat_dry over liquid, PSH:127-157
+__device__ __forceinline__ double qv_sat_dry_liquid(double t, double p, unsigned& err) {
+  check_temperature(t, err);
+  return p3m_div(ep_2 * mk_svp_liquid(t, p3m_log(t), p3m_recip(t)), vmax(p, 1.e-3));
+}
+// qv_sat_dry over liquid and over ice (liquid again from Tmelt up) at one point:
+// log(t) and both reciprocals are formed once
+__device__ __forceinline__ void qv_sat_dry_both(double t, double p, double& liquid, double& ice, unsigned& err) {
+  check_temperature(t, err);
+  const double logt = p3m_log(t), rt = p3m_recip(t);
+  const double pm = vmax(p, 1.e-3), rp = p3m_recip(pm);
+  liquid = p3m_div_y(ep_2 * mk_svp_liquid(t, logt, rt), pm, rp);
+  ice = liquid;
+  if (t < Tmelt) ice = p3m_div_y(ep_2 * mk_svp_ice(t, logt, rt), pm, rp);
 }
 
 // ---------------------------------------------------------------- runtime options
@@ -125,13 +155,13 @@ template <class R> struct Tab3 { int dumii, dumjj; R rdumii, rdumjj; };
 template <class R>
 __device__ __forceinline__ TabIce<R> lookup_ice(R qi, R ni, R qm, R rhop) {
   TabIce<R> t;
-  t.dum1 = (m_log10(qi / ni) + R(18)) * R(lookup_table_1a_dum1_c) - R(10);
+  t.dum1 = (m_log10(m_div(qi, ni)) + R(18)) * R(lookup_table_1a_dum1_c) - R(10);
   t.dumi = (int)t.dum1;
   t.dum1 = vmin(t.dum1, R(isize));
   t.dum1 = vmax(t.dum1, R(1.));
   t.dumi = vmax(1, t.dumi);
   t.dumi = vmin(isize - 1, t.dumi);
-  t.dum4 = (qm / qi) * R(3) + R(1);
+  t.dum4 = m_div(qm, qi) * R(3) + R(1);
   t.dumii = (int)t.dum4;
   t.dum4 = vmin(t.dum4, R(rimsize));
   t.dum4 = vmax(t.dum4, R(1.));
@@ -156,7 +186,7 @@ __device__ __forceinline__ TabRain<R> lookup_rain(R qr, R nr) {
   TabRain<R> t;
   const bool gt_small = qr > R(QSMALL) && nr > R(0.0);
   R dumlr = R(1);
-  if (gt_small) dumlr = m_cbrt(qr / (R(Pi) * R(RHO_H2O) * nr));
+  if (gt_small) dumlr = m_cbrt(m_div(qr, R(Pi) * R(RHO_H2O) * nr));
   t.dum3 = (m_log10(R(1) * dumlr) + R(5)) * R(10.70415);
   t.dumj = (int)t.dum3;
   t.dum3 = vmin(t.dum3, R(rcollsize));
@@ -310,7 +340,7 @@ __device__ __forceinline__ void apply_table_coll2(const R* __restrict__ tab, con
 template <class R>
 __device__ __forceinline__ Tab3<R> lookup3(R mu_r, R lamr) {
   Tab3<R> t;
-  const R dum1 = (mu_r + R(1)) / lamr;
+  const R dum1 = m_div(mu_r + R(1), lamr);
   if (dum1 <= R(195.e-6)) {
     const R inv_dum3 = R(0.1);
     R rdumii = (dum1 * R(1.e6) + R(5)) * inv_dum3;
@@ -380,20 +410,20 @@ __device__ __forceinline__ void get_cloud_dsd2(R qc, R& nc, R& mu_c, R rho, R& l
   if (qc >= R(QSMALL)) {
     nc = vmax(nc, R(NSMALL));
     R m = R(0.0005714) * (nc * R(1.e-6) * rho) + R(0.2714);
-    m = R(1) / (m * m) - R(1);
+    m = m_div(R(1), m * m) - R(1);
     m = vmax(m, R(2));
     m = vmin(m, R(15));
     mu_c = m;
-    lamc = m_cbrt(R(CONS1) * nc * (m + R(3)) * (m + R(2)) * (m + R(1)) / qc);
+    lamc = m_cbrt(m_div(R(CONS1) * nc * (m + R(3)) * (m + R(2)) * (m + R(1)), qc));
     const R lammin = (m + R(1)) * R(2.5e+4);
     const R lammax = (m + R(1)) * R(1.e+6);
     const bool lt = lamc < lammin, gt = lamc > lammax;
     if (lt) lamc = lammin;
     if (gt) lamc = lammax;
     if (lt || gt)
-      nc = R(6) * (lamc * lamc * lamc) * qc / (R(Pi) * R(RHO_H2O) * (m + R(3)) * (m + R(2)) * (m + R(1)));
-    cdist = nc * (m + R(1)) / lamc;
-    cdist1 = nc / m_tgamma(m + R(1));
+      nc = m_div(R(6) * (lamc * lamc * lamc) * qc, R(Pi) * R(RHO_H2O) * (m + R(3)) * (m + R(2)) * (m + R(1)));
+    cdist = m_div(nc * (m + R(1)), lamc);
+    cdist1 = m_div(nc, m_tgamma(m + R(1)));
   }
 }
 
@@ -405,7 +435,7 @@ __device__ __forceinline__ void get_rain_dsd2(const Runtime& rt, R qr, R& nr, R&
     const R nr_lim = vmax(nr, R(NSMALL));
     mu_r = R(rt.constant_mu_rain);
     const R f = R(CONS1) * (mu_r + R(3)) * (mu_r + R(2)) * (mu_r + R(1));
-    lamr = m_cbrt(f * nr_lim / qr);
+    lamr = m_cbrt(m_div(f * nr_lim, qr));
     const R lammax = (mu_r + R(1.)) * R(1.e+5);
     const R lammin = (mu_r + R(1.)) * R(500);
     const bool lt = lamr < lammin, gt = lamr > lammax;
@@ -413,7 +443,7 @@ __device__ __forceinline__ void get_rain_dsd2(const Runtime& rt, R qr, R& nr, R&
     if (lt || gt) {
       if (lt) lamr = lammin;
       if (gt) lamr = lammax;
-      nr = lamr * lamr * lamr * qr / f;
+      nr = m_div(lamr * lamr * lamr * qr, f);
     }
   }
 }
@@ -423,7 +453,7 @@ template <class R>
 __device__ __forceinline__ R calc_bulk_rho_rime(const Runtime& rt, R qi_tot, R& qi_rim, R& bi_rim) {
   R rho_rime = R(0);
   const bool gt = bi_rim >= R(BSMALL), lt = bi_rim < R(BSMALL);
-  if (gt) rho_rime = qi_rim / bi_rim;
+  if (gt) rho_rime = m_div(qi_rim, bi_rim);
   const bool lt_min = rho_rime < R(rt.min_rime_rho), gt_max = rho_rime > R(rt.max_rime_rho);
   if (gt && lt_min) rho_rime = R(rt.min_rime_rho);
   if (gt && gt_max) rho_rime = R(rt.max_rime_rho);
@@ -433,7 +463,7 @@ __device__ __forceinline__ R calc_bulk_rho_rime(const Runtime& rt, R qi_tot, R& 
   // again with qi_rim = qi_tot when the rime exceeds the total; the second
   // overrides the first, and `lt` excludes both, so one division serves.
   const bool over = qi_rim > qi_tot && rho_rime > R(0);
-  if (over || clamped) bi_rim = (over ? qi_tot : qi_rim) / rho_rime;
+  if (over || clamped) bi_rim = m_div(over ? qi_tot : qi_rim, rho_rime);
   if (over) qi_rim = qi_tot;
   if (qi_rim < R(QSMALL)) { qi_rim = R(0); bi_rim = R(0); }
   return rho_rime;
@@ -460,7 +490,7 @@ __device__ __forceinline__ Incld incloud(double qc, double qr, double qi, double
 // impose_max_total_ni, P3I/p3_impose_max_total_ni_impl.hpp:9-26
 template <class R>
 __device__ __forceinline__ void impose_max_total_ni(R& ni, R max_total_ni, R inv_rho) {
-  if (ni >= R(1e-20)) ni = ni * vmin(max_total_ni * inv_rho / ni, R(1));
+  if (ni >= R(1e-20)) ni = ni * vmin(m_div(max_total_ni * inv_rho, ni), R(1));
 }
 
 }  // namespace p3d

@@ -110,6 +110,13 @@ template <class R, int L> constexpr bool ice_rec_dif() {
 }
 template <class R, int L> constexpr int ice_lds_len() { return kIceCells * (ice_rec_dif<R, L>() ? 8 : 4); }
 
+// An in-cloud value q / cf after the first substep.  In FP64 the reciprocal
+// rcf = p3m_recip(cf) is formed once per level and run (cf does not change over
+// the substeps): four instructions instead of a division's thirteen issue
+// slots, for up to four fields per level and substep.
+__device__ __forceinline__ double incloud_div(double q, double cf, double rcf) { return p3m_div_y(q, cf, rcf); }
+__device__ __forceinline__ float incloud_div(float q, float cf, float) { return q / cf; }
+
 // Per-lane geometry of the owned levels.
 template <int L>
 struct Geo {
@@ -134,6 +141,7 @@ struct SedRun {
   static constexpr int NF = SP == 2 ? 4 : 2;  // fields held (cloud always holds nc: its DSD rewrites it)
   Geo<L> g;
   double q[NF][L], cf[L], coef[L], cfl_ice[L], pflux[L];
+  R rcf[L];  // FP64: p3m_recip(cf)
   int kbase, k_top, k_bot;
   double dt_left, prt_accum;  // prt_accum: mass through the surface, on the lane owning the lowest level
   int nsub;
@@ -160,12 +168,13 @@ struct SedRun {
       const size_t x = p.at(i, ok ? k : 0);
       const double dz = ok ? p.dz[x] : 1.0;
       const double dp = ok ? p.dpres[x] : 1.0;
-      g.rho[t] = dp / dz / gravit;
-      g.inv_rho[t] = 1 / g.rho[t];
-      g.inv_dz[t] = 1 / dz;
+      g.rho[t] = air_density(dp, dz);
+      g.inv_rho[t] = p3m_div(1.0, g.rho[t]);
+      g.inv_dz[t] = p3m_div(1.0, dz);
 #pragma unroll
       for (int f = 0; f < NF; ++f) q[f][t] = ok ? fld[f][x] : 0.0;
       cf[t] = ok ? cfp[x] : 1.0;
+      rcf[t] = sizeof(R) == 8 ? R(p3m_recip(cf[t])) : R(0);
       coef[t] = ok ? p.sc(coef_f, i, ok ? k : 0) : 0.0;
       cfl_ice[t] = (SP == 2 && ok) ? p.cld_frac_l[x] : 1.0;
       pflux[t] = 0;
@@ -200,21 +209,21 @@ struct SedRun {
           const R qc = R(q[0][t]), nc = R(q[1][t]);
           R qc_incld, nc_incld;
           if (first) {
-            const R icfl = R(1) / cfl;
+            const R icfl = m_div(R(1), cfl);
             if (q[0][t] >= QSMALL) { qc_incld = vmin(qc * icfl, R(incloud_limit)); nc_incld = vmax(nc * icfl, R(0)); }
             else { qc_incld = 0; nc_incld = 0; }
           } else {
-            qc_incld = qc / cfl;
-            nc_incld = nc / cfl;
+            qc_incld = incloud_div(qc, cfl, rcf[t]);
+            nc_incld = incloud_div(nc, cfl, rcf[t]);
           }
           if (qc_incld > R(QSMALL)) {
             R ncr = nc_incld, mu_c, lamc, cdist, cdist1;
             get_cloud_dsd2<R>(qc_incld, ncr, mu_c, R(rho), lamc, cdist, cdist1);
             q[1][t] = double(ncr) * cf[t];
-            const R dum = R(1) / m_pow(lamc, R(bcn));
+            const R dum = m_div(R(1), m_pow(lamc, R(bcn)));
             const R acn = R(coef[t]);
-            V1[t] = double(acn * m_tgamma(R(4 + bcn) + mu_c) * dum / m_tgamma(mu_c + R(4)));
-            if (p.predictNc) V2[t] = double(acn * m_tgamma(R(1 + bcn) + mu_c) * dum / m_tgamma(mu_c + R(1)));
+            V1[t] = double(m_div(acn * m_tgamma(R(4 + bcn) + mu_c) * dum, m_tgamma(mu_c + R(4))));
+            if (p.predictNc) V2[t] = double(m_div(acn * m_tgamma(R(1 + bcn) + mu_c) * dum, m_tgamma(mu_c + R(1))));
           }
         } else if constexpr (SP == 1) {
           // rain_sedimentation + compute_rain_fall_velocity, P3I/p3_rain_sed_impl.hpp:14-34,104-126
@@ -222,12 +231,12 @@ struct SedRun {
           const R qr = R(q[0][t]), nr = R(q[1][t]);
           R qr_incld, nr_incld;
           if (first) {
-            const R icfr = R(1) / cfr;
+            const R icfr = m_div(R(1), cfr);
             if (q[0][t] >= QSMALL) { qr_incld = vmin(qr * icfr, R(precip_limit)); nr_incld = vmax(nr * icfr, R(0)); }
             else { qr_incld = 0; nr_incld = 0; }
           } else {
-            qr_incld = qr / cfr;
-            nr_incld = nr / cfr;
+            qr_incld = incloud_div(qr, cfr, rcf[t]);
+            nr_incld = incloud_div(nr, cfr, rcf[t]);
           }
           if (qr_incld > R(QSMALL)) {
             R nrr = nr_incld, mu_r = 0, lamr;
@@ -246,16 +255,16 @@ struct SedRun {
           const R qi = R(q[0][t]), ni = R(q[1][t]), qm = R(q[2][t]), bm = R(q[3][t]);
           R qi_incld, ni_incld, qm_incld, bm_incld;
           if (first) {
-            const R icfi = R(1) / cfi, icfl = R(1) / R(cfl_ice[t]);
+            const R icfi = m_div(R(1), cfi), icfl = m_div(R(1), R(cfl_ice[t]));
             if (q[0][t] >= QSMALL) { qi_incld = vmin(qi * icfi, R(incloud_limit)); ni_incld = vmax(ni * icfi, R(0)); }
             else { qi_incld = 0; ni_incld = 0; }
             if (q[0][t] >= QSMALL && q[2][t] >= QSMALL) { qm_incld = qm * icfi; bm_incld = vmin(vmax(bm * icfl, R(0)), R(incloud_limit)); }
             else { qm_incld = 0; bm_incld = 0; }
           } else {
-            qi_incld = qi / cfi;
-            ni_incld = ni / cfi;
-            qm_incld = qm / cfi;
-            bm_incld = bm / cfi;
+            qi_incld = incloud_div(qi, cfi, rcf[t]);
+            ni_incld = incloud_div(ni, cfi, rcf[t]);
+            qm_incld = incloud_div(qm, cfi, rcf[t]);
+            bm_incld = incloud_div(bm, cfi, rcf[t]);
           }
           if (qi_incld > R(QSMALL)) {
             R nir = vmax(ni_incld, R(NSMALL));
@@ -298,7 +307,7 @@ struct SedRun {
 
     // generalized_sedimentation + calc_first_order_upwind_step, P3I/p3_upwind_impl.hpp:14-129
     const int tmpint1 = (int)(Co_max + 1);
-    const double dt_sub = dt_left / tmpint1;
+    const double dt_sub = p3m_div(dt_left, (double)tmpint1);
     const int k_temp = (k_bot == kbot) ? k_bot : k_bot + 1;
     // fluxes F = V r rho.  Only the levels in [k_top, k_temp] update, and
     // they read F of their own level and of the level above, which is in
@@ -477,16 +486,17 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
       if (qr_ge) { qr = 0; nr = 0; }
     }
     // p3_main_part3, P3I/p3_main_impl_part3.hpp:60-199 (only the fields p3_main outputs)
-    const double rho = p.dpres[x] / p.dz[x] / gravit;
-    const double inv_rho = 1 / rho;
+    const double rho = air_density(p.dpres[x], p.dz[x]);
+    const double inv_rho = p3m_div(1.0, rho);
     const double cfl = p.cld_frac_l[x], cfr = p.cld_frac_r[x], cfi = p.cld_frac_i[x];
     double vap_liq = p.vap_liq_exchange[x];
     // cloud
     if (qc >= QSMALL) {
-      R ncr = R(nc / cfl), mu_c, lamc, cd, cd1;
-      get_cloud_dsd2<R>(R(qc / cfl), ncr, mu_c, R(rho), lamc, cd, cd1);
+      const double rcfl = p3m_recip(cfl);
+      R ncr = R(p3m_div_y(nc, cfl, rcfl)), mu_c, lamc, cd, cd1;
+      get_cloud_dsd2<R>(R(p3m_div_y(qc, cfl, rcfl)), ncr, mu_c, R(rho), lamc, cd, cd1);
       nc = double(ncr) * cfl;
-      reff_c = double(R(0.5) * (mu_c + R(3)) / lamc);
+      reff_c = double(m_div(R(0.5) * (mu_c + R(3)), lamc));
     } else {
       qv = qv + qc;
       th = th - inv_exner * qc * latvap * inv_cp;
@@ -495,10 +505,11 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
     }
     // rain
     if (qr >= QSMALL) {
-      R nrr = R(nr / cfr), mu_r = 0, lamr;
-      get_rain_dsd2<R>(rt, R(qr / cfr), nrr, mu_r, lamr);
+      const double rcfr = p3m_recip(cfr);
+      R nrr = R(p3m_div_y(nr, cfr, rcfr)), mu_r = 0, lamr;
+      get_rain_dsd2<R>(rt, R(p3m_div_y(qr, cfr, rcfr)), nrr, mu_r, lamr);
       nr = double(nrr) * cfr;
-      reff_r = double(R(1.5) / lamr);
+      reff_r = double(m_div(R(1.5), lamr));
     } else {
       qv = qv + qr;
       th = th - inv_exner * qr * latvap * inv_cp;
@@ -509,10 +520,11 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
     {
       const bool qi_gt = qi >= QSMALL;
       ni = vmax(ni, NSMALL);
-      const double qi_incld = qi / cfi;
-      double ni_incld = ni / cfi;
-      R qmr = R(qm / cfi), bmr = R(bm / cfi);
-      double qm_incld = qm / cfi, bm_incld = bm / cfi;
+      const double rcfi = p3m_recip(cfi);
+      const double qi_incld = p3m_div_y(qi, cfi, rcfi);
+      double ni_incld = p3m_div_y(ni, cfi, rcfi);
+      double qm_incld = p3m_div_y(qm, cfi, rcfi), bm_incld = p3m_div_y(bm, cfi, rcfi);
+      R qmr = R(qm_incld), bmr = R(bm_incld);
       R rhop = 0;
       if (qi_gt) {
         rhop = calc_bulk_rho_rime<R>(rt, R(qi_incld), qmr, bmr);
@@ -562,14 +574,16 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
     const Amble& a = p.amble;
     const double dp = a.dp_wet[x], dp_dry = p.dpres[x];
     const double T_before = a.T_mid[x];
-    double T = (th * exner_function(a.p_mid[x]) - T_before) * dp_dry / dp;
+    const double rdp = p3m_recip(dp);
+    auto to_wet = [&](double q) { return p3m_div_y(q * dp_dry, dp, rdp); };
+    double T = to_wet(th * exner_function(a.p_mid[x]) - T_before);
     T += T_before;
     a.T_mid[x] = T;
     a.T_prev[x] = T;
-    qv = qv * dp_dry / dp;
-    p.qc[x] = qc * dp_dry / dp; p.nc[x] = nc * dp_dry / dp; p.qr[x] = qr * dp_dry / dp;
-    p.nr[x] = nr * dp_dry / dp; p.qi[x] = qi * dp_dry / dp; p.ni[x] = ni * dp_dry / dp;
-    p.qm[x] = qm * dp_dry / dp; p.bm[x] = bm * dp_dry / dp; p.qv[x] = qv;
+    qv = to_wet(qv);
+    p.qc[x] = to_wet(qc); p.nc[x] = to_wet(nc); p.qr[x] = to_wet(qr);
+    p.nr[x] = to_wet(nr); p.qi[x] = to_wet(qi); p.ni[x] = to_wet(ni);
+    p.qm[x] = to_wet(qm); p.bm[x] = to_wet(bm); p.qv[x] = qv;
     a.qv_prev[x] = qv;
     reff_c *= 1e6;
     reff_i *= 1e6;

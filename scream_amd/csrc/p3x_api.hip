@@ -225,8 +225,7 @@ int fill_params(const p3x_context* c, const p3x_runtime* runtime, const p3x_prog
   k.exch_zero = infra->exchange_zeroed_on_entry ? 1 : 0;
   // qv_sat_dry(Tmelt, p) = ep_2 e_melt / max(p, 1e-3) for melting and wet growth: the same
   // portable arithmetic on the host as on the device
-  unsigned no_err = 0;
-  k.e_melt = p3d::mk_svp(p3c::Tmelt, false, no_err);
+  k.e_melt = p3d::mk_svp_liquid(p3c::Tmelt, p3m_log(p3c::Tmelt), p3m_recip(p3c::Tmelt));
   k.amble = p3d::Amble{};  // no fused pre/post-amble
   return P3X_OK;
 }

@@ -154,16 +154,15 @@ typedef struct p3x_launch {
   int precision;           /* P3X_FP64 (drop-in) or P3X_MIXED (FP32 bulk rates)  */
   int ld;                  /* level-major: row stride (>= nj; 0 means nj);        */
                            /* column-major: column stride (>= nk; 0 means nk)     */
-  /* part 1 kernel: columns per block x threads per block, both 0 for the
-   * default, else one of 16x128, 16x256, 32x256, 64x256, 32x512, 64x512      */
+  /* both 0, else one of 16x128, 16x256, 32x256, 64x256, 32x512, 64x512: accepted
+   * without effect (parts 1 and 2 run in one kernel of one shape)            */
   int columns_per_block;
   int threads_per_block;
   /* sedimentation kernels: lanes per column, 0 for each species group's
    * default, else 16, 32 or 64 for both groups; nk may not exceed 8 x this
    * (nk <= 512 in any case)                                                   */
   int sed_lanes_per_column;
-  /* part 2 kernel: wavefronts per SIMD its registers must allow, 0 for the
-   * default (2), else 1 or 2; an explicit block shape without it means 1    */
+  /* 0, 1 or 2: accepted without effect                                       */
   int part12_waves_per_simd;
   void* stream;            /* hipStream_t; NULL = default stream                  */
   int async;               /* 1: return after enqueueing (status from p3x_sync)   */

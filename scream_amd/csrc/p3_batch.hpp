@@ -41,49 +41,28 @@ __device__ __forceinline__ int find_set(const int* __restrict__ first, int nsets
   return lo;
 }
 
-template <class R, int CB, int NT>
-__global__ __launch_bounds__(NT) void p3_part1_batch(const KParams* __restrict__ sets,
-                                                     const int* __restrict__ first, int nsets) {
-  __shared__ int s_i[NT];
-  const auto sets4 = (const __attribute__((address_space(4))) KParams*)sets;
-  const int total = first[nsets];
-  for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {
-    const int s = find_set(first, nsets, vb);
-    part1_block<R, CB, NT>(*(const KParams*)(sets4 + s), vb - first[s], s_i);
-  }
-}
-
-// Zeroes every set's column status words before p3_part1_lvl_batch: block b
-// takes sets b, b + gridDim.x, ...
+// Zeroes the column status words of the sets that keep them, before
+// p3_front_batch: block b takes sets b, b + gridDim.x, ...
 template <class R>
 __global__ __launch_bounds__(256) void p3_colstat_clear_batch(const KParams* __restrict__ sets, int nsets) {
   const auto sets4 = (const __attribute__((address_space(4))) KParams*)sets;
   for (int s = blockIdx.x; s < nsets; s += gridDim.x) {
     const KParams& p = *(const KParams*)(sets4 + s);
+    if (!p.track()) continue;
     for (int i = threadIdx.x; i < p.ncol; i += blockDim.x) p.colstat[i] = 0;
   }
 }
 
-// Part 1 one thread per (level, column); first: the pointwise tile offsets.
+// Parts 1 and 2; first: the pointwise tile offsets (pw_tiles per set).
 template <class R, bool PERSIST>
-__global__ __launch_bounds__(kTileThreads) void p3_part1_lvl_batch(const KParams* __restrict__ sets,
-                                                                   const int* __restrict__ first, int nsets) {
+__global__ __launch_bounds__(kTileThreads, kFrontWaves<R>) void p3_front_batch(const KParams* __restrict__ sets,
+                                                                               const int* __restrict__ first,
+                                                                               int nsets) {
+  __shared__ double s_lds[S_COUNT * kTileThreads];
   const auto sets4 = (const __attribute__((address_space(4))) KParams*)sets;
   for_virtual_blocks<PERSIST>(first[nsets], [&](int vb) {
     const int s = find_set(first, nsets, vb);
-    part1_tile<R>(*(const KParams*)(sets4 + s), vb - first[s]);
-  });
-}
-
-// first: the pointwise tile offsets (pw_tiles per set).
-template <class R, int WPE, bool PERSIST>
-__global__ __launch_bounds__(kPart2Cols * kPart2Levels, WPE) void p3_part2_batch(const KParams* __restrict__ sets,
-                                                                                const int* __restrict__ first,
-                                                                                int nsets) {
-  const auto sets4 = (const __attribute__((address_space(4))) KParams*)sets;
-  for_virtual_blocks<PERSIST>(first[nsets], [&](int vb) {
-    const int s = find_set(first, nsets, vb);
-    part2_tile<R>(*(const KParams*)(sets4 + s), vb - first[s]);
+    front_tile<R>(*(const KParams*)(sets4 + s), vb - first[s], s_lds);
   });
 }
 

@@ -1,25 +1,11 @@
-// p3_kernel.hpp -- p3_main_init, part 1 and part 2 of a P3 step (the first
-// two of its four kernels; sedimentation and part 3 are in p3_sed.hpp).
+// p3_kernel.hpp -- p3_main_init, part 1 and part 2 of a P3 step in one kernel
+// (sedimentation and part 3 are in p3_sed.hpp).
 //
-// Part 1 (part1_level) runs in one of two kernels:
-//  * p3_part1_lvl_kernel, one thread per (level, column) on the part 2 tiles
-//    below; the column's early-exit flag (nucleationPossible ||
-//    hydrometeorsPresent) is the OR of its levels' flags, set with atomicOr
-//    into status words p3_colstat_clear_kernel zeroed first;
-//  * p3_part1_kernel, a workgroup of CB consecutive columns whose NT threads
-//    split every column's levels into NCH = NT/CB contiguous chunks (thread t:
-//    column t % CB, chunk t / CB), the flag an OR-reduction through LDS.
-// Either way the column status goes to KParams::colstat.
-//
-// Part 2 (p3_part2_kernel): pointwise in the level once the column's part-1
-// status is known, so one thread per (level, column): a workgroup is 64
-// consecutive columns x 4 levels, one level per wavefront.  Every wavefront
-// then carries the same work whatever the column count, and a grid of ncol/64
-// x nlev/4 blocks keeps every CU busy to the end (one block of whole columns
-// per CU left most of the chip idle in a second, partial round).  A level
-// with hydrometeors after part 2 ORs bit 2 into its column's status, so the
-// sedimentation kernel sees 0 (skipped after part 1), 1 (after part 2) or 3
-// (full step).
+// Both parts are pointwise in the level, so p3_front_kernel runs them with one
+// thread per (level, column).  The reference's early exits are column-wide, but
+// nothing a point computes depends on them (front_level says why); the column
+// status words are kept only where a caller reads them or needs the exchange
+// fields untouched (KParams::track).
 //
 // The step follows components/eamxx/src/physics/p3/impl/p3_main_impl.hpp:74-260.
 #pragma once
@@ -28,10 +14,11 @@
 
 namespace p3d {
 
-// Scratch fields (ncol x nlev doubles each, in the layout of the column set)
-// that carry per-level results of part 1 to part 2 and to the sedimentation
-// kernel.
-enum Scr { SC_T = 0, SC_QVSL, SC_QVSI, SC_SUPI, SC_RHOFACR, SC_RHOFACI, SC_ACN, SC_COUNT };
+// Scratch fields (ncol x nlev doubles each, in the layout of the column set):
+// per-level results of part 1 for sedimentation and part 3 (T, rhofacr,
+// rhofaci, acn), and the marks of part 2's pending levels (SC_PEND, only
+// without exch_zero).  Room for SC_COUNT fields is reserved.
+enum Scr { SC_T = 0, SC_RHOFACR, SC_RHOFACI, SC_ACN, SC_PEND, SC_COUNT = 7 };
 
 // The P3Microphysics pre- and post-amble (eamxx_p3_process_interface.hpp:63-261),
 // fused into part 1 and part 3 when `on`.  The prognostic pointers then hold the
@@ -60,7 +47,7 @@ struct KParams {
   // P3HistoryOnly (in/out unless exch_zero)
   double *liq_ice_exchange, *vap_liq_exchange, *vap_ice_exchange;
   double* scratch;      // SC_COUNT fields of sfs doubles
-  int* colstat;         // per column: 0 skipped after part 1, 1 after part 2, 3 full step
+  int* colstat;         // per column: 0 skipped after part 1, 1 after part 2, 3 full step (if track())
   unsigned* err;        // device error word
   int *dbg_status, *dbg_substeps, *dbg_ice_idx;
   int* dbg_check;       // per column: check_values flags (NULL = the check is off)
@@ -83,6 +70,10 @@ struct KParams {
   double e_melt;        // saturation vapour pressure over liquid at Tmelt (qv_sat_dry(Tmelt, p) numerator)
   Amble amble;
 
+  // The step keeps the column status words: for the status array, for
+  // check_values (fully stepped columns only), or for exchange fields that a
+  // skipped column leaves as they were.
+  __host__ __device__ __forceinline__ bool track() const { return dbg_status || dbg_check || !exch_zero; }
   __host__ __device__ __forceinline__ size_t at(int i, int k) const { return (size_t)i * cs + (size_t)k * ks; }
   __host__ __device__ __forceinline__ size_t atf(int i, int k) const { return (size_t)i * fcs + (size_t)k * fks; }
   __host__ __device__ __forceinline__ double& sc(int f, int i, int k) const {
@@ -103,17 +94,40 @@ constexpr int kMaxSubsteps = 100000;
 // Column status bits: part 1 found work, part 2 left hydrometeors.
 constexpr int kStatusPart1 = 1, kStatusPart2 = 2, kStatusFull = 3;
 
-// p3_main_init + p3_main_part1 (P3I/p3_main_impl_part1.hpp:18-185) for level k of
-// column i; returns its flags: bit 0 nucleationPossible, bit 1 hydrometeorsPresent.
+// p3_main_init, part 1 (P3I/p3_main_impl_part1.hpp:18-185) and part 2
+// (P3I/p3_main_impl_part2.hpp:113-524) of level k of column i.
+//
+// The reference skips a column after part 1 unless some level of it has
+// hydrometeors or may nucleate ice (P3I/p3_main_impl.hpp:222-230), and after
+// part 2 unless some level has hydrometeors (:255-260).  A point needs neither:
+//  * a level with hydrometeors or possible nucleation (its own flag is set)
+//    makes its column run, so part 2 runs exactly there (unless skip_all);
+//  * a level without, in a column that runs because of other levels, is either
+//    skip_all or warm and clear; part 2 changes nothing at the latter (every
+//    tendency is zero) but zeroes its exchange fields.  Where those are not
+//    zeroed on entry, the level is marked pending in scratch and part 3, which
+//    knows the column's status, zeroes them;
+//  * sedimentation runs for a species that is present, and a level that has
+//    hydrometeors after part 2 makes its column run.
+//
+// What part 2 needs later than it is computed stays in LDS (s), not in
+// registers: 26 doubles per point.  Without that part 2 alone spilled at two
+// wavefronts per SIMD in FP64 and could not run at three in the mixed form.
+//
+// Bound by VALU issue: 66 % busy in FP64, 91 % in the mixed form.  As kernels of
+// their own, part 1 (at the HBM rate) wrote seven scratch fields and part 2
+// (43 % busy, waiting on loads) read them and the state again.  Together, at
+// 21600 x 72 FP64 48 + 187 -> 225 us, at 16384 x 128 mixed 67 + 189 -> 195 us,
+// and a launch (two with the status words' clear) fewer.
 template <class R>
-__device__ __forceinline__ int part1_level(const KParams& p, int k, int i, unsigned& err) {
+__device__ __forceinline__ void front_level(const KParams& p, int k, int i, const Pt s, int& stat, unsigned& err) {
   const double dt = p.dt;
   const double latvap = LatVap, latice = LatIce, inv_cp = INV_CP;
   const Runtime& rt = p.rt;
-  auto scr = [&](int f, int kk) -> double& { return p.sc(f, i, kk); };
   const size_t x = p.at(i, k);
-  int flags = 0;
-  double inv_exner, th, qv, qc, nc, qr, nr, qi, ni, qm, bm, dz, cfl;
+  int flags = 0;  // bit 0 nucleationPossible, bit 1 hydrometeorsPresent
+  double inv_exner, th, qv, qc, nc, qr, nr, qi, ni, qm, bm, dz;
+  double cfl = 1.0, cfr = 1.0, cfi = 1.0, qv_prev = 0, t_prev = 0, ni_act = 0;
   if (p.amble.on) {
     // p3_preamble, eamxx_p3_process_interface.hpp:63-124
     const Amble& a = p.amble;
@@ -130,16 +144,18 @@ __device__ __forceinline__ int part1_level(const KParams& p, int k, int i, unsig
     nr = to_dry(p.nr[x]); qi = to_dry(p.qi[x]); ni = to_dry(p.ni[x]);
     qm = to_dry(p.qm[x]); bm = to_dry(p.bm[x]);
     qv = to_dry(p.qv[x]);
-    a.qv_prev[x] = to_dry(a.qv_prev[x]);
+    qv_prev = to_dry(a.qv_prev[x]);
+    a.qv_prev[x] = qv_prev;
     const double ex = exner_function(pmid), rex = p3m_recip(ex);
     inv_exner = p3m_div_y(1.0, ex, rex);
     a.inv_exner[x] = inv_exner;
     th = p3m_div_y(T, ex, rex);
     // cloud fractions with the 1e-4 floor and the maximum-overlap rain fraction
     cfl = cft > 0.0001 ? cft : 0.0001;
+    cfi = cfl;
     a.cld_frac_l[x] = cfl;
     a.cld_frac_i[x] = cfl;
-    double cfr = cfl;
+    cfr = cfl;
     if (k != 0) {
       const double above = a.cldfrac_tot[x - p.ks];
       cfr = above > cfr ? above : cfr;
@@ -152,16 +168,31 @@ __device__ __forceinline__ int part1_level(const KParams& p, int k, int i, unsig
     qc = p.qc[x]; nc = p.nc[x]; qr = p.qr[x]; nr = p.nr[x];
     qi = p.qi[x]; ni = p.ni[x]; qm = p.qm[x]; bm = p.bm[x];
     dz = p.dz[x];
-    cfl = p.prescribedCCN ? p.cld_frac_l[x] : 1.0;
+    if (p.prescribedCCN) cfl = p.cld_frac_l[x];
   }
-  // the state as it is in memory: a field part 1 leaves bit for bit unchanged
-  // is not stored again (with the pre-amble every field changes to dry)
+  const double pres = p.pres[x], dpres = p.dpres[x];
+  // What only part 2 reads is requested as soon as the point is known to need
+  // it, and arrives while part 1 computes.
+  auto load_late = [&] {
+    if (!p.amble.on) {
+      cfl = p.cld_frac_l[x];
+      cfr = p.cld_frac_r[x];
+      cfi = p.cld_frac_i[x];
+      qv_prev = p.qv_prev[x];
+    }
+    t_prev = p.t_prev[x];
+    ni_act = p.ni_activated[x];
+  };
+  const bool wet = qc >= QSMALL || qr >= QSMALL || qi >= QSMALL;
+  if (wet) load_late();
+
+  // the state as it is in memory: a field left bit for bit unchanged is not
+  // stored again (with the pre-amble every field changes to dry)
   const double in[10] = {qc, nc, qr, nr, qi, ni, qm, bm, qv, th};
   qv = vmax(qv, 0.0);
   const double exner = p3m_div(1.0, inv_exner);
-  const double pres = p.pres[x];
   double T_atm = th * exner;
-  const double rho = air_density(p.dpres[x], dz);
+  const double rho = air_density(dpres, dz);
   const double inv_rho = p3m_div(1.0, rho);
   double qv_sat_l, qv_sat_i;
   qv_sat_dry_both(T_atm, pres, qv_sat_l, qv_sat_i, err);
@@ -207,64 +238,58 @@ __device__ __forceinline__ int part1_level(const KParams& p, int k, int i, unsig
   }
   T_atm = th * exner;
 
-  {
-    double* const f[10] = {p.qc, p.nc, p.qr, p.nr, p.qi, p.ni, p.qm, p.bm, p.qv, p.th};
-    const double out[10] = {qc, nc, qr, nr, qi, ni, qm, bm, qv, th};
+  p.sc(SC_T, i, k) = T_atm;
+  p.sc(SC_RHOFACR, i, k) = rhofacr;
+  p.sc(SC_RHOFACI, i, k) = rhofaci;
+  p.sc(SC_ACN, i, k) = acn;
+
+  // state fields to store: bit q for field q of f
+  unsigned chg = p.amble.on ? 0x3ffu : 0u;
+  double st[10] = {qc, nc, qr, nr, qi, ni, qm, bm, qv, th};
 #pragma unroll
-    for (int q = 0; q < 10; ++q)
-      if (p.amble.on || __double_as_longlong(out[q]) != __double_as_longlong(in[q])) f[q][x] = out[q];
+  for (int q = 0; q < 10; ++q)
+    if (__double_as_longlong(st[q]) != __double_as_longlong(in[q])) chg |= 1u << q;
+
+  const bool skip_all = qc < QSMALL && qr < QSMALL && qi < QSMALL && T_atm < T_zerodegc && qv_supersat_i < -0.05;
+  const bool done = flags && !skip_all;
+  if (p.track()) {
+    stat = flags ? kStatusPart1 : 0;
+    if (!p.exch_zero) p.sc(SC_PEND, i, k) = !flags && !skip_all ? 1.0 : 0.0;
   }
-  scr(SC_T, k) = T_atm;
-  scr(SC_QVSL, k) = qv_sat_l;
-  scr(SC_QVSI, k) = qv_sat_i;
-  scr(SC_SUPI, k) = qv_supersat_i;
-  scr(SC_RHOFACR, k) = rhofacr;
-  scr(SC_RHOFACI, k) = rhofaci;
-  scr(SC_ACN, k) = acn;
-  return flags;
-}
-
-// One block's work: columns bid*CB .. bid*CB+CB-1 of the column set p.
-// s_i is an LDS array of NT ints.
-template <class R, int CB, int NT>
-__device__ __forceinline__ void part1_block(const KParams& p, int bid, int* s_i) {
-  constexpr int NCH = NT / CB;
-  static_assert(NT % CB == 0, "block must hold whole chunk rows");
-
-  const int tid = threadIdx.x;
-  const int c = tid % CB;
-  const int ch = tid / CB;
-  const int i = bid * CB + c;
-  const bool col_ok = i < p.ncol;
-  const int nlev = p.nlev;
-  const int L = (nlev + NCH - 1) / NCH;
-  const int k0 = ch * L < nlev ? ch * L : nlev;
-  const int k1 = k0 + L < nlev ? k0 + L : nlev;
-  unsigned err = 0;
-
-  auto red_or = [&](int v) {
-    s_i[tid] = v;
-    __syncthreads();
-    int r = 0;
-    for (int j = 0; j < NCH; ++j) r |= s_i[j * CB + c];
-    __syncthreads();
-    return r;
-  };
-
-  int flags = 0;  // bit0 nucleationPossible, bit1 hydrometeorsPresent
-  if (col_ok) {
-    for (int k = k0; k < k1; ++k) flags |= part1_level<R>(p, k, i, err);
+  if (done) {
+    if (!wet) load_late();
+#pragma unroll
+    for (int q = 0; q < 10; ++q) s[S_QC + q] = st[q];
+    s[S_T] = T_atm; s[S_PRES] = pres; s[S_RHO] = rho; s[S_INV_RHO] = inv_rho;
+    s[S_QVSL] = qv_sat_l; s[S_QVSI] = qv_sat_i; s[S_SUPI] = qv_supersat_i;
+    s[S_RHOFACI] = rhofaci; s[S_ACN] = acn;
+    s[S_CFL] = cfl; s[S_CFR] = cfr; s[S_CFI] = cfi;
+    s[S_INV_EXNER] = inv_exner; s[S_QV_PREV] = qv_prev; s[S_T_PREV] = t_prev; s[S_NI_ACT] = ni_act;
+    lds_fence();
+    P2Out o;
+    // hydrometeorsPresent after part 2 (P3I/p3_main_impl.hpp:255-260): a column flag
+    if (part2_level<R>(rt, p.tab, dt, p.predictNc, p.prescribedCCN, p.e_melt, s, st, chg, o, err))
+      stat |= kStatusPart2;
+    p.qv2qi_depos_tend[x] = o.qv2qi_depos_tend;
+    p.precip_total_tend[x] = o.precip_total_tend;
+    p.nevapr[x] = o.nevapr;
+    p.vap_ice_exchange[x] = o.vap_ice_exchange;
+    p.vap_liq_exchange[x] = o.vap_liq_exchange;
+    p.liq_ice_exchange[x] = o.liq_ice_exchange;
+  } else {
+    p.qv2qi_depos_tend[x] = 0;
+    p.precip_total_tend[x] = 0;
+    p.nevapr[x] = 0;
+    if (p.exch_zero) {
+      p.vap_ice_exchange[x] = 0;
+      p.vap_liq_exchange[x] = 0;
+      p.liq_ice_exchange[x] = 0;
+    }
   }
-  const int cflags = red_or(flags);
-  if (col_ok && ch == 0) p.colstat[i] = (cflags & 3) ? kStatusPart1 : 0;
-  if (col_ok && ch == 0 && p.dbg_check) p.dbg_check[i] = 0;
-  if (err) atomicOr(p.err, err);
-}
-
-template <class R, int CB, int NT>
-__global__ __launch_bounds__(NT) void p3_part1_kernel(const KParams p) {
-  __shared__ int s_i[NT];
-  part1_block<R, CB, NT>(p, blockIdx.x, s_i);
+  double* const f[10] = {p.qc, p.nc, p.qr, p.nr, p.qi, p.ni, p.qm, p.bm, p.qv, p.th};
+#pragma unroll
+  for (int q = 0; q < 10; ++q)
+    if (chg >> q & 1) f[q][x] = st[q];
 }
 
 // Tiles of the pointwise kernels (part 1, part 2, part 3): 256 threads, one
@@ -273,9 +298,9 @@ __global__ __launch_bounds__(NT) void p3_part1_kernel(const KParams p) {
 //    columns fastest, so a wavefront reads 64 consecutive doubles of a row
 //    (and holds points of one level, whose work is alike);
 //  * column-major, two arrangements:
-//    - PW_RUNS (part 1, part 3, memory-bound): 256 consecutive points of the
+//    - PW_RUNS (part 3, memory-bound): 256 consecutive points of the
 //      column-by-column order, so a wavefront reads 512 contiguous bytes;
-//    - PW_BLOCKS (part 2): a wavefront holds 8 columns x 8 consecutive levels
+//    - PW_BLOCKS (parts 1 and 2): a wavefront holds 8 columns x 8 consecutive levels
 //      (levels fastest, 8 runs of 64 bytes per load), a block 32 columns x 8
 //      levels, so that a wavefront's points are of nearby levels: the upper
 //      levels are mostly dry and skip part 2's processes, and a wavefront
@@ -283,7 +308,8 @@ __global__ __launch_bounds__(NT) void p3_part1_kernel(const KParams p) {
 //      330 -> 270 us at 21600 x 72 against PW_RUNS).
 //    Both take the same grid (the larger of their tile counts); tiles past an
 //    arrangement's end hold no points.
-constexpr int kPart2Cols = 64, kPart2Levels = 4, kTileThreads = kPart2Cols * kPart2Levels;
+constexpr int kPart2Cols = 64, kPart2Levels = 4;
+static_assert(kTileThreads == kPart2Cols * kPart2Levels, "one point per thread");
 constexpr int kBlkCols = 32, kBlkLevels = 8;
 enum PwMap { PW_RUNS = 0, PW_BLOCKS = 1 };
 __host__ __device__ __forceinline__ int part2_tiles(int ncol, int nlev) {
@@ -347,27 +373,7 @@ __device__ __forceinline__ void colstat_or(const KParams& p, int i, int k, bool 
   if (set && !(m & run_below)) atomicOr(&p.colstat[i], bit);
 }
 
-// Part 1 with one thread per (level, column), on the pointwise tiles: a
-// column's status is the OR of its levels' flags, set atomically in a word that
-// p3_colstat_clear_kernel zeroed before.  Same per-level arithmetic as
-// part1_block; many more wavefronts, so the chip stays busy.
-template <class R>
-__device__ __forceinline__ void part1_tile(const KParams& p, int tile) {
-  int i, k;
-  if (!pw_point<PW_RUNS>(p, tile, i, k)) return;
-  unsigned err = 0;
-  const int flags = part1_level<R>(p, k, i, err);
-  colstat_or<PW_RUNS>(p, i, k, (flags & 3) != 0, kStatusPart1);
-  if (k == 0 && p.dbg_check) p.dbg_check[i] = 0;  // part 3 ORs the column's check_values flags
-  if (err) atomicOr(p.err, err);
-}
-
-template <class R>
-__global__ __launch_bounds__(kPart2Cols * kPart2Levels) void p3_part1_lvl_kernel(const KParams p) {
-  part1_tile<R>(p, blockIdx.x);
-}
-
-// Zeroes the column status words before p3_part1_lvl_kernel (templated only so
+// Zeroes the column status words before p3_front_kernel (templated only so
 // that each precision's translation unit has its own copy).
 template <class R>
 __global__ __launch_bounds__(256) void p3_colstat_clear_kernel(int* colstat, int n) {
@@ -375,83 +381,32 @@ __global__ __launch_bounds__(256) void p3_colstat_clear_kernel(int* colstat, int
   if (i < n) colstat[i] = 0;
 }
 
-// ================= p3_main_part2 (P3I/p3_main_impl_part2.hpp:113-524) for the
-// level of this wavefront and the column of this lane in tile `tile`.
+// Parts 1 and 2 on the pointwise tiles; s_lds holds S_COUNT * kTileThreads doubles.
 template <class R>
-__device__ __forceinline__ void part2_tile(const KParams& p, int tile) {
+__device__ __forceinline__ void front_tile(const KParams& p, int tile, double* s_lds) {
   int i, k;
   if (!pw_point<PW_BLOCKS>(p, tile, i, k)) return;
-  const size_t x = p.at(i, k);
-  auto scr = [&](int f) -> double { return p.sc(f, i, k); };
   unsigned err = 0;
-  bool done = false, hydro = false;
-  // The column status and the level's skip-test inputs are loaded together (one
-  // memory round trip for the decision); bit 1 only: other levels of the column
-  // may already have set bit 2.
-  {
-    Lvl s;
-    const int cstat = p.colstat[i];
-    s.qc = p.qc[x]; s.qr = p.qr[x]; s.qi = p.qi[x];
-    s.T_atm = scr(SC_T);
-    s.qv_supersat_i = scr(SC_SUPI);
-    const bool skip_all = s.qc < QSMALL && s.qr < QSMALL && s.qi < QSMALL && s.T_atm < T_zerodegc &&
-                          s.qv_supersat_i < -0.05;
-    if ((cstat & kStatusPart1) && !skip_all) {
-      s.nc = p.nc[x]; s.nr = p.nr[x]; s.qm = p.qm[x]; s.ni = p.ni[x]; s.bm = p.bm[x];
-      s.qv = p.qv[x]; s.th = p.th[x];
-      s.pres = p.pres[x];
-      s.rho = air_density(p.dpres[x], p.dz[x]);
-      s.inv_rho = p3m_div(1.0, s.rho);
-      s.qv_sat_l = scr(SC_QVSL);
-      s.qv_sat_i = scr(SC_QVSI);
-      s.rhofaci = scr(SC_RHOFACI);
-      s.acn = scr(SC_ACN);
-      s.cfl = p.cld_frac_l[x]; s.cfr = p.cld_frac_r[x]; s.cfi = p.cld_frac_i[x];
-      s.icfl = p3m_div(1.0, s.cfl); s.icfr = p3m_div(1.0, s.cfr); s.icfi = p3m_div(1.0, s.cfi);
-      s.inv_exner = p.inv_exner[x];
-      s.qv_prev = p.qv_prev[x]; s.t_prev = p.t_prev[x];
-      s.ni_activated = p.ni_activated[x];
-      const double in[10] = {s.qc, s.nc, s.qr, s.nr, s.qi, s.ni, s.qm, s.bm, s.qv, s.th};
-      // hydrometeorsPresent after part 2 (P3I/p3_main_impl.hpp:255-260): a column flag
-      hydro = part2_level<R>(p.rt, p.tab, p.dt, p.predictNc, p.prescribedCCN, p.e_melt, s, err);
-      {
-        // mixed form: a state field whose bits part 2 left unchanged is not stored
-        // again (in FP64 the ten held originals cost more registers than the
-        // stores they save)
-        double* const f[10] = {p.qc, p.nc, p.qr, p.nr, p.qi, p.ni, p.qm, p.bm, p.qv, p.th};
-        const double out[10] = {s.qc, s.nc, s.qr, s.nr, s.qi, s.ni, s.qm, s.bm, s.qv, s.th};
-#pragma unroll
-        for (int q = 0; q < 10; ++q)
-          if (sizeof(R) == 8 || __double_as_longlong(out[q]) != __double_as_longlong(in[q])) f[q][x] = out[q];
-      }
-      p.qv2qi_depos_tend[x] = s.qv2qi_depos_tend;
-      p.precip_total_tend[x] = s.precip_total_tend;
-      p.nevapr[x] = s.nevapr;
-      p.vap_ice_exchange[x] = s.vap_ice_exchange;
-      p.vap_liq_exchange[x] = s.vap_liq_exchange;
-      p.liq_ice_exchange[x] = s.liq_ice_exchange;
-      done = true;
-    }
+  int stat = 0;
+  front_level<R>(p, k, i, Pt{s_lds + threadIdx.x}, stat, err);
+  if (p.track()) {
+    colstat_or<PW_BLOCKS>(p, i, k, (stat & kStatusPart1) != 0, kStatusPart1);
+    colstat_or<PW_BLOCKS>(p, i, k, (stat & kStatusPart2) != 0, kStatusPart2);
+    if (k == 0 && p.dbg_check) p.dbg_check[i] = 0;  // part 3 ORs the column's check_values flags
   }
-  if (!done) {
-    p.qv2qi_depos_tend[x] = 0;
-    p.precip_total_tend[x] = 0;
-    p.nevapr[x] = 0;
-    if (p.exch_zero) {
-      p.vap_ice_exchange[x] = 0;
-      p.vap_liq_exchange[x] = 0;
-      p.liq_ice_exchange[x] = 0;
-    }
-  }
-  // hydrometeorsPresent after part 2 (P3I/p3_main_impl.hpp:255-260): a column flag
-  colstat_or<PW_BLOCKS>(p, i, k, hydro, kStatusPart2);
   if (err) atomicOr(p.err, err);
 }
 
-// WPE: minimum wavefronts per SIMD the register allocation must allow (1 or 2).
-template <class R, int WPE>
-__global__ __launch_bounds__(kPart2Cols * kPart2Levels, WPE) void p3_part2_kernel(const KParams p) {
-  part2_tile<R>(p, blockIdx.x);
+// Wavefronts per SIMD the front kernel is compiled for.  Two in FP64 (244
+// VGPRs; at three it spills 89 of them: 276 against 225 us at 21600 x 72), three
+// in the mixed form (164 VGPRs).  The LDS slots are 52 KB per block of four
+// wavefronts, so three blocks fit a CU.
+template <class R> constexpr int kFrontWaves = sizeof(R) == 8 ? 2 : 3;
+
+template <class R>
+__global__ __launch_bounds__(kTileThreads, kFrontWaves<R>) void p3_front_kernel(const KParams p) {
+  __shared__ double s_lds[S_COUNT * kTileThreads];
+  front_tile<R>(p, blockIdx.x, s_lds);
 }
 
 }  // namespace p3d

@@ -7,22 +7,13 @@
 
 namespace p3d {
 
-// Shape of one step's launches.
-//   part 1: p1lvl = 1, one thread per (level, column) on the pointwise tiles
-//     (pw_tiles); else cb columns per block x nt threads per block (compiled:
-//     16x128, 16x256, 32x256, 64x256, 32x512, 64x512);
-//   part 2: one thread per (level, column) on the pointwise tiles, register
-//     allocation for wpe = 1 or 2 wavefronts per SIMD (2: fewer registers,
-//     with spills in FP64);
-//   sedimentation, two kernels: the liquid group (cloud, rain) on lpc lanes
-//     per column and the ice group on lpc_ice (16, 32 or 64 each), each lane
-//     holding L = ceil(nlev / lanes) levels (at most 8), 4 wavefronts per
-//     block (the batched form runs both groups on lpc);
-//   part 3: one thread per (level, column) on the pointwise tiles.
+// Shape of one step's launches: the lanes per column of the sedimentation
+// kernels (16, 32 or 64), of the liquid group (cloud, rain) and of the ice
+// group; each lane holds L = ceil(nlev / lanes) levels (at most 8), 4 wavefronts
+// per block (the batched form runs both groups on lpc).  Parts 1 to 3 run one
+// thread per (level, column) on the pointwise tiles.
 struct Shape {
-  int cb, nt, lpc, wpe;
-  int p1lvl;    // 1: part 1 one thread per (level, column); 0: the cb x nt block kernel
-  int lpc_ice;  // lanes per column of the ice group's sedimentation kernel
+  int lpc, lpc_ice;
 };
 
 // Largest levels-per-lane count of the sedimentation kernel.
@@ -75,19 +66,19 @@ struct SedLaunch {
 };
 struct BatchPlan {
   Shape shape;
-  const KParams* sets;  // device array, all sets (part 1 and part 2 launches)
-  const int* first;     // device array, nsets + 1 entries: part 1 blocks
-  const int* first2;    // device array, nsets + 1 entries: pointwise tiles (parts 1 to 3)
+  const KParams* sets;  // device array, all sets (pointwise launches)
+  const int* first;     // device array, nsets + 1 entries: pointwise tiles (parts 1 to 3)
   int nsets;
-  int grid, grid2;      // blocks of the part 1 block kernel and of the pointwise launches
-  int total2;           // pointwise virtual blocks (first2[nsets]); grid2 >= total2: one block each, no loop
+  int track;            // some set keeps its column status words (KParams::track)
+  int grid;             // blocks of the pointwise launches
+  int total;            // pointwise virtual blocks (first[nsets]); grid >= total: one block each, no loop
   int nclass;
   SedClass cls[kMaxLevelsPerLane];
 };
 hipError_t launch_p3_batch_fp64(const BatchPlan& b, hipStream_t s);
 hipError_t launch_p3_batch_mixed(const BatchPlan& b, hipStream_t s);
 // Resident blocks per CU of the batched kernels for this shape (occupancy API).
-hipError_t occupancy_p3_fp64(const Shape& sh, int L, int* blocks1, int* blocks2, int* blocks_sed);
-hipError_t occupancy_p3_mixed(const Shape& sh, int L, int* blocks1, int* blocks2, int* blocks_sed);
+hipError_t occupancy_p3_fp64(const Shape& sh, int L, int* blocks, int* blocks_sed);
+hipError_t occupancy_p3_mixed(const Shape& sh, int L, int* blocks, int* blocks_sed);
 
 }  // namespace p3d

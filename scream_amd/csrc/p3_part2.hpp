@@ -10,32 +10,55 @@
 
 namespace p3d {
 
-// Per-level values p3_main_part2 reads and updates.
-struct Lvl {
-  // prognostic state (in/out)
-  double qc, nc, qr, nr, qi, qm, ni, bm, qv, th;
-  // part-1 quantities and inputs
-  double T_atm, pres, rho, inv_rho, qv_sat_l, qv_sat_i, qv_supersat_i, rhofaci, acn;
-  double cfl, cfr, cfi, icfl, icfr, icfi, inv_exner, qv_prev, t_prev, ni_activated;
-  // outputs
+// A point's values that part 2 reads at several places, far apart: one LDS slot
+// each, kTileThreads doubles per slot (conflict-free: a wavefront's lanes are
+// consecutive), this thread's at b[slot * kTileThreads].
+constexpr int kTileThreads = 256;
+enum Slot {
+  S_QC, S_NC, S_QR, S_NR, S_QI, S_NI, S_QM, S_BM, S_QV, S_TH,  // the state after part 1
+  S_T, S_PRES, S_RHO, S_INV_RHO, S_QVSL, S_QVSI, S_SUPI, S_RHOFACI, S_ACN,
+  S_CFL, S_CFR, S_CFI, S_INV_EXNER, S_QV_PREV, S_T_PREV, S_NI_ACT, S_COUNT
+};
+struct Pt {
+  double* b;
+  __device__ __forceinline__ double& operator[](int slot) const { return b[slot * kTileThreads]; }
+};
+// Keeps the compiler from carrying LDS values in registers across this point
+// (a thread reads only its own slots: no synchronisation is needed).
+__device__ __forceinline__ void lds_fence() { asm volatile("" ::: "memory"); }
+
+// The outputs of part 2.
+struct P2Out {
   double qv2qi_depos_tend, precip_total_tend, nevapr;
   double vap_ice_exchange, vap_liq_exchange, liq_ice_exchange;
 };
 
 // Returns true when a hydrometeor survives the end-of-part-2 clipping at this
 // level (the per-level contribution to hydrometeorsPresent, :465-508).
+// st is the state after part 2 (qc nc qr nr qi ni qm bm qv th); a bit of chg is
+// set for each of its fields that differs from the one after part 1.
 template <class R>
-__device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool predictNc,
-                            bool prescribedCCN, double e_melt, Lvl& s, unsigned& err) {
+__device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool predictNc,
+                                            bool prescribedCCN, double e_melt, const Pt s, double (&st)[10],
+                                            unsigned& chg, P2Out& o, unsigned& err) {
   const double inv_dt = 1 / dt;
   const double latvap = LatVap, latice = LatIce, inv_cp = INV_CP;
-  const double T_atm = s.T_atm, rho = s.rho, inv_rho = s.inv_rho, pres = s.pres;
-  const double cld_frac_l = s.cfl, cld_frac_r = s.cfr, cld_frac_i = s.cfi;
 
+  // rewrites a state slot
+  auto put = [&](int slot, double v) {
+    if (__double_as_longlong(v) != __double_as_longlong(s[slot])) chg |= 1u << (slot - S_QC);
+    s[slot] = v;
+  };
   // in-cloud values on entry: calculate_incloud_mixingratios of the current state
-  const Incld in0 = incloud(s.qc, s.qr, s.qi, s.qm, s.nc, s.nr, s.ni, s.bm, s.icfl, s.icfi, s.icfr);
-  R qc_incld = R(in0.qc), qr_incld = R(in0.qr), qi_incld = R(in0.qi), qm_incld = R(in0.qm);
-  R nc_incld = R(in0.nc), nr_incld = R(in0.nr), ni_incld = R(in0.ni), bm_incld = R(in0.bm);
+  R qc_incld, qr_incld, qi_incld, qm_incld, nc_incld, nr_incld, ni_incld, bm_incld;
+  double qr_incld_d;
+  {
+    const Incld in0 = incloud(s[S_QC], s[S_QR], s[S_QI], s[S_QM], s[S_NC], s[S_NR], s[S_NI], s[S_BM],
+                              p3m_div(1.0, s[S_CFL]), p3m_div(1.0, s[S_CFI]), p3m_div(1.0, s[S_CFR]));
+    qc_incld = R(in0.qc); qr_incld = R(in0.qr); qi_incld = R(in0.qi); qm_incld = R(in0.qm);
+    nc_incld = R(in0.nc); nr_incld = R(in0.nr); ni_incld = R(in0.ni); bm_incld = R(in0.bm);
+    qr_incld_d = in0.qr;
+  }
 
   R qc2qr_accret_tend = 0, qc2qr_autoconv_tend = 0, nc_accret_tend = 0,
     nc_selfcollect_tend = 0, nc2nr_autoconv_tend = 0, nr_selfcollect_tend = 0, ncautr = 0;
@@ -49,19 +72,20 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
   bool wetgrowth = false;
   R mu_c = 0, lamc = 0, cdist = 0, cdist1 = 0, mu_r = 0, lamr = 0, cdistr = 0, logn0r = 0;
 
+  const double T_atm = s[S_T];
   const bool skip_micro = !(qc_incld >= R(QSMALL) || qr_incld >= R(QSMALL) || qi_incld >= R(QSMALL));
   if (!skip_micro) {
-    const R Tr = R(T_atm), rhor = R(rho), rhofaci = R(s.rhofaci);
+    const R Tr = R(T_atm), rhor = R(s[S_RHO]), rhofaci = R(s[S_RHOFACI]);
     const R dT_melt = R(T_atm - Tmelt);  // FP64 difference (exact in the FP64 form)
     // get_time_space_phys_variables, P3I/p3_get_time_space_phys_variables_impl.hpp:10-46
     R T15, T181;  // T^1.5, T^1.81
     pow_15_181(Tr, T15, T181);
     const R mu = m_div(R(1.496e-6) * T15, Tr + R(120));
-    const R dv = m_div(R(8.794e-5) * T181, R(pres));
+    const R dv = m_div(R(8.794e-5) * T181, R(s[S_PRES]));
     const R sc = m_div(mu, rhor * dv);
     const R dum_t = m_div(R(1), R(RV) * (Tr * Tr));
-    const R dqsdt = R(latvap) * R(s.qv_sat_l) * dum_t;
-    const R dqsidt = R(latvap + latice) * R(s.qv_sat_i) * dum_t;
+    const R dqsdt = R(latvap) * R(s[S_QVSL]) * dum_t;
+    const R dqsidt = R(latvap + latice) * R(s[S_QVSI]) * dum_t;
     const R ab = R(1) + dqsdt * R(latvap) * R(INV_CP);
     const R abi = R(1) + dqsidt * R(latvap + latice) * R(INV_CP);
     const R kap = R(1.414e+3) * mu;
@@ -71,7 +95,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     else eii = R(0.3);
 
     get_cloud_dsd2<R>(qc_incld, nc_incld, mu_c, rhor, lamc, cdist, cdist1);
-    s.nc = double(nc_incld) * cld_frac_l;
+    put(S_NC, double(nc_incld) * s[S_CFL]);
 
     get_rain_dsd2<R>(rt, qr_incld, nr_incld, mu_r, lamr);
     // get_cdistr_logn0r, P3I/p3_dsd2_impl.hpp:128-148
@@ -79,9 +103,9 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
       cdistr = m_div(nr_incld, m_tgamma(mu_r + R(1)));
       logn0r = m_log10(cdistr) + (mu_r + R(1)) * m_log10(lamr);
     }
-    s.nr = double(nr_incld) * cld_frac_r;
+    put(S_NR, double(nr_incld) * s[S_CFR]);
 
-    impose_max_total_ni<R>(ni_incld, R(rt.max_total_ni), R(inv_rho));
+    impose_max_total_ni<R>(ni_incld, R(rt.max_total_ni), R(s[S_INV_RHO]));
 
     R tv_qi_fallspd = 0, tv_ni_self_collect = 0, tv_qc2qi_collect = 0, tv_qi2qr_melting = 0,
       tv_nr_collect = 0, tv_qr2qi_collect = 0, tv_lammax = 0, tv_lammin = 0, tv_vent_melt = 0;
@@ -89,8 +113,9 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
       ni_incld = vmax(ni_incld, R(NSMALL));
       nr_incld = vmax(nr_incld, R(NSMALL));
       const R rhop = calc_bulk_rho_rime<R>(rt, qi_incld, qm_incld, bm_incld);
-      s.qm = double(qm_incld) * cld_frac_i;
-      s.bm = double(bm_incld) * cld_frac_i;
+      const double cld_frac_i = s[S_CFI];
+      put(S_QM, double(qm_incld) * cld_frac_i);
+      put(S_BM, double(bm_incld) * cld_frac_i);
       const TabIce<R> ti = lookup_ice<R>(qi_incld, ni_incld, qm_incld, rhop);
       const TabRain<R> tr = lookup_rain<R>(qr_incld, nr_incld);
       // ice quantities 1,2,3,4 then 6,7,9 of the part 2 records (in FP64 two at a
@@ -178,8 +203,8 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
 
     // ice_melting, P3I/p3_ice_melting_impl.hpp:11-52
     if (qi_incld >= R(QSMALL) && T_atm > Tmelt) {
-      const double qsat0 = ep_2 * e_melt / vmax(pres, 1.e-3);  // qv_sat_dry(Tmelt, pres, liquid)
-      const R dqs = R(qsat0 - s.qv);
+      const double qsat0 = p3m_div(ep_2 * e_melt, vmax(s[S_PRES], 1.e-3));  // qv_sat_dry(Tmelt, pres, liquid)
+      const R dqs = R(qsat0 - s[S_QV]);
       qi2qr_melt_tend = (vent * (dT_melt * kap - rhor * R(latvap) * dv * dqs) * R(2) * R(Pi) / R(latice)) * ni_incld;
       qi2qr_melt_tend = vmax(qi2qr_melt_tend, R(0));
       ni2nr_melt_tend = qi2qr_melt_tend * m_div(ni_incld, qi_incld);
@@ -191,8 +216,8 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
       const bool any_if = qi_incld >= R(QSMALL) && (qc_incld + qr_incld) >= R(1.0e-6) && t_is_negative;
       const bool any_if_col = any_if && (qc2qi_collect_tend + qr2qi_collect_tend) >= R(1.0e-10);
       if (any_if) {
-        const double qsat0 = ep_2 * e_melt / vmax(pres, 1.e-3);  // qv_sat_dry(Tmelt, pres, liquid)
-        const R dqs = R(qsat0 - s.qv);
+        const double qsat0 = p3m_div(ep_2 * e_melt, vmax(s[S_PRES], 1.e-3));  // qv_sat_dry(Tmelt, pres, liquid)
+        const R dqs = R(qsat0 - s[S_QV]);
         R qc_growth_rate = (vent * R(Pi * 2) * (rhor * R(latvap) * dv * dqs - dT_melt * kap) /
                             (R(latice) + R(CpLiq) * dT_melt)) * ni_incld;
         qc_growth_rate = vmax(qc_growth_rate, R(0.0));
@@ -222,7 +247,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     if (qc2qi_collect_tend >= R(QSMALL) && T_atm < T_zerodegc) {
       const R vtrmi1 = tv_qi_fallspd * rhofaci;
       if (qc_incld >= R(QSMALL)) {
-        const R Vt_qc = m_div(R(s.acn) * m_tgamma(R(4 + bcn) + mu_c), m_pow(lamc, R(bcn)) * m_tgamma(R(4) + mu_c));
+        const R Vt_qc = m_div(R(s[S_ACN]) * m_tgamma(R(4 + bcn) + mu_c), m_pow(lamc, R(bcn)) * m_tgamma(R(4) + mu_c));
         const R D_c = m_div(R(4) + mu_c, lamc);
         const R V_impact = m_fabs(vtrmi1 - Vt_qc);
         const R inv_Tc = m_div(R(1), vmin(R(-0.001), R(T_atm - T_zerodegc)));
@@ -267,20 +292,20 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
 
     // evaporate_rain, P3I/p3_evaporate_rain_impl.hpp:83-201
     {
-      const double ssat_r_d = s.qv - s.qv_sat_l;  // FP64 difference of near-equal values
+      const double ssat_r_d = s[S_QV] - s[S_QVSL];  // FP64 difference of near-equal values
       const R ssat_r = R(ssat_r_d);
-      const R cld_frac = ((qc_incld + qi_incld) < R(1.e-6)) ? R(0) : R(cld_frac_l);
-      const R cfr = R(cld_frac_r);
+      const R cld_frac = ((qc_incld + qi_incld) < R(1.e-6)) ? R(0) : R(s[S_CFL]);
+      const R cfr = R(s[S_CFR]);
       if (qr_incld >= R(QSMALL) && ssat_r_d < 0 && cfr > cld_frac) {
         const R inv_dt_r = R(1 / dt);
         const R tau_r = m_div(R(1), epsr);
-        const R dqv_dt = R((s.qv - s.qv_prev) * (1 / dt));
-        const R dT = R(T_atm - s.t_prev);
+        const R dqv_dt = R((s[S_QV] - s[S_QV_PREV]) * (1 / dt));
+        const R dT = R(T_atm - s[S_T_PREV]);
         R eps_eff, A_c;
         if (T_atm < Tmelt) {
           const R fac = R(1) + R(latvap + latice) * R(1 / Cpair) * dqsdt;
           eps_eff = epsr + m_div(epsi_tot * fac, abi);
-          A_c = dqv_dt - dqsdt * dT * inv_dt_r - m_div(R(s.qv_sat_l - s.qv_sat_i) * fac, abi) * epsi_tot;
+          A_c = dqv_dt - dqsdt * dT * inv_dt_r - m_div(R(s[S_QVSL] - s[S_QVSI]) * fac, abi) * epsi_tot;
         } else {
           eps_eff = epsr;
           A_c = dqv_dt - dqsdt * dT * inv_dt_r;
@@ -290,10 +315,9 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
         // The limits below can remove all rain; they run in FP64 on the FP64
         // in-cloud mass (qr_incld is unchanged since entry) so that complete
         // evaporation leaves the same clipped residual in both forms.
-        const double qr_incld_d = in0.qr;
         const double inv_dt_d = 1 / dt;
         double ev;
-        if (qr_incld < R(1e-12) && p3m_div(s.qv, s.qv_sat_l) < 0.999) {
+        if (qr_incld < R(1e-12) && p3m_div(s[S_QV], s[S_QVSL]) < 0.999) {
           ev = qr_incld_d * inv_dt_d;
         } else {
           const R dt_over_tau = m_div(R(dt), tau_eff);
@@ -307,7 +331,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
         if (ev > ev_max) ev = ev_max;
         if (ev < 0) ev = 0;
         if (ev > qr_incld_d * inv_dt_d) ev = qr_incld_d * inv_dt_d;
-        ev = p3m_div(ev * (cld_frac_r - cfd), cld_frac_r);
+        ev = p3m_div(ev * (s[S_CFR] - cfd), s[S_CFR]);
         evap_d = ev;
         nr_evap_d = ev * p3m_div(double(nr_incld), qr_incld_d);
       }
@@ -317,14 +341,14 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
       // ice_deposition_sublimation, P3I/p3_ice_deposition_sublimation_impl.hpp:10-65
       if (qi_incld > R(QSMALL)) {
         const R epsi_abi = m_div(epsi, abi);
-        const R qi_tend = vmin(epsi_abi, R(inv_dt)) * R(s.qv - s.qv_sat_i);
+        const R qi_tend = vmin(epsi_abi, R(inv_dt)) * R(s[S_QV] - s[S_QVSI]);
         const bool neg = qi_tend < R(0);
         if (neg) {
           qi2qv_sublim_tend = -qi_tend;
           ni_sublim_tend = qi2qv_sublim_tend * m_div(ni_incld, qi_incld);
         }
         if (T_atm < T_zerodegc && !neg) qv2qi_vapdep_tend = qi_tend;
-        if (T_atm < T_zerodegc) qc2qi_berg_tend = vmax(epsi_abi * R(s.qv_sat_l - s.qv_sat_i), R(0));
+        if (T_atm < T_zerodegc) qc2qi_berg_tend = vmax(epsi_abi * R(s[S_QVSL] - s[S_QVSI]), R(0));
       }
     }
   }  // !skip_micro
@@ -333,22 +357,22 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
   if (rt.do_ice_production) {
     const R mi0 = R(4.0 * PIOV3 * 900.0 * 1.e-18);
     const bool lt = T_atm < (Tmelt - 15.0);
-    const bool ge = s.qv_supersat_i >= 0.05;
+    const bool ge = s[S_SUPI] >= 0.05;
     const bool do_log = (!predictNc || prescribedCCN);
     const bool any_if_log = lt && ge && !do_log;
     const bool any_if_not_log = lt && ge && do_log;
     if (any_if_not_log) {
-      const R ir = R(inv_rho);
+      const R ir = R(s[S_INV_RHO]);
       R dum = R(0.005) * m_exp(R(rt.deposition_nucleation_exponent) * R(Tmelt - T_atm)) * R(1.0e3) * ir;
       dum = vmin(dum, R(1.0e5) * ir);
-      const R N_nuc = vmax(R(0.0), (dum - R(s.ni)) * R(inv_dt));
+      const R N_nuc = vmax(R(0.0), (dum - R(s[S_NI])) * R(inv_dt));
       if (N_nuc >= R(NSMALL)) {
-        const R Q_nuc = vmax(R(0.0), (dum - R(s.ni)) * mi0 * R(inv_dt));
+        const R Q_nuc = vmax(R(0.0), (dum - R(s[S_NI])) * mi0 * R(inv_dt));
         qv2qi_nucleat_tend = Q_nuc;
         ni_nucleat_tend = N_nuc;
       }
     } else if (any_if_log) {
-      ni_nucleat_tend = vmax(R(0.0), R((s.ni_activated - s.ni) * inv_dt));
+      ni_nucleat_tend = vmax(R(0.0), R((s[S_NI_ACT] - s[S_NI]) * inv_dt));
       qv2qi_nucleat_tend = ni_nucleat_tend * mi0;
     }
   }
@@ -359,7 +383,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     const R cons3 = R((radius == 25.0e-6) ? CONS3 : 1.0 / (CONS2 * p3m_pow(radius, 3.0)));
     if (qc_incld >= R(1e-8)) {
       qc2qr_autoconv_tend = R(1.0) * R(rt.autoconversion_prefactor) * m_pow(qc_incld, R(rt.autoconversion_qc_exponent)) *
-                            m_pow(nc_incld * R(1.e-6) * R(rho), R(-rt.autoconversion_nc_exponent));
+                            m_pow(nc_incld * R(1.e-6) * R(s[S_RHO]), R(-rt.autoconversion_nc_exponent));
       ncautr = qc2qr_autoconv_tend * cons3;
       nc2nr_autoconv_tend = m_div(qc2qr_autoconv_tend * nc_incld, qc_incld);
     }
@@ -385,10 +409,18 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     R dum;
     if (dum2 < bd) dum = R(1);
     else dum = R(2) - m_exp(R(2300) * (dum2 - bd));
-    nr_selfcollect_tend = dum * R(rt.rain_selfcollection_prefactor) * nr_incld * qr_incld * R(rho);
+    nr_selfcollect_tend = dum * R(rt.rain_selfcollection_prefactor) * nr_incld * qr_incld * R(s[S_RHO]);
   }
 
   // ---------------- FP64 from here: cell averages, limiters, updates ----------------
+  lds_fence();
+  struct {
+    double qc, nc, qr, nr, qi, ni, qm, bm, qv, th;
+  } u;  // the state being updated
+  // (S_NC, S_NR, S_QM and S_BM: as rewritten above)
+  u.qc = s[S_QC]; u.nc = s[S_NC]; u.qr = s[S_QR]; u.nr = s[S_NR]; u.qi = s[S_QI]; u.ni = s[S_NI];
+  u.qm = s[S_QM]; u.bm = s[S_BM]; u.qv = s[S_QV]; u.th = s[S_TH];
+  const double cld_frac_l = s[S_CFL], cld_frac_r = s[S_CFR], cld_frac_i = s[S_CFI];
   double t_qc2qr_accret = qc2qr_accret_tend, t_qr2qv_evap = evap_d,
          t_qc2qr_autoconv = qc2qr_autoconv_tend, t_nc_accret = nc_accret_tend,
          t_nc_selfcollect = nc_selfcollect_tend, t_nc2nr_autoconv = nc2nr_autoconv_tend,
@@ -442,7 +474,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
   {
     const double sinks = (t_qc2qr_autoconv + t_qc2qr_accret + t_qc2qi_collect + t_qc2qi_hetero + t_qc2qr_ice_shed +
                           t_qc2qi_berg) * dt;
-    const double sources = s.qc;
+    const double sources = u.qc;
     double ratio;
     if (sinks > sources && sinks >= QTENDSMALL) {
       ratio = p3m_div(sources, sinks);
@@ -463,7 +495,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
   // rain_water_conservation, P3I/p3_conservation_impl.hpp:42-65
   {
     const double sinks = (t_qr2qv_evap + t_qr2qi_collect + t_qr2qi_immers) * dt;
-    const double sources = s.qr + (t_qc2qr_autoconv + t_qc2qr_accret + t_qi2qr_melt + t_qc2qr_ice_shed) * dt;
+    const double sources = u.qr + (t_qc2qr_autoconv + t_qc2qr_accret + t_qi2qr_melt + t_qc2qr_ice_shed) * dt;
     if (sinks > sources && sinks >= QTENDSMALL) {
       const double ratio = p3m_div(sources, sinks);
       t_qr2qv_evap *= ratio;
@@ -474,7 +506,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
   // ice_water_conservation, P3I/p3_conservation_impl.hpp:67-96
   {
     const double sinks = (t_qi2qv_sublim + t_qi2qr_melt) * dt;
-    const double sources = s.qi + (t_qv2qi_vapdep + t_qv2qi_nucleat + t_qr2qi_collect + t_qc2qi_collect + t_qr2qi_immers +
+    const double sources = u.qi + (t_qv2qi_vapdep + t_qv2qi_nucleat + t_qr2qi_collect + t_qc2qi_collect + t_qr2qi_immers +
                                    t_qc2qi_hetero + t_qc2qi_berg) * dt;
     if (sinks > sources && sinks >= QTENDSMALL) {
       const double ratio = p3m_div(sources, sinks);
@@ -485,7 +517,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
   // nc_conservation, P3I/p3_nc_conservation_impl.hpp:16-28
   {
     const double sink_nc = (t_nc_collect + t_nc2ni_immers + t_nc_accret + t_nc2nr_autoconv) * dt;
-    const double source_nc = s.nc + t_nc_selfcollect * dt;
+    const double source_nc = u.nc + t_nc_selfcollect * dt;
     if (sink_nc > source_nc) {
       const double ratio = source_nc / sink_nc;
       t_nc_collect *= ratio;
@@ -497,7 +529,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
   // nr_conservation, P3I/p3_nr_conservation_impl.hpp:16-28
   {
     const double sink_nr = (t_nr_collect + t_nr2ni_immers + t_nr_selfcollect + t_nr_evap) * dt;
-    const double source_nr = s.nr + (t_ni2nr_melt * nmltratio + t_nr_ice_shed + t_ncshdc + t_nc2nr_autoconv) * dt;
+    const double source_nr = u.nr + (t_ni2nr_melt * nmltratio + t_nr_ice_shed + t_ncshdc + t_nc2nr_autoconv) * dt;
     if (sink_nr > source_nr) {
       const double ratio = source_nr / sink_nr;
       t_nr_collect *= ratio;
@@ -509,7 +541,7 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
   // ni_conservation, P3I/p3_ni_conservation_impl.hpp:16-27
   {
     const double sink_ni = (t_ni2nr_melt + t_ni_sublim + t_ni_selfcollect) * dt;
-    const double source_ni = s.ni + (t_ni_nucleat + t_nr2ni_immers + t_nc2ni_immers) * dt;
+    const double source_ni = u.ni + (t_ni_nucleat + t_nr2ni_immers + t_nc2ni_immers) * dt;
     if (sink_ni > source_ni) {
       const double ratio = source_ni / sink_ni;
       t_ni2nr_melt *= ratio;
@@ -519,12 +551,12 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
   }
   // ice_supersat_conservation, P3I/p3_ice_supersat_conservation_impl.hpp:14-43
   {
-    const double t_atm = p3m_div(s.th, s.inv_exner);
+    const double t_atm = p3m_div(u.th, s[S_INV_EXNER]);
     const double latsublim2 = (latvap + latice) * (latvap + latice);
     const double qv_sink = t_qv2qi_vapdep + t_qv2qi_nucleat;
     if (qv_sink > QSMALL && cld_frac_i > 1e-20) {
-      double qv_avail = p3m_div(p3m_div(s.qv + (t_qi2qv_sublim + t_qr2qv_evap) * dt - s.qv_sat_i,
-                                        1 + p3m_div(latsublim2 * s.qv_sat_i, CP * RH2O * (t_atm * t_atm))), dt);
+      double qv_avail = p3m_div(p3m_div(u.qv + (t_qi2qv_sublim + t_qr2qv_evap) * dt - s[S_QVSI],
+                                        1 + p3m_div(latsublim2 * s[S_QVSI], CP * RH2O * (t_atm * t_atm))), dt);
       qv_avail = vmax(qv_avail, 0.0);
       if (qv_sink > qv_avail) {
         const double fract = p3m_div(qv_avail, qv_sink);
@@ -538,12 +570,12 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
     const double qv_sources = t_qi2qv_sublim + t_qr2qv_evap;
     if (qv_sources >= QSMALL) {
       const double qv_sinks = t_qv2qi_vapdep + t_qv2qi_nucleat;
-      const double T_endstep = T_atm + ((qv_sinks - t_qi2qv_sublim) * (latvap + latice) * inv_cp -
+      const double T_endstep = s[S_T] + ((qv_sinks - t_qi2qv_sublim) * (latvap + latice) * inv_cp -
                                         t_qr2qv_evap * latvap * inv_cp) * dt;
-      const double qsl = qv_sat_dry_liquid(T_endstep, pres, err);
+      const double qsl = qv_sat_dry_liquid(T_endstep, s[S_PRES], err);
       const double A = p3m_div(latvap * qsl * dt * inv_cp, RV * T_endstep * T_endstep) *
                        ((latvap + latice) * t_qi2qv_sublim + latvap * t_qr2qv_evap);
-      double frac = p3m_div(qsl - s.qv + qv_sinks * dt + A, qv_sources * dt + A);
+      double frac = p3m_div(qsl - u.qv + qv_sinks * dt + A, qv_sources * dt + A);
       frac = vmax(0.0, frac);
       frac = vmin(1.0, frac);
       t_qi2qv_sublim = frac * t_qi2qv_sublim;
@@ -553,69 +585,76 @@ __device__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool
 
   // update_prognostic_ice, P3I/p3_update_prognostics_impl.hpp:9-87
   {
-    const double inv_exner = s.inv_exner;
-    s.qc = s.qc + (-t_qc2qi_hetero - t_qc2qi_collect - t_qc2qr_ice_shed - t_qc2qi_berg) * dt;
-    if (predictNc) s.nc = s.nc + (-t_nc_collect - t_nc2ni_immers) * dt;
-    s.qr = s.qr + (-t_qr2qi_collect + t_qi2qr_melt - t_qr2qi_immers + t_qc2qr_ice_shed) * dt;
-    s.nr = s.nr + (-t_nr_collect - t_nr2ni_immers + nmltratio * t_ni2nr_melt + t_nr_ice_shed + t_ncshdc) * dt;
-    if (s.qi >= QSMALL) {
-      const double rqi = p3m_recip(s.qi);
-      s.bm = s.bm - p3m_div_y(t_qi2qv_sublim + t_qi2qr_melt, s.qi, rqi) * dt * s.bm;
-      s.qm = s.qm - p3m_div_y((t_qi2qv_sublim + t_qi2qr_melt) * s.qm, s.qi, rqi) * dt;
-      s.qi = s.qi - (t_qi2qv_sublim + t_qi2qr_melt) * dt;
+    const double inv_exner = s[S_INV_EXNER];
+    u.qc = u.qc + (-t_qc2qi_hetero - t_qc2qi_collect - t_qc2qr_ice_shed - t_qc2qi_berg) * dt;
+    if (predictNc) u.nc = u.nc + (-t_nc_collect - t_nc2ni_immers) * dt;
+    u.qr = u.qr + (-t_qr2qi_collect + t_qi2qr_melt - t_qr2qi_immers + t_qc2qr_ice_shed) * dt;
+    u.nr = u.nr + (-t_nr_collect - t_nr2ni_immers + nmltratio * t_ni2nr_melt + t_nr_ice_shed + t_ncshdc) * dt;
+    if (u.qi >= QSMALL) {
+      const double rqi = p3m_recip(u.qi);
+      u.bm = u.bm - p3m_div_y(t_qi2qv_sublim + t_qi2qr_melt, u.qi, rqi) * dt * u.bm;
+      u.qm = u.qm - p3m_div_y((t_qi2qv_sublim + t_qi2qr_melt) * u.qm, u.qi, rqi) * dt;
+      u.qi = u.qi - (t_qi2qv_sublim + t_qi2qr_melt) * dt;
     }
     const double dum = (t_qr2qi_collect + t_qc2qi_collect + t_qr2qi_immers + t_qc2qi_hetero) * dt;
-    s.qi = s.qi + (t_qv2qi_vapdep + t_qv2qi_nucleat + t_qc2qi_berg) * dt + dum;
-    s.qm = s.qm + dum;
-    s.bm = s.bm + (t_qr2qi_collect * INV_RHO_RIMEMAX + p3m_div(t_qc2qi_collect, rho_qm_cloud) +
+    u.qi = u.qi + (t_qv2qi_vapdep + t_qv2qi_nucleat + t_qc2qi_berg) * dt + dum;
+    u.qm = u.qm + dum;
+    u.bm = u.bm + (t_qr2qi_collect * INV_RHO_RIMEMAX + p3m_div(t_qc2qi_collect, rho_qm_cloud) +
                    (t_qr2qi_immers + t_qc2qi_hetero) * INV_RHO_RIMEMAX) * dt;
-    s.ni = s.ni + (t_ni_nucleat - t_ni2nr_melt - t_ni_sublim - t_ni_selfcollect + t_nr2ni_immers + t_nc2ni_immers) * dt;
-    if (s.qm < 0) { s.qm = 0; s.bm = 0; }
-    if (wetgrowth) { s.qm = s.qi; s.bm = s.qm * INV_RHO_RIMEMAX; }
-    s.qv = s.qv + (-t_qv2qi_vapdep + t_qi2qv_sublim - t_qv2qi_nucleat) * dt;
-    s.th = s.th + inv_exner * ((t_qv2qi_vapdep - t_qi2qv_sublim + t_qv2qi_nucleat) * (latvap + latice) * INV_CP +
+    u.ni = u.ni + (t_ni_nucleat - t_ni2nr_melt - t_ni_sublim - t_ni_selfcollect + t_nr2ni_immers + t_nc2ni_immers) * dt;
+    if (u.qm < 0) { u.qm = 0; u.bm = 0; }
+    if (wetgrowth) { u.qm = u.qi; u.bm = u.qm * INV_RHO_RIMEMAX; }
+    u.qv = u.qv + (-t_qv2qi_vapdep + t_qi2qv_sublim - t_qv2qi_nucleat) * dt;
+    u.th = u.th + inv_exner * ((t_qv2qi_vapdep - t_qi2qv_sublim + t_qv2qi_nucleat) * (latvap + latice) * INV_CP +
                                (t_qr2qi_collect + t_qc2qi_collect + t_qc2qi_hetero + t_qr2qi_immers - t_qi2qr_melt +
                                 t_qc2qi_berg) * latice * INV_CP) * dt;
 
     // update_prognostic_liquid, P3I/p3_update_prognostics_impl.hpp:89-122
-    s.qc = s.qc + (-t_qc2qr_accret - t_qc2qr_autoconv) * dt;
-    s.qr = s.qr + (t_qc2qr_accret + t_qc2qr_autoconv - t_qr2qv_evap) * dt;
-    if (predictNc || prescribedCCN) s.nc = s.nc + (-t_nc_accret - t_nc2nr_autoconv + t_nc_selfcollect) * dt;
-    else s.nc = NCCNST * inv_rho;
-    s.nr = s.nr + (t_ncautr - t_nr_selfcollect - t_nr_evap) * dt;
-    s.qv = s.qv + t_qr2qv_evap * dt;
-    s.th = s.th + inv_exner * (-t_qr2qv_evap * latvap * INV_CP) * dt;
+    u.qc = u.qc + (-t_qc2qr_accret - t_qc2qr_autoconv) * dt;
+    u.qr = u.qr + (t_qc2qr_accret + t_qc2qr_autoconv - t_qr2qv_evap) * dt;
+    if (predictNc || prescribedCCN) u.nc = u.nc + (-t_nc_accret - t_nc2nr_autoconv + t_nc_selfcollect) * dt;
+    else u.nc = NCCNST * s[S_INV_RHO];
+    u.nr = u.nr + (t_ncautr - t_nr_selfcollect - t_nr_evap) * dt;
+    u.qv = u.qv + t_qr2qv_evap * dt;
+    u.th = u.th + inv_exner * (-t_qr2qv_evap * latvap * INV_CP) * dt;
 
     // outputs, P3I/p3_main_impl_part2.hpp:456-463
-    s.qv2qi_depos_tend = t_qv2qi_vapdep - t_qi2qv_sublim + t_qv2qi_nucleat;
-    s.precip_total_tend = t_qc2qr_accret + t_qc2qr_autoconv + t_qc2qr_ice_shed + t_qc2qi_collect;
-    s.nevapr = t_qi2qv_sublim + t_qr2qv_evap;
-    s.vap_ice_exchange = t_qv2qi_vapdep - t_qi2qv_sublim + t_qv2qi_nucleat;
-    s.vap_liq_exchange = -t_qr2qv_evap;
-    s.liq_ice_exchange = t_qc2qi_hetero + t_qr2qi_immers - t_qi2qr_melt + t_qc2qi_berg + t_qc2qi_collect + t_qr2qi_collect;
+    o.qv2qi_depos_tend = t_qv2qi_vapdep - t_qi2qv_sublim + t_qv2qi_nucleat;
+    o.precip_total_tend = t_qc2qr_accret + t_qc2qr_autoconv + t_qc2qr_ice_shed + t_qc2qi_collect;
+    o.nevapr = t_qi2qv_sublim + t_qr2qv_evap;
+    o.vap_ice_exchange = t_qv2qi_vapdep - t_qi2qv_sublim + t_qv2qi_nucleat;
+    o.vap_liq_exchange = -t_qr2qv_evap;
+    o.liq_ice_exchange = t_qc2qi_hetero + t_qr2qi_immers - t_qi2qr_melt + t_qc2qi_berg + t_qc2qi_collect + t_qr2qi_collect;
 
     // clipping, P3I/p3_main_impl_part2.hpp:465-508
     bool present = false;
-    if (s.qc < QSMALL) {
-      s.qv = s.qv + s.qc;
-      s.th = s.th - inv_exner * s.qc * latvap * inv_cp;
-      s.qc = 0; s.nc = 0;
+    if (u.qc < QSMALL) {
+      u.qv = u.qv + u.qc;
+      u.th = u.th - inv_exner * u.qc * latvap * inv_cp;
+      u.qc = 0; u.nc = 0;
     } else present = true;
-    if (s.qr < QSMALL) {
-      s.qv = s.qv + s.qr;
-      s.th = s.th - inv_exner * s.qr * latvap * inv_cp;
-      s.qr = 0; s.nr = 0;
+    if (u.qr < QSMALL) {
+      u.qv = u.qv + u.qr;
+      u.th = u.th - inv_exner * u.qr * latvap * inv_cp;
+      u.qr = 0; u.nr = 0;
     } else present = true;
-    if (s.qi < QSMALL) {
-      s.qv = s.qv + s.qi;
-      s.th = s.th - inv_exner * s.qi * (latvap + latice) * inv_cp;
-      s.qi = 0; s.ni = 0; s.qm = 0; s.bm = 0;
+    if (u.qi < QSMALL) {
+      u.qv = u.qv + u.qi;
+      u.th = u.th - inv_exner * u.qi * (latvap + latice) * inv_cp;
+      u.qi = 0; u.ni = 0; u.qm = 0; u.bm = 0;
     } else present = true;
 
     // P3I/p3_main_impl_part2.hpp:514-517
-    double ni_incld_d = p3m_div(s.ni, cld_frac_i);
-    impose_max_total_ni<double>(ni_incld_d, rt.max_total_ni, inv_rho);
-    s.ni = ni_incld_d * cld_frac_i;
+    double ni_incld_d = p3m_div(u.ni, cld_frac_i);
+    impose_max_total_ni<double>(ni_incld_d, rt.max_total_ni, s[S_INV_RHO]);
+    u.ni = ni_incld_d * cld_frac_i;
+    const double out[10] = {u.qc, u.nc, u.qr, u.nr, u.qi, u.ni, u.qm, u.bm, u.qv, u.th};
+#pragma unroll
+    for (int q = 0; q < 10; ++q) {
+      // (a field rewritten above has its bit already)
+      if (__double_as_longlong(out[q]) != __double_as_longlong(s[S_QC + q])) chg |= 1u << q;
+      st[q] = out[q];
+    }
     return present;
   }
 }

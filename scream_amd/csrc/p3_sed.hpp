@@ -628,8 +628,11 @@ __device__ __forceinline__ void sed_wave(const KParams& p, int col0, const R* __
   // choice of levels per lane); columns past ncol or without a full step only
   // skip the arithmetic.
   const bool live = i < p.ncol;
-  const int status = live ? p.colstat[i] : 0;
-  const bool run = live && status == kStatusFull;
+  // (a column that the reference skips has none of the species: without the
+  // status words each species' own top level decides)
+  const bool track = p.track();
+  const int status = live && track ? p.colstat[i] : 0;
+  const bool run = live && (!track || status == kStatusFull);
   const double inv_dt = 1 / p.dt;
   if constexpr (G == SED_LIQ) {
     double prt_c, prt_r;
@@ -695,7 +698,17 @@ __device__ __forceinline__ void part3_tile(const KParams& p, int tile) {
   int i, k;
   if (!pw_point<PW_RUNS>(p, tile, i, k)) return;
   unsigned err = 0;
-  part3_level<R>(p, k, i, p.colstat[i] == kStatusFull, err);
+  // without the status words every column counts as stepped: a level of a
+  // skipped one is empty, and part 3 changes nothing there
+  const int status = p.track() ? p.colstat[i] : kStatusFull;
+  if (!p.exch_zero && (status & kStatusPart1) && p.sc(SC_PEND, i, k) != 0) {
+    // a warm clear level of a column that part 2 ran in (front_level)
+    const size_t x = p.at(i, k);
+    p.vap_ice_exchange[x] = 0;
+    p.vap_liq_exchange[x] = 0;
+    p.liq_ice_exchange[x] = 0;
+  }
+  part3_level<R>(p, k, i, status == kStatusFull, err);
   if (k == 0 && p.amble.on && p.amble.water_flux) {
     // the post-amble's boundary fluxes (eamxx_p3_process_interface.hpp:245-258),
     // from the surface precipitation both sedimentation kernels wrote

@@ -61,18 +61,8 @@ int status_of_err(unsigned err) {
 }
 
 // Default launch shape per (precision, nlev), from sweeps on MI355X at 21600x72
-// and 16384x128 in both precisions.  Part 1: one thread per (level, column).
-// Part 2: compiled for two wavefronts per SIMD (in FP64 that spills a little,
-// which costs less than the latency a single wavefront leaves exposed).
+// and 16384x128 in both precisions.
 void default_shape(int precision, int nk, p3d::Shape* sh) {
-  sh->cb = 32;
-  sh->nt = 256;
-  sh->wpe = 2;
-  // Part 1 one thread per (level, column): part 1 + 2 take 267 instead of 317 us
-  // (FP64) and 180 instead of 221 us (mixed) at 21600 x 72.  Every form uses it
-  // unless an explicit cb x nt shape asks for the block kernel (the batch tuner
-  // tries those too).  Part 3 runs in a kernel of its own in every form.
-  sh->p1lvl = 1;
   // Sedimentation lanes per column, per species group (kernel trace, us):
   //                     liquid 16 / 32 / 64     ice 16 / 32 / 64
   //   FP64  21600 x 72     115 / 184 / 247     766 / 767 / 891
@@ -500,15 +490,13 @@ namespace p3x_detail {
 
 int resolve_shape(int precision, int nk_max, int cb, int nt, int lpc, int wpe, p3d::Shape* sh) {
   default_shape(precision, nk_max, sh);
-  if (cb != 0 || nt != 0) {  // an explicit block shape runs at one wavefront per SIMD unless told otherwise
-    sh->cb = cb;
-    sh->nt = nt;
-    sh->wpe = 1;
-    sh->p1lvl = 0;
-  }
+  // the block shapes and register budgets that parts 1 and 2 once had stay
+  // accepted; they have no effect on the one kernel that now runs both
+  static const int shapes[][2] = {{0, 0}, {16, 128}, {16, 256}, {32, 256}, {64, 256}, {32, 512}, {64, 512}};
+  bool known = false;
+  for (const auto& b : shapes) known |= cb == b[0] && nt == b[1];
+  if (!known || wpe < 0 || wpe > 2) return P3X_ERR_ARG;
   if (lpc != 0) sh->lpc = sh->lpc_ice = lpc;
-  if (wpe != 0) sh->wpe = wpe;
-  if (sh->wpe != 1 && sh->wpe != 2) return P3X_ERR_ARG;
   for (int l : {sh->lpc, sh->lpc_ice}) {
     if (l != 16 && l != 32 && l != 64) return P3X_ERR_ARG;
     if (nk_max > l * p3d::kMaxLevelsPerLane) return P3X_ERR_ARG;
@@ -519,10 +507,10 @@ int resolve_shape(int precision, int nk_max, int cb, int nt, int lpc, int wpe, p
 int layout_batch(const p3d::KParams* sets, int n, const p3d::Shape& sh, Layout* out) {
   Layout& L = *out;
   L.first.assign(n + 1, 0);
-  L.first2.assign(n + 1, 0);
+  L.track = 0;
   for (int i = 0; i < n; ++i) {
-    L.first[i + 1] = L.first[i] + (sets[i].ncol + sh.cb - 1) / sh.cb;
-    L.first2[i + 1] = L.first2[i] + p3d::pw_tiles(sets[i]);
+    L.first[i + 1] = L.first[i] + p3d::pw_tiles(sets[i]);
+    L.track |= sets[i].track() ? 1 : 0;
   }
   const int cols_sed = p3d::kSedWaves * (64 / sh.lpc);
   std::vector<int> cls_of(n);
@@ -554,9 +542,9 @@ int grid_for(int ncu, int blocks_per_cu, int total, int resident) {
   return (int)std::max(1L, std::min<long>(g, std::max(total, 1)));
 }
 
-hipError_t occupancy(int precision, const p3d::Shape& sh, int L, int* r1, int* r2, int* rsed) {
-  return precision == P3X_FP64 ? p3d::occupancy_p3_fp64(sh, L, r1, r2, rsed)
-                               : p3d::occupancy_p3_mixed(sh, L, r1, r2, rsed);
+hipError_t occupancy(int precision, const p3d::Shape& sh, int L, int* r1, int* rsed) {
+  return precision == P3X_FP64 ? p3d::occupancy_p3_fp64(sh, L, r1, rsed)
+                               : p3d::occupancy_p3_mixed(sh, L, r1, rsed);
 }
 
 hipError_t launch_plan(int precision, const p3d::BatchPlan& plan, hipStream_t s) {
@@ -570,8 +558,8 @@ struct p3x_batch {
   p3x_batch_options opt{};
   std::vector<p3d::KParams> sets;  // in the caller's order
   double* d_scratch = nullptr;
-  p3d::KParams* d_sets = nullptr;  // caller's order (part 1 and part 2 launches)
-  int* d_first = nullptr;          // part 1 blocks, then part 2 tiles (2 x (nsets + 1))
+  p3d::KParams* d_sets = nullptr;  // caller's order (pointwise launches)
+  int* d_first = nullptr;          // pointwise tiles (nsets + 1)
   p3d::KParams* d_sets_sed = nullptr;  // grouped by sedimentation class
   int* d_first_sed = nullptr;
   p3d::BatchPlan plan{};
@@ -616,10 +604,9 @@ int build_plan(p3x_batch* b) {
   std::vector<p3d::KParams> sed_sets;
   for (int i : lay.sed_order) sed_sets.push_back(b->sets[i]);
 
-  std::vector<int> firsts(lay.first);
-  firsts.insert(firsts.end(), lay.first2.begin(), lay.first2.end());
-  e = hipMalloc((void**)&b->d_first, firsts.size() * sizeof(int));
-  if (e == hipSuccess) e = hipMemcpy(b->d_first, firsts.data(), firsts.size() * sizeof(int), hipMemcpyHostToDevice);
+  e = hipMalloc((void**)&b->d_first, lay.first.size() * sizeof(int));
+  if (e == hipSuccess)
+    e = hipMemcpy(b->d_first, lay.first.data(), lay.first.size() * sizeof(int), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_sets_sed, sed_sets.size() * sizeof(p3d::KParams));
   if (e == hipSuccess)
     e = hipMemcpy(b->d_sets_sed, sed_sets.data(), sed_sets.size() * sizeof(p3d::KParams), hipMemcpyHostToDevice);
@@ -632,8 +619,8 @@ int build_plan(p3x_batch* b) {
   b->plan.shape = sh;
   b->plan.sets = b->d_sets;
   b->plan.first = b->d_first;
-  b->plan.first2 = b->d_first + (n + 1);
   b->plan.nsets = n;
+  b->plan.track = lay.track;
   b->plan.nclass = (int)lay.cls.size();
   for (int ci = 0; ci < b->plan.nclass; ++ci) {
     const Layout::Cls& lc = lay.cls[ci];
@@ -642,15 +629,14 @@ int build_plan(p3x_batch* b) {
     sc.sets = b->d_sets_sed + lc.set_off;
     sc.first = b->d_first_sed + lc.first_off;
     sc.nsets = lc.nsets;
-    int r1 = 1, r2 = 1, rsed = 1;
-    e = occupancy(b->opt.precision, sh, sc.L, &r1, &r2, &rsed);
+    int r1 = 1, rsed = 1;
+    e = occupancy(b->opt.precision, sh, sc.L, &r1, &rsed);
     if (e == hipErrorInvalidValue) return P3X_ERR_ARG;
     if (e != hipSuccess) return P3X_ERR_DEVICE;
     sc.grid = grid_for(c->ncu, b->opt.blocks_per_cu, lc.total, rsed);
     if (ci == 0) {
       b->plan.grid = grid_for(c->ncu, b->opt.blocks_per_cu, lay.first[n], r1);
-      b->plan.grid2 = grid_for(c->ncu, b->opt.blocks_per_cu, lay.first2[n], r2);
-      b->plan.total2 = lay.first2[n];
+      b->plan.total = lay.first[n];
     }
   }
 
@@ -805,8 +791,6 @@ extern "C" int p3x_batch_tune(p3x_batch* b, void* stream, int reps, p3x_batch_op
   p3x_batch_options best = b->opt;
   double best_t = 0;
   if (e == hipSuccess) trial(&best_t);
-  static const int shapes[][3] = {{16, 128, 1}, {16, 256, 1}, {32, 256, 1}, {64, 256, 1}, {32, 512, 1},
-                                  {64, 512, 1},  {16, 256, 2}, {32, 256, 2}, {64, 256, 2}};
   static const int lanes[] = {16, 32, 64};
   static const int bpcs[] = {0, -1, 1, 2, 4};
   auto consider = [&](const p3x_batch_options& cand) {
@@ -823,13 +807,6 @@ extern "C" int p3x_batch_tune(p3x_batch* b, void* stream, int reps, p3x_batch_op
       best = cand;
     }
   };
-  for (const auto& sh : shapes) {
-    p3x_batch_options cand = best;
-    cand.columns_per_block = sh[0];
-    cand.threads_per_block = sh[1];
-    cand.part12_waves_per_simd = sh[2];
-    consider(cand);
-  }
   for (int l : lanes) {
     p3x_batch_options cand = best;
     cand.sed_lanes_per_column = l;

@@ -66,7 +66,7 @@ struct p3x_server {
   p3x_runtime rt{};
   p3x_server_options opt{};
   p3d::Shape shape{};
-  int occ1 = 1, occ2 = 1;  // resident blocks per CU of the part 1 and part 2 kernels
+  int occ1 = 1;  // resident blocks per CU of the pointwise kernels
   int occ_sed[p3d::kMaxLevelsPerLane + 1] = {};
   struct Member {
     p3d::KParams k;
@@ -101,9 +101,9 @@ namespace {
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Bytes of descriptors a batch of n sets needs in a slot: [sets][sed sets],
-// [first], [first2], [sed_first], [error words], each 256-aligned.
+// [first], [sed_first], [error words], each 256-aligned.
 size_t desc_bytes_for(int n) {
-  return align256(2 * (size_t)n * sizeof(p3d::KParams)) + 2 * align256((size_t)(n + 1) * sizeof(int)) +
+  return align256(2 * (size_t)n * sizeof(p3d::KParams)) + align256((size_t)(n + 1) * sizeof(int)) +
          align256((size_t)(n + p3d::kMaxLevelsPerLane) * sizeof(int)) + align256((size_t)n * sizeof(unsigned));
 }
 
@@ -123,11 +123,10 @@ size_t member_bytes(const p3d::KParams& k) {
 int launch_slot(p3x_server* srv, Slot& sl) {
   const int n = (int)sl.reqs.size();
   std::vector<p3d::KParams> sets(n);
-  // staging layout: [sets][sed sets][first][first2][sed_first][error words]
+  // staging layout: [sets][sed sets][first][sed_first][error words]
   const size_t o_sets = 0, o_sed = (size_t)n * sizeof(p3d::KParams);
   const size_t o_first = align256(2 * (size_t)n * sizeof(p3d::KParams));
-  const size_t o_first2 = o_first + align256((size_t)(n + 1) * sizeof(int));
-  const size_t o_sfirst = o_first2 + align256((size_t)(n + 1) * sizeof(int));
+  const size_t o_sfirst = o_first + align256((size_t)(n + 1) * sizeof(int));
   const size_t o_err = o_sfirst + align256((size_t)(n + p3d::kMaxLevelsPerLane) * sizeof(int));
   unsigned* d_err = (unsigned*)(sl.d_desc + o_err);
   size_t off = 0;
@@ -149,7 +148,6 @@ int launch_slot(p3x_server* srv, Slot& sl) {
   for (int i = 0; i < n; ++i)
     std::memcpy(h + o_sed + i * sizeof(p3d::KParams), &sets[lay.sed_order[i]], sizeof(p3d::KParams));
   std::memcpy(h + o_first, lay.first.data(), lay.first.size() * sizeof(int));
-  std::memcpy(h + o_first2, lay.first2.data(), lay.first2.size() * sizeof(int));
   std::memcpy(h + o_sfirst, lay.sed_first.data(), lay.sed_first.size() * sizeof(int));
   std::memset(h + o_err, 0, (size_t)n * sizeof(unsigned));  // the error words start at zero
   const size_t bytes = o_err + (size_t)n * sizeof(unsigned);
@@ -158,13 +156,12 @@ int launch_slot(p3x_server* srv, Slot& sl) {
   plan.shape = srv->shape;
   plan.sets = (const p3d::KParams*)(sl.d_desc + o_sets);
   plan.first = (const int*)(sl.d_desc + o_first);
-  plan.first2 = (const int*)(sl.d_desc + o_first2);
   plan.nsets = n;
   // one block per virtual block: the pointwise kernels then run without their
   // persistent loop, which costs them registers
   plan.grid = grid_for(srv->ctx->ncu, -1, lay.first[n], srv->occ1);
-  plan.grid2 = grid_for(srv->ctx->ncu, -1, lay.first2[n], srv->occ2);
-  plan.total2 = lay.first2[n];
+  plan.total = lay.first[n];
+  plan.track = lay.track;
   plan.nclass = (int)lay.cls.size();
   for (int c = 0; c < plan.nclass; ++c) {
     const Layout::Cls& lc = lay.cls[c];
@@ -349,10 +346,9 @@ extern "C" int p3x_server_create(p3x_context* c, const p3x_runtime* rt, const p3
   hipError_t e = hipSuccess;
   for (int L = 1; L <= p3d::kMaxLevelsPerLane && e == hipSuccess; ++L) {
     if (L == 7) continue;
-    int r1 = 1, r2 = 1, rsed = 1;
-    e = occupancy(o.precision, s->shape, L, &r1, &r2, &rsed);
+    int r1 = 1, rsed = 1;
+    e = occupancy(o.precision, s->shape, L, &r1, &rsed);
     s->occ1 = r1;
-    s->occ2 = r2;
     s->occ_sed[L] = rsed;
   }
   s->occ_sed[7] = s->occ_sed[8];

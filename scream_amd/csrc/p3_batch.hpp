@@ -78,6 +78,40 @@ __global__ __launch_bounds__(kTileThreads) void p3_part3_lvl_batch(const KParams
   });
 }
 
+// The virtual block that block b of nb runs, one block per virtual block: block
+// b is on XCD b % 8, so within each run of 8 * kXcdRun blocks an XCD takes
+// kXcdRun consecutive virtual blocks.  Neighbouring blocks hold parts of the same
+// 128-byte lines (4 to 16 columns each), while the runs keep the sets in order:
+// the longest steps start first (layout_batch).
+constexpr int kXcdRun = 16;
+__device__ __forceinline__ int run_block(int b, int nb) {
+  constexpr int chunk = kXcds * kXcdRun;
+  const int c0 = b / chunk * chunk;
+  if (c0 + chunk > nb) return b;
+  const int r = b - c0;
+  return c0 + r % kXcds * kXcdRun + r / kXcds;
+}
+
+// Both species groups of one class of sets in one launch, the ice blocks first
+// (p3_sed_fused_kernel); one block per virtual block, nb of them per group.
+template <class R, int LPC, int L, int WPB>
+__global__ __launch_bounds__(64 * WPB, (sed_waves_per_simd<R, SED_ICE, L>())) void p3_sed_fused_batch(
+    const KParams* __restrict__ sets, const int* __restrict__ first, int nsets, int nb) {
+  static_assert(WPB == 4 || !ice_rec_dif<R, L>(), "the LDS budget assumes blocks of 4 wavefronts");
+  __shared__ __align__(16) R s_tab[ice_lds_len<R, L>()];
+  const auto sets4 = (const __attribute__((address_space(4))) KParams*)sets;
+  const int b = blockIdx.x;  // uniform over the block: the whole block takes one branch
+  const int vb = run_block(b < nb ? b : b - nb, nb);
+  const int s = find_set(first, nsets, vb);
+  const KParams& p = *(const KParams*)(sets4 + s);
+  if (b < nb) {
+    stage_ice_table<R, ice_lds_len<R, L>()>(ice_lds_source<R, L>(p), s_tab);
+    sed_block<R, LPC, L, WPB, SED_ICE>(p, vb - first[s], s_tab);
+  } else {
+    sed_block<R, LPC, L, WPB, SED_LIQ>(p, vb - first[s], nullptr);
+  }
+}
+
 // Sedimentation of species group G (SED_LIQ or SED_ICE).  The sets of a batch
 // share their context's tables, so the ice group stages the first set's ice
 // records in LDS once per block.

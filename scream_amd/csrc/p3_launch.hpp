@@ -10,7 +10,7 @@ namespace p3d {
 // Shape of one step's launches: the lanes per column of the sedimentation
 // kernels (16, 32 or 64), of the liquid group (cloud, rain) and of the ice
 // group; each lane holds L = ceil(nlev / lanes) levels (at most 8), 4 wavefronts
-// per block (the batched form runs both groups on lpc).  Parts 1 to 3 run one
+// per block (the batched form runs both groups of a set on lpc).  Parts 1 to 3 run one
 // thread per (level, column) on the pointwise tiles.
 struct Shape {
   int lpc, lpc_ice;
@@ -49,14 +49,18 @@ hipError_t launch_p3_mixed(const KParams& p, const Shape& sh, hipStream_t s, hip
                            const SedFork* fork = nullptr);
 
 // ---- batched form (p3_batch.hpp)
-// Sets whose sedimentation kernel uses the same levels-per-lane count.
+// Sets whose sedimentation runs on the same lanes per column and levels per lane.
 struct SedClass {
-  int L;
+  int lpc, L;
   const KParams* sets;  // device array
   const int* first;     // device array, nsets + 1 entries
   int nsets;
+  int total;            // virtual blocks per species group (first[nsets])
   int grid;             // blocks (one per virtual block, or a persistent grid)
 };
+constexpr int kMaxSedClasses = 3 * kMaxLevelsPerLane;
+// Streams beside the batch's own for its second and later classes.
+constexpr int kSideStreams = 3;
 // The sedimentation launches on one lanes-per-column count.
 struct SedLaunch {
   hipError_t (*single)(const KParams& p, int group, int L, hipStream_t s);  // one species group
@@ -65,7 +69,6 @@ struct SedLaunch {
   hipError_t (*occupancy)(int L, int* blocks);  // resident blocks per CU of the batched kernels
 };
 struct BatchPlan {
-  Shape shape;
   const KParams* sets;  // device array, all sets (pointwise launches)
   const int* first;     // device array, nsets + 1 entries: pointwise tiles (parts 1 to 3)
   int nsets;
@@ -73,12 +76,16 @@ struct BatchPlan {
   int grid;             // blocks of the pointwise launches
   int total;            // pointwise virtual blocks (first[nsets]); grid >= total: one block each, no loop
   int nclass;
-  SedClass cls[kMaxLevelsPerLane];
+  SedClass cls[kMaxSedClasses];
+  // with side streams (NULL: none), the classes run side by side, forked from
+  // the batch's stream after parts 1 and 2 and joined before part 3
+  hipStream_t side[kSideStreams];
+  hipEvent_t fork, join[kSideStreams];
 };
 hipError_t launch_p3_batch_fp64(const BatchPlan& b, hipStream_t s);
 hipError_t launch_p3_batch_mixed(const BatchPlan& b, hipStream_t s);
 // Resident blocks per CU of the batched kernels for this shape (occupancy API).
-hipError_t occupancy_p3_fp64(const Shape& sh, int L, int* blocks, int* blocks_sed);
-hipError_t occupancy_p3_mixed(const Shape& sh, int L, int* blocks, int* blocks_sed);
+hipError_t occupancy_p3_fp64(int lpc, int L, int* blocks, int* blocks_sed);
+hipError_t occupancy_p3_mixed(int lpc, int L, int* blocks, int* blocks_sed);
 
 }  // namespace p3d

@@ -60,23 +60,35 @@ int status_of_err(unsigned err) {
   return err ? P3X_ERR_DEVICE : P3X_OK;
 }
 
-// Default launch shape per (precision, nlev), from sweeps on MI355X at 21600x72
-// and 16384x128 in both precisions.
-void default_shape(int precision, int nk, p3d::Shape* sh) {
-  // Sedimentation lanes per column, per species group (kernel trace, us):
-  //                     liquid 16 / 32 / 64     ice 16 / 32 / 64
-  //   FP64  21600 x 72     115 / 184 / 247     766 / 767 / 891
-  //   FP64  16384 x 128    111 /  77 / 105     284 / 184 / 171
-  //   mixed 21600 x 72      63 /  84 / 121     412 / 363 / 427
-  //   mixed 16384 x 128     51 /  49 /  60     131 / 122 / 133
-  // (at most 5 levels per lane keep two wavefronts per SIMD; the batched form
-  // runs both groups on lpc, which its tuner also searches).  Since the group
-  // reductions run on DPP inside a 16-lane row, 16 lanes per column pay off for
-  // the FP64 ice group at up to 80 levels: whole step at 21600 x 72, four runs
-  // of each build alternating, 1143 us against 1159 at 32 lanes (mixed: no
-  // difference; at 128 levels 32 or 64 lanes for both groups were slower).
+// Default sedimentation lanes per column of a step over ncol columns of nk levels.
+//
+// Few columns (their wavefronts at 64 lanes, one per column, all fit the chip at
+// two per SIMD: 2048): a wavefront's time is its chain of level bodies per
+// substep, so the fewest levels per lane are the fastest.  Sedimentation and part
+// 3, us, at 16 / 32 / 64 lanes:
+//   FP64   72 levels, dt 1800: 256 columns 146 / 118 / 71, 2048 161 / 129 / 115,
+//                              3072 171 / 176 / 164, 4096 171 / 177 / 198
+//   FP64  128 levels, dt 100:  256 columns  62 /  38 / 27, 2048  81 /  56 /  57
+//   mixed  72 levels, dt 1800: 256 columns  99 /  67 / 52, 2048 108 /  76 /  75
+// More columns than that: the lanes that waste the fewest level slots and leave
+// two wavefronts per SIMD their registers (at most 5 levels per lane), per
+// species group (kernel trace, us):
+//                     liquid 16 / 32 / 64     ice 16 / 32 / 64
+//   FP64  21600 x 72     115 / 184 / 247     766 / 767 / 891
+//   FP64  16384 x 128    111 /  77 / 105     284 / 184 / 171
+//   mixed 21600 x 72      63 /  84 / 121     412 / 363 / 427
+//   mixed 16384 x 128     51 /  49 /  60     131 / 122 / 133
+// (FP64 ice at up to 80 levels: 16 lanes, 1143 against 1159 us a step at 32; the
+// mixed ice group up to 48 levels: 16 lanes, 20000 x 48 118 us against 140 with
+// ice on 32.)
+constexpr int kFewColumns = 2048;
+void default_shape(int precision, int nk, long long ncol, p3d::Shape* sh) {
+  if (ncol <= kFewColumns) {
+    sh->lpc = sh->lpc_ice = 64;
+    return;
+  }
   sh->lpc = nk <= 80 ? 16 : (nk <= 32 * 5 ? 32 : 64);
-  if (precision == P3X_MIXED) sh->lpc_ice = nk <= 32 * 5 ? 32 : 64;
+  if (precision == P3X_MIXED) sh->lpc_ice = nk <= 48 ? 16 : (nk <= 32 * 5 ? 32 : 64);
   else sh->lpc_ice = nk <= 80 ? 16 : (nk <= 96 ? 32 : 64);
 }
 
@@ -418,9 +430,11 @@ int p3x_detail::main_impl(p3x_context* c, const p3x_runtime* runtime, const p3x_
   if (nk > 64 * p3d::kMaxLevelsPerLane) return P3X_ERR_ARG;
   p3d::Shape sh;
   {
-    const int st = resolve_shape(o.precision, nk, o.columns_per_block, o.threads_per_block,
-                                 o.sed_lanes_per_column, o.part12_waves_per_simd, &sh);
+    const int st = check_options(nk, o.columns_per_block, o.threads_per_block, o.sed_lanes_per_column,
+                                 o.part12_waves_per_simd);
     if (st != P3X_OK) return st;
+    default_shape(o.precision, nk, nj, &sh);
+    if (o.sed_lanes_per_column != 0) sh.lpc = sh.lpc_ice = o.sed_lanes_per_column;
   }
   hipStream_t s = (hipStream_t)o.stream;
   if (nj == 0) return P3X_OK;
@@ -488,50 +502,67 @@ extern "C" int p3x_last_kernel_times(p3x_context* c, double* part12_us, double* 
 
 namespace p3x_detail {
 
-int resolve_shape(int precision, int nk_max, int cb, int nt, int lpc, int wpe, p3d::Shape* sh) {
-  default_shape(precision, nk_max, sh);
+int check_options(int nk_max, int cb, int nt, int lpc, int wpe) {
   // the block shapes and register budgets that parts 1 and 2 once had stay
   // accepted; they have no effect on the one kernel that now runs both
   static const int shapes[][2] = {{0, 0}, {16, 128}, {16, 256}, {32, 256}, {64, 256}, {32, 512}, {64, 512}};
   bool known = false;
   for (const auto& b : shapes) known |= cb == b[0] && nt == b[1];
   if (!known || wpe < 0 || wpe > 2) return P3X_ERR_ARG;
-  if (lpc != 0) sh->lpc = sh->lpc_ice = lpc;
-  for (int l : {sh->lpc, sh->lpc_ice}) {
-    if (l != 16 && l != 32 && l != 64) return P3X_ERR_ARG;
-    if (nk_max > l * p3d::kMaxLevelsPerLane) return P3X_ERR_ARG;
-  }
-  return P3X_OK;
+  if (lpc != 0 && lpc != 16 && lpc != 32 && lpc != 64) return P3X_ERR_ARG;
+  return nk_max > (lpc != 0 ? lpc : 64) * p3d::kMaxLevelsPerLane ? P3X_ERR_ARG : P3X_OK;
 }
 
-int layout_batch(const p3d::KParams* sets, int n, const p3d::Shape& sh, Layout* out) {
+// Lanes per column of one set of a batch of ncol columns altogether: both groups
+// on the lanes of the group that takes longer, the ice group.
+int batch_lanes(int precision, int nk, long long ncol) {
+  p3d::Shape sh;
+  default_shape(precision, nk, ncol, &sh);
+  return sh.lpc_ice;
+}
+
+int layout_batch(const p3d::KParams* sets, int n, int precision, int lpc, Layout* out) {
   Layout& L = *out;
   L.first.assign(n + 1, 0);
   L.track = 0;
+  long long ncol = 0;
   for (int i = 0; i < n; ++i) {
     L.first[i + 1] = L.first[i] + p3d::pw_tiles(sets[i]);
     L.track |= sets[i].track() ? 1 : 0;
+    ncol += sets[i].ncol;
   }
-  const int cols_sed = p3d::kSedWaves * (64 / sh.lpc);
-  std::vector<int> cls_of(n);
+  // class of a set: its lanes per column and levels per lane
+  std::vector<std::pair<int, int>> cls_of(n);
   for (int i = 0; i < n; ++i) {
-    cls_of[i] = p3d::sed_levels_per_lane(sets[i].nlev, sh.lpc);
-    if (cls_of[i] == 0) return P3X_ERR_ARG;
+    const int l = lpc != 0 ? lpc : batch_lanes(precision, sets[i].nlev, ncol);
+    cls_of[i] = {l, p3d::sed_levels_per_lane(sets[i].nlev, l)};
+    if (cls_of[i].second == 0) return P3X_ERR_ARG;
   }
+  // the longest steps first: their blocks start first, and the class that holds
+  // the longest one too, so that no long block starts when the others have ended
+  std::vector<int> order(n);
+  for (int i = 0; i < n; ++i) order[i] = i;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+    return sets[a].dt * sets[a].nlev > sets[b].dt * sets[b].nlev;
+  });
   L.sed_order.clear();
   L.sed_first.clear();
   L.cls.clear();
-  for (int l = 1; l <= p3d::kMaxLevelsPerLane; ++l) {
-    Layout::Cls c{l, (int)L.sed_order.size(), (int)L.sed_first.size(), 0, 0};
-    for (int i = 0; i < n; ++i) {
-      if (cls_of[i] != l) continue;
-      if (c.nsets == 0) L.sed_first.push_back(0);
+  std::vector<char> placed(n, 0);
+  for (int lead : order) {
+    if (placed[lead]) continue;
+    Layout::Cls c{cls_of[lead].first, cls_of[lead].second, (int)L.sed_order.size(), (int)L.sed_first.size(), 0, 0};
+    const int cols = p3d::kSedWaves * (64 / c.lpc);  // columns per block
+    L.sed_first.push_back(0);
+    for (int i : order) {
+      if (cls_of[i] != cls_of[lead]) continue;
+      placed[i] = 1;
       L.sed_order.push_back(i);
-      c.total += (sets[i].ncol + cols_sed - 1) / cols_sed;
+      c.total += (sets[i].ncol + cols - 1) / cols;
       L.sed_first.push_back(c.total);
       c.nsets++;
     }
-    if (c.nsets > 0) L.cls.push_back(c);
+    L.cls.push_back(c);
   }
   return P3X_OK;
 }
@@ -542,9 +573,9 @@ int grid_for(int ncu, int blocks_per_cu, int total, int resident) {
   return (int)std::max(1L, std::min<long>(g, std::max(total, 1)));
 }
 
-hipError_t occupancy(int precision, const p3d::Shape& sh, int L, int* r1, int* rsed) {
-  return precision == P3X_FP64 ? p3d::occupancy_p3_fp64(sh, L, r1, rsed)
-                               : p3d::occupancy_p3_mixed(sh, L, r1, rsed);
+hipError_t occupancy(int precision, int lpc, int L, int* r1, int* rsed) {
+  return precision == P3X_FP64 ? p3d::occupancy_p3_fp64(lpc, L, r1, rsed)
+                               : p3d::occupancy_p3_mixed(lpc, L, r1, rsed);
 }
 
 hipError_t launch_plan(int precision, const p3d::BatchPlan& plan, hipStream_t s) {
@@ -563,6 +594,9 @@ struct p3x_batch {
   p3d::KParams* d_sets_sed = nullptr;  // grouped by sedimentation class
   int* d_first_sed = nullptr;
   p3d::BatchPlan plan{};
+  // the second and later sedimentation classes' streams (created when needed)
+  hipStream_t side[p3d::kSideStreams] = {};
+  hipEvent_t fork = nullptr, join[p3d::kSideStreams] = {};
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
 };
@@ -584,6 +618,20 @@ void free_plan(p3x_batch* b) {
 
 hipError_t launch_batch(const p3x_batch* b, hipStream_t s) { return launch_plan(b->opt.precision, b->plan, s); }
 
+// The batch's side streams and events, in its plan.
+int side_streams(p3x_batch* b) {
+  hipError_t e = hipSuccess;
+  if (!b->fork) e = hipEventCreateWithFlags(&b->fork, hipEventDisableTiming);
+  for (int i = 0; i < p3d::kSideStreams && e == hipSuccess; ++i) {
+    if (!b->side[i]) e = hipStreamCreateWithFlags(&b->side[i], hipStreamNonBlocking);
+    if (e == hipSuccess && !b->join[i]) e = hipEventCreateWithFlags(&b->join[i], hipEventDisableTiming);
+    b->plan.side[i] = b->side[i];
+    b->plan.join[i] = b->join[i];
+  }
+  b->plan.fork = b->fork;
+  return e == hipSuccess ? P3X_OK : dev_fail(e);
+}
+
 // Lay the sets out for b->opt: virtual-block offsets of both launches, the
 // sedimentation classes, grid sizes and (use_graph) the graph.
 int build_plan(p3x_batch* b) {
@@ -594,12 +642,11 @@ int build_plan(p3x_batch* b) {
   free_plan(b);
   int nk_max = 1;
   for (const auto& k : b->sets) nk_max = std::max(nk_max, k.nlev);
-  p3d::Shape sh;
-  int st = resolve_shape(b->opt.precision, nk_max, b->opt.columns_per_block, b->opt.threads_per_block,
-                         b->opt.sed_lanes_per_column, b->opt.part12_waves_per_simd, &sh);
+  int st = check_options(nk_max, b->opt.columns_per_block, b->opt.threads_per_block, b->opt.sed_lanes_per_column,
+                         b->opt.part12_waves_per_simd);
   if (st != P3X_OK) return st;
   Layout lay;
-  st = layout_batch(b->sets.data(), n, sh, &lay);
+  st = layout_batch(b->sets.data(), n, b->opt.precision, b->opt.sed_lanes_per_column, &lay);
   if (st != P3X_OK) return st;
   std::vector<p3d::KParams> sed_sets;
   for (int i : lay.sed_order) sed_sets.push_back(b->sets[i]);
@@ -616,7 +663,10 @@ int build_plan(p3x_batch* b) {
   if (e != hipSuccess) return dev_fail(e);
 
   b->plan = p3d::BatchPlan{};
-  b->plan.shape = sh;
+  if (lay.cls.size() > 1) {
+    st = side_streams(b);
+    if (st != P3X_OK) return st;
+  }
   b->plan.sets = b->d_sets;
   b->plan.first = b->d_first;
   b->plan.nsets = n;
@@ -625,12 +675,14 @@ int build_plan(p3x_batch* b) {
   for (int ci = 0; ci < b->plan.nclass; ++ci) {
     const Layout::Cls& lc = lay.cls[ci];
     p3d::SedClass& sc = b->plan.cls[ci];
+    sc.lpc = lc.lpc;
     sc.L = lc.L;
+    sc.total = lc.total;
     sc.sets = b->d_sets_sed + lc.set_off;
     sc.first = b->d_first_sed + lc.first_off;
     sc.nsets = lc.nsets;
     int r1 = 1, rsed = 1;
-    e = occupancy(b->opt.precision, sh, sc.L, &r1, &rsed);
+    e = occupancy(b->opt.precision, sc.lpc, sc.L, &r1, &rsed);
     if (e == hipErrorInvalidValue) return P3X_ERR_ARG;
     if (e != hipSuccess) return P3X_ERR_DEVICE;
     sc.grid = grid_for(c->ncu, b->opt.blocks_per_cu, lc.total, rsed);
@@ -836,6 +888,11 @@ extern "C" void p3x_batch_destroy(p3x_batch* b) {
   if (!b) return;
   (void)hipDeviceSynchronize();
   free_plan(b);
+  for (int i = 0; i < p3d::kSideStreams; ++i) {
+    if (b->side[i]) (void)hipStreamDestroy(b->side[i]);
+    if (b->join[i]) (void)hipEventDestroy(b->join[i]);
+  }
+  if (b->fork) (void)hipEventDestroy(b->fork);
   (void)hipFree(b->d_sets);
   (void)hipFree(b->d_scratch);
   delete b;

@@ -40,8 +40,8 @@ namespace p3x_detail {
 int dev_fail(hipError_t e);
 // The P3X status of a nonzero device error word.
 int status_of_err(unsigned err);
-// Default launch shape per (precision, nlev).
-void default_shape(int precision, int nk, p3d::Shape* sh);
+// Default launch shape of a step over ncol columns of nk levels.
+void default_shape(int precision, int nk, long long ncol, p3d::Shape* sh);
 // Grows the context's scratch to at least need bytes (P3X_OK or an error status).
 int grow_scratch(p3x_context* c, size_t need);
 // Layout strides of a column set in k (P3X_ERR_ARG for an invalid layout or stride).
@@ -92,26 +92,27 @@ int chain_check(const p3x_process* p, const p3x_atm_fields* f, const p3x_step_ch
 int chain_before(const p3x_process* p, const p3x_atm_fields* f, const p3x_step_chain* c, hipStream_t s);
 int chain_after(const p3x_process* p, const p3x_atm_fields* f, const p3x_step_chain* c, double dt, hipStream_t s);
 
-// Launch shape for a batch whose deepest set has nk_max levels: the defaults,
-// overridden by the nonzero options.  P3X_ERR_ARG if not compiled in.
-int resolve_shape(int precision, int nk_max, int cb, int nt, int lpc, int wpe, p3d::Shape* sh);
+// The launch options of a step or batch whose deepest set has nk_max levels:
+// P3X_ERR_ARG for a value that does not exist or lanes that nk_max does not fit.
+int check_options(int nk_max, int cb, int nt, int lpc, int wpe);
 
-// Host-side layout of a batch of column sets for one shape.
+// Host-side layout of a batch of column sets on lpc lanes per column (0: the
+// default of each set).
 struct Layout {
   std::vector<int> first;      // pointwise tile offsets, nsets + 1
   int track;                   // some set keeps its column status words
-  std::vector<int> sed_order;  // set indices grouped by sedimentation class (ascending L)
+  std::vector<int> sed_order;  // set indices grouped by sedimentation class, the longest steps first
   std::vector<int> sed_first;  // per class nsets_c + 1 offsets, classes concatenated
   struct Cls {
-    int L, set_off, first_off, nsets, total;
+    int lpc, L, set_off, first_off, nsets, total;
   };
   std::vector<Cls> cls;
 };
-int layout_batch(const p3d::KParams* sets, int n, const p3d::Shape& sh, Layout* out);
+int layout_batch(const p3d::KParams* sets, int n, int precision, int lpc, Layout* out);
 // Persistent grid for `total` virtual blocks: blocks_per_cu x CUs (0: the
 // resident count from the occupancy API; -1: one block per virtual block).
 int grid_for(int ncu, int blocks_per_cu, int total, int resident);
-hipError_t occupancy(int precision, const p3d::Shape& sh, int L, int* r1, int* rsed);
+hipError_t occupancy(int precision, int lpc, int L, int* r1, int* rsed);
 hipError_t launch_plan(int precision, const p3d::BatchPlan& plan, hipStream_t s);
 
 }  // namespace p3x_detail

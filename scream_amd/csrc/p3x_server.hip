@@ -65,9 +65,8 @@ struct p3x_server {
   p3x_context* ctx = nullptr;
   p3x_runtime rt{};
   p3x_server_options opt{};
-  p3d::Shape shape{};
-  int occ1 = 1;  // resident blocks per CU of the pointwise kernels
-  int occ_sed[p3d::kMaxLevelsPerLane + 1] = {};
+  int lpc = 0;   // sedimentation lanes per column (0: by the batch)
+  int lpc_max = 0;  // members' levels must fit these lanes
   struct Member {
     p3d::KParams k;
     size_t scratch;   // scratch bytes of one step
@@ -104,7 +103,7 @@ size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // [first], [sed_first], [error words], each 256-aligned.
 size_t desc_bytes_for(int n) {
   return align256(2 * (size_t)n * sizeof(p3d::KParams)) + align256((size_t)(n + 1) * sizeof(int)) +
-         align256((size_t)(n + p3d::kMaxLevelsPerLane) * sizeof(int)) + align256((size_t)n * sizeof(unsigned));
+         align256((size_t)(n + p3d::kMaxSedClasses) * sizeof(int)) + align256((size_t)n * sizeof(unsigned));
 }
 
 // Bytes the device arrays of a member span (every field of its column set).
@@ -127,7 +126,7 @@ int launch_slot(p3x_server* srv, Slot& sl) {
   const size_t o_sets = 0, o_sed = (size_t)n * sizeof(p3d::KParams);
   const size_t o_first = align256(2 * (size_t)n * sizeof(p3d::KParams));
   const size_t o_sfirst = o_first + align256((size_t)(n + 1) * sizeof(int));
-  const size_t o_err = o_sfirst + align256((size_t)(n + p3d::kMaxLevelsPerLane) * sizeof(int));
+  const size_t o_err = o_sfirst + align256((size_t)(n + p3d::kMaxSedClasses) * sizeof(int));
   unsigned* d_err = (unsigned*)(sl.d_desc + o_err);
   size_t off = 0;
   for (int i = 0; i < n; ++i) {
@@ -141,7 +140,7 @@ int launch_slot(p3x_server* srv, Slot& sl) {
     sets[i] = k;
   }
   Layout lay;
-  int st = layout_batch(sets.data(), n, srv->shape, &lay);
+  int st = layout_batch(sets.data(), n, srv->opt.precision, srv->lpc, &lay);
   if (st != P3X_OK) return st;
   char* h = sl.h_stage;
   std::memcpy(h + o_sets, sets.data(), n * sizeof(p3d::KParams));
@@ -153,24 +152,25 @@ int launch_slot(p3x_server* srv, Slot& sl) {
   const size_t bytes = o_err + (size_t)n * sizeof(unsigned);
 
   p3d::BatchPlan plan{};
-  plan.shape = srv->shape;
   plan.sets = (const p3d::KParams*)(sl.d_desc + o_sets);
   plan.first = (const int*)(sl.d_desc + o_first);
   plan.nsets = n;
   // one block per virtual block: the pointwise kernels then run without their
   // persistent loop, which costs them registers
-  plan.grid = grid_for(srv->ctx->ncu, -1, lay.first[n], srv->occ1);
+  plan.grid = lay.first[n];
   plan.total = lay.first[n];
   plan.track = lay.track;
   plan.nclass = (int)lay.cls.size();
   for (int c = 0; c < plan.nclass; ++c) {
     const Layout::Cls& lc = lay.cls[c];
     p3d::SedClass& sc = plan.cls[c];
+    sc.lpc = lc.lpc;
     sc.L = lc.L;
+    sc.total = lc.total;
     sc.sets = (const p3d::KParams*)(sl.d_desc + o_sed) + lc.set_off;
     sc.first = (const int*)(sl.d_desc + o_sfirst) + lc.first_off;
     sc.nsets = lc.nsets;
-    sc.grid = grid_for(srv->ctx->ncu, -1, lc.total, srv->occ_sed[lc.L]);
+    sc.grid = lc.total;
   }
   // the neighbour stages of process members before their steps ...
   for (int i = 0; i < n; ++i) {
@@ -335,23 +335,15 @@ extern "C" int p3x_server_create(p3x_context* c, const p3x_runtime* rt, const p3
   s->ctx = c;
   s->rt = *rt;
   s->opt = o;
-  // one shape for every batch; members are checked against its lanes per column
-  const int st = resolve_shape(o.precision, 1, o.columns_per_block, o.threads_per_block,
-                               o.sed_lanes_per_column != 0 ? o.sed_lanes_per_column : 32,
-                               o.part12_waves_per_simd, &s->shape);
+  // members are checked against 32 lanes per column unless the options name another count
+  s->lpc = o.sed_lanes_per_column;
+  s->lpc_max = s->lpc != 0 ? s->lpc : 32;
+  const int st = check_options(1, o.columns_per_block, o.threads_per_block, s->lpc, o.part12_waves_per_simd);
   if (st != P3X_OK) {
     delete s;
     return st;
   }
   hipError_t e = hipSuccess;
-  for (int L = 1; L <= p3d::kMaxLevelsPerLane && e == hipSuccess; ++L) {
-    if (L == 7) continue;
-    int r1 = 1, rsed = 1;
-    e = occupancy(o.precision, s->shape, L, &r1, &rsed);
-    s->occ1 = r1;
-    s->occ_sed[L] = rsed;
-  }
-  s->occ_sed[7] = s->occ_sed[8];
   s->slots.resize(o.slots);
   const size_t arena = (size_t)(o.scratch_budget_bytes / o.slots) & ~(size_t)255;
   s->scratch_total = (double)arena * o.slots;
@@ -378,7 +370,7 @@ extern "C" int p3x_server_create(p3x_context* c, const p3x_runtime* rt, const p3
 extern "C" int p3x_server_add_member(p3x_server* s, const p3x_column_set* set, int* member) {
   if (!s || !set || !member) return P3X_ERR_ARG;
   if (set->nj <= 0 || set->nk <= 0) return P3X_ERR_ARG;
-  if (p3d::sed_levels_per_lane(set->nk, s->shape.lpc) == 0) return P3X_ERR_ARG;
+  if (p3d::sed_levels_per_lane(set->nk, s->lpc_max) == 0) return P3X_ERR_ARG;
   if (!fields_present(&set->prognostic_state, &set->diagnostic_inputs, &set->diagnostic_outputs,
                       &set->history_only))
     return P3X_ERR_ARG;
@@ -413,7 +405,7 @@ extern "C" int p3x_server_add_process(p3x_server* s, p3x_process* proc, const p3
   int st = process_kparams(proc, fields, 1.0, &m.k);  // dt is replaced per request
   if (st != P3X_OK) return st;
   if (process_context(proc) != s->ctx) return P3X_ERR_ARG;  // the batch shares one context's tables
-  if (p3d::sed_levels_per_lane(m.k.nlev, s->shape.lpc) == 0) return P3X_ERR_ARG;
+  if (p3d::sed_levels_per_lane(m.k.nlev, s->lpc_max) == 0) return P3X_ERR_ARG;
   st = chain_check(proc, fields, chain);
   if (st != P3X_OK) return st;
   const size_t need = scratch_bytes_for(m.k.ncol, m.k.nlev);

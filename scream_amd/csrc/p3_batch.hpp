@@ -58,7 +58,7 @@ template <class R, bool PERSIST>
 __global__ __launch_bounds__(kTileThreads, kFrontWaves<R>) void p3_front_batch(const KParams* __restrict__ sets,
                                                                                const int* __restrict__ first,
                                                                                int nsets) {
-  __shared__ double s_lds[S_COUNT * kTileThreads];
+  __shared__ double s_lds[kSlots<R> * kTileThreads];
   const auto sets4 = (const __attribute__((address_space(4))) KParams*)sets;
   for_virtual_blocks<PERSIST>(first[nsets], [&](int vb) {
     const int s = find_set(first, nsets, vb);

@@ -53,6 +53,7 @@ struct KParams {
   int* dbg_check;       // per column: check_values flags (NULL = the check is off)
   Tables tab;
   Runtime rt;
+  RainGamma rg, rgf;    // of the FP64 and of the mixed form
   int ncol, nlev;
   // Layout.  Element (column i, level k) of a level field is at i*cs + k*ks, of
   // an interface field (nlev + 1 levels) at i*fcs + k*fks: level-major
@@ -94,6 +95,10 @@ constexpr int kMaxSubsteps = 100000;
 // Column status bits: part 1 found work, part 2 left hydrometeors.
 constexpr int kStatusPart1 = 1, kStatusPart2 = 2, kStatusFull = 3;
 
+template <class R> struct RainOf {
+  static __device__ __forceinline__ const RainGamma& get(const KParams& p) { return sizeof(R) == 8 ? p.rg : p.rgf; }
+};
+
 // p3_main_init, part 1 (P3I/p3_main_impl_part1.hpp:18-185) and part 2
 // (P3I/p3_main_impl_part2.hpp:113-524) of level k of column i.
 //
@@ -118,7 +123,10 @@ constexpr int kStatusPart1 = 1, kStatusPart2 = 2, kStatusFull = 3;
 // their own, part 1 (at the HBM rate) wrote seven scratch fields and part 2
 // (43 % busy, waiting on loads) read them and the state again.  Together, at
 // 21600 x 72 FP64 48 + 187 -> 225 us, at 16384 x 128 mixed 67 + 189 -> 195 us,
-// and a launch (two with the status words' clear) fewer.
+// and a launch (two with the status words' clear) fewer.  One logarithm of T for
+// the saturation values, T^1.5 and T^1.81, one viscosity for both parts, the rain
+// gammas from outside (RainGamma) and polynomial coefficients in scalar registers
+// then made it 203 and 187 us.
 template <class R>
 __device__ __forceinline__ void front_level(const KParams& p, int k, int i, const Pt s, int& stat, unsigned& err) {
   const double dt = p.dt;
@@ -194,16 +202,20 @@ __device__ __forceinline__ void front_level(const KParams& p, int k, int i, cons
   double T_atm = th * exner;
   const double rho = air_density(dpres, dz);
   const double inv_rho = p3m_div(1.0, rho);
+  const double T_first = T_atm;
+  double lh, ll;
+  log_temperature(T_atm, lh, ll);
   double qv_sat_l, qv_sat_i;
-  qv_sat_dry_both(T_atm, pres, qv_sat_l, qv_sat_i, err);
+  qv_sat_dry_both(T_atm, lh + ll, pres, qv_sat_l, qv_sat_i, err);
   const double qv_supersat_i = p3m_div(qv, qv_sat_i) - 1;
   double rhofacr, rhofaci, acn;
+  R mu;
   {
     const R ir = R(inv_rho), Tr = R(T_atm);
     rhofacr = double(m_pow(R(RHO_1000MB) * ir, R(.54)));
     rhofaci = double(m_pow(R(RHO_600MB) * ir, R(.54)));
-    const R dum = m_div(R(1.496e-6) * m_pow(Tr, R(1.5)), Tr + R(120));
-    acn = double(m_div(R(gravit) * R(RHO_H2O), R(18) * dum));
+    mu = viscosity(Tr, pow_of_log(Tr, lh, ll, R(1.5)));
+    acn = double(m_div(R(gravit) * R(RHO_H2O), R(18) * mu));
   }
   if (T_atm < T_zerodegc && qv_supersat_i >= -0.05) flags |= 1;
 
@@ -262,13 +274,26 @@ __device__ __forceinline__ void front_level(const KParams& p, int k, int i, cons
     for (int q = 0; q < 10; ++q) s[S_QC + q] = st[q];
     s[S_T] = T_atm; s[S_PRES] = pres; s[S_RHO] = rho; s[S_INV_RHO] = inv_rho;
     s[S_QVSL] = qv_sat_l; s[S_QVSI] = qv_sat_i; s[S_SUPI] = qv_supersat_i;
-    s[S_RHOFACI] = rhofaci; s[S_ACN] = acn;
+    s[S_RHOFACI] = rhofaci;
     s[S_CFL] = cfl; s[S_CFR] = cfr; s[S_CFI] = cfi;
     s[S_INV_EXNER] = inv_exner; s[S_QV_PREV] = qv_prev; s[S_T_PREV] = t_prev; s[S_NI_ACT] = ni_act;
+    // T and so its logarithm and viscosity are part 1's unless it clipped a trace
+    if (T_atm != T_first) {
+      if constexpr (sizeof(R) == 8) log_temperature(T_atm, lh, ll);
+      mu = viscosity(R(T_atm), pow_of_log(R(T_atm), lh, ll, R(1.5)));
+    }
+    if constexpr (sizeof(R) == 8) {
+      s[S_MU] = mu;
+      s[S_ACN] = acn;
+      s[S_T181] = p3m_pow_log(lh, ll, 1.81);
+    } else {
+      s.pair(S_MU) = make_float2(mu, float(acn));  // acn was formed in FP32
+    }
     lds_fence();
     P2Out o;
     // hydrometeorsPresent after part 2 (P3I/p3_main_impl.hpp:255-260): a column flag
-    if (part2_level<R>(rt, p.tab, dt, p.predictNc, p.prescribedCCN, p.e_melt, s, st, chg, o, err))
+    if (part2_level<R>(rt, RainOf<R>::get(p), p.tab, dt, p.predictNc, p.prescribedCCN, p.e_melt,
+                       s, st, chg, o, err))
       stat |= kStatusPart2;
     p.qv2qi_depos_tend[x] = o.qv2qi_depos_tend;
     p.precip_total_tend[x] = o.precip_total_tend;
@@ -381,7 +406,7 @@ __global__ __launch_bounds__(256) void p3_colstat_clear_kernel(int* colstat, int
   if (i < n) colstat[i] = 0;
 }
 
-// Parts 1 and 2 on the pointwise tiles; s_lds holds S_COUNT * kTileThreads doubles.
+// Parts 1 and 2 on the pointwise tiles; s_lds holds kSlots<R> * kTileThreads doubles.
 template <class R>
 __device__ __forceinline__ void front_tile(const KParams& p, int tile, double* s_lds) {
   int i, k;
@@ -397,15 +422,15 @@ __device__ __forceinline__ void front_tile(const KParams& p, int tile, double* s
   if (err) atomicOr(p.err, err);
 }
 
-// Wavefronts per SIMD the front kernel is compiled for.  Two in FP64 (244
-// VGPRs; at three it spills 89 of them: 276 against 225 us at 21600 x 72), three
-// in the mixed form (164 VGPRs).  The LDS slots are 52 KB per block of four
+// Wavefronts per SIMD the front kernel is compiled for.  Two in FP64 (248
+// VGPRs; at three it spilled 89 of them: 276 against 225 us at 21600 x 72), three
+// in the mixed form (165 VGPRs).  The LDS slots are 52 KB per block of four
 // wavefronts, so three blocks fit a CU.
 template <class R> constexpr int kFrontWaves = sizeof(R) == 8 ? 2 : 3;
 
 template <class R>
 __global__ __launch_bounds__(kTileThreads, kFrontWaves<R>) void p3_front_kernel(const KParams p) {
-  __shared__ double s_lds[S_COUNT * kTileThreads];
+  __shared__ double s_lds[kSlots<R> * kTileThreads];
   front_tile<R>(p, blockIdx.x, s_lds);
 }
 

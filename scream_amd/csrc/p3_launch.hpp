@@ -48,6 +48,10 @@ hipError_t launch_p3_fp64(const KParams& p, const Shape& sh, hipStream_t s, hipE
 hipError_t launch_p3_mixed(const KParams& p, const Shape& sh, hipStream_t s, hipEvent_t between = nullptr,
                            const SedFork* fork = nullptr);
 
+// RainGamma of the mixed form for the shape parameter mu, in its own arithmetic on
+// the current device; d: four floats of device memory for the result.
+hipError_t rain_gamma_mixed(float mu, float* d, RainGamma* out);
+
 // ---- batched form (p3_batch.hpp)
 // Sets whose sedimentation runs on the same lanes per column and levels per lane.
 struct SedClass {

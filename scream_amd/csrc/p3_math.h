@@ -79,6 +79,20 @@ P3M_FN double p3m_div_y(double a, double b, double y) { (void)y; return a / b; }
 P3M_FN double p3m_div(double a, double b) { return p3m_div_y(a, b, p3m_recip(b)); }
 P3M_FN double p3m_div_n(double a, double b) { return p3m_div_yn(a, b, p3m_recip(b)); }
 
+/* a * b + c for a constant c.  hipcc forms v_fmac, which overwrites c, and so
+ * moves every polynomial coefficient into vector registers first (three
+ * instructions a Horner step); the three-address form takes it from scalar
+ * registers, which the scalar unit fills. */
+#if P3M_DEVICE
+P3M_FN double p3m_fmac(double a, double b, double c) {
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+  return d;
+}
+#else
+P3M_FN double p3m_fmac(double a, double b, double c) { return fma(a, b, c); }
+#endif
+
 /* x * 2^k for x in [0.5, 2), one rounding where the result is subnormal (the
  * device's v_ldexp rounds the same) */
 P3M_FN double p3m_scale2(double x, int k) {
@@ -102,16 +116,16 @@ P3M_FN double p3m_exp_core(double x) {
   double r = fma(-kd, P3M_LN2_HI, x);
   r = fma(-kd, P3M_LN2_LO, r);
   double p = 1.0 / 6227020800.0;
-  p = fma(p, r, 1.0 / 479001600.0);
-  p = fma(p, r, 1.0 / 39916800.0);
-  p = fma(p, r, 1.0 / 3628800.0);
-  p = fma(p, r, 1.0 / 362880.0);
-  p = fma(p, r, 1.0 / 40320.0);
-  p = fma(p, r, 1.0 / 5040.0);
-  p = fma(p, r, 1.0 / 720.0);
-  p = fma(p, r, 1.0 / 120.0);
-  p = fma(p, r, 1.0 / 24.0);
-  p = fma(p, r, 1.0 / 6.0);
+  p = p3m_fmac(p, r, 1.0 / 479001600.0);
+  p = p3m_fmac(p, r, 1.0 / 39916800.0);
+  p = p3m_fmac(p, r, 1.0 / 3628800.0);
+  p = p3m_fmac(p, r, 1.0 / 362880.0);
+  p = p3m_fmac(p, r, 1.0 / 40320.0);
+  p = p3m_fmac(p, r, 1.0 / 5040.0);
+  p = p3m_fmac(p, r, 1.0 / 720.0);
+  p = p3m_fmac(p, r, 1.0 / 120.0);
+  p = p3m_fmac(p, r, 1.0 / 24.0);
+  p = p3m_fmac(p, r, 1.0 / 6.0);
   p = fma(p, r, 0.5);
   p = fma(p, r, 1.0);
   p = fma(p, r, 1.0);
@@ -161,27 +175,32 @@ P3M_FN double p3m_split(double x, int* e) {
 #endif
 }
 
+/* p * z + c for the logarithm's series: with the coefficient in scalar registers
+ * (p3m_fmac), or as the compiler forms it, which suits a wavefront that waits on
+ * its own chain: the moves then fill the wait, and an asm statement only keeps the
+ * scheduler from mixing chains. */
+#define P3M_LOG_STEP(p, z, c) (scalar ? p3m_fmac(p, z, c) : fma(p, z, c))
 /* log of a positive finite x as an unevaluated sum hi + lo.  x = 2^e m,
  * f = m - 1, s = f/(2+f), log m = 2 atanh s = f - f^2/2 + s (f^2/2 + R) with
  * R = sum_{k>=1} 2 s^(2k)/(2k+1) (the formulation of Sun's fdlibm __ieee754_log,
  * here with the exact series coefficients up to s^22). */
-P3M_FN void p3m_log_core(double x, double* hi, double* lo) {
+P3M_FN void p3m_log_series(double x, double* hi, double* lo, int scalar) {
   int e;
   const double m = p3m_split(x, &e);
   const double f = m - 1.0;
   const double s = p3m_div_n(f, 2.0 + f);
   const double z = s * s;
   double R = 2.0 / 23.0;
-  R = fma(R, z, 2.0 / 21.0);
-  R = fma(R, z, 2.0 / 19.0);
-  R = fma(R, z, 2.0 / 17.0);
-  R = fma(R, z, 2.0 / 15.0);
-  R = fma(R, z, 2.0 / 13.0);
-  R = fma(R, z, 2.0 / 11.0);
-  R = fma(R, z, 2.0 / 9.0);
-  R = fma(R, z, 2.0 / 7.0);
-  R = fma(R, z, 2.0 / 5.0);
-  R = fma(R, z, 2.0 / 3.0);
+  R = P3M_LOG_STEP(R, z, 2.0 / 21.0);
+  R = P3M_LOG_STEP(R, z, 2.0 / 19.0);
+  R = P3M_LOG_STEP(R, z, 2.0 / 17.0);
+  R = P3M_LOG_STEP(R, z, 2.0 / 15.0);
+  R = P3M_LOG_STEP(R, z, 2.0 / 13.0);
+  R = P3M_LOG_STEP(R, z, 2.0 / 11.0);
+  R = P3M_LOG_STEP(R, z, 2.0 / 9.0);
+  R = P3M_LOG_STEP(R, z, 2.0 / 7.0);
+  R = P3M_LOG_STEP(R, z, 2.0 / 5.0);
+  R = P3M_LOG_STEP(R, z, 2.0 / 3.0);
   R = R * z;
   const double hfsq = 0.5 * f * f;
   const double ed = (double)e;
@@ -191,6 +210,7 @@ P3M_FN void p3m_log_core(double x, double* hi, double* lo) {
   *hi = h;
   *lo = (A - h) + B;  /* |A| >= |B| whenever A != 0 */
 }
+P3M_FN void p3m_log_core(double x, double* hi, double* lo) { p3m_log_series(x, hi, lo, 1); }
 /* log of zero, an infinity, NaN or a negative number */
 P3M_FN double p3m_log_special(double x) {
   if (!(x == x) || x < 0) return p3m_nan();
@@ -208,6 +228,20 @@ P3M_FN double p3m_log10(double x) {
   double h, l;
   if (!p3m_positive(x)) return p3m_log_special(x);
   p3m_log_core(x, &h, &l);
+  return fma(h, P3M_INVLN10_HI, fma(h, P3M_INVLN10_LO, l * P3M_INVLN10_HI));
+}
+
+/* log10 of x > 0 without a branch: 0 and infinity count as the nearest positive
+ * finite numbers (the ice table's index is clamped far inside those), and
+ * chains of several arguments can be scheduled side by side. */
+P3M_FN double p3m_log10_pos(double x) {
+  double h, l;
+#if P3M_DEVICE
+  x = fmin(fmax(x, 2.2250738585072014e-308), 1.7976931348623157e308);
+#else
+  x = x > 1.7976931348623157e308 ? 1.7976931348623157e308 : (x < 2.2250738585072014e-308 ? 2.2250738585072014e-308 : x);
+#endif
+  p3m_log_series(x, &h, &l, 0);
   return fma(h, P3M_INVLN10_HI, fma(h, P3M_INVLN10_LO, l * P3M_INVLN10_HI));
 }
 
@@ -291,19 +325,19 @@ P3M_FN double p3m_expm1(double x) {
   const double ax = x < 0 ? -x : x;
   if (ax < 0.5) {
     double p = 1.0 / 20922789888000.0;     /* 1/16! */
-    p = fma(p, x, 1.0 / 1307674368000.0);  /* 1/15! */
-    p = fma(p, x, 1.0 / 87178291200.0);
-    p = fma(p, x, 1.0 / 6227020800.0);
-    p = fma(p, x, 1.0 / 479001600.0);
-    p = fma(p, x, 1.0 / 39916800.0);
-    p = fma(p, x, 1.0 / 3628800.0);
-    p = fma(p, x, 1.0 / 362880.0);
-    p = fma(p, x, 1.0 / 40320.0);
-    p = fma(p, x, 1.0 / 5040.0);
-    p = fma(p, x, 1.0 / 720.0);
-    p = fma(p, x, 1.0 / 120.0);
-    p = fma(p, x, 1.0 / 24.0);
-    p = fma(p, x, 1.0 / 6.0);
+    p = p3m_fmac(p, x, 1.0 / 1307674368000.0);  /* 1/15! */
+    p = p3m_fmac(p, x, 1.0 / 87178291200.0);
+    p = p3m_fmac(p, x, 1.0 / 6227020800.0);
+    p = p3m_fmac(p, x, 1.0 / 479001600.0);
+    p = p3m_fmac(p, x, 1.0 / 39916800.0);
+    p = p3m_fmac(p, x, 1.0 / 3628800.0);
+    p = p3m_fmac(p, x, 1.0 / 362880.0);
+    p = p3m_fmac(p, x, 1.0 / 40320.0);
+    p = p3m_fmac(p, x, 1.0 / 5040.0);
+    p = p3m_fmac(p, x, 1.0 / 720.0);
+    p = p3m_fmac(p, x, 1.0 / 120.0);
+    p = p3m_fmac(p, x, 1.0 / 24.0);
+    p = p3m_fmac(p, x, 1.0 / 6.0);
     p = fma(p, x, 0.5);
     return fma(p * x, x, x);
   }

@@ -16,12 +16,21 @@ namespace p3d {
 constexpr int kTileThreads = 256;
 enum Slot {
   S_QC, S_NC, S_QR, S_NR, S_QI, S_NI, S_QM, S_BM, S_QV, S_TH,  // the state after part 1
-  S_T, S_PRES, S_RHO, S_INV_RHO, S_QVSL, S_QVSI, S_SUPI, S_RHOFACI, S_ACN,
-  S_CFL, S_CFR, S_CFI, S_INV_EXNER, S_QV_PREV, S_T_PREV, S_NI_ACT, S_COUNT
+  S_T, S_PRES, S_RHO, S_INV_RHO, S_QVSL, S_QVSI, S_SUPI, S_RHOFACI,
+  S_MU,   // the viscosity at part 2's temperature (mixed form: with acn, two floats)
+  S_CFL, S_CFR, S_CFI, S_INV_EXNER, S_QV_PREV, S_T_PREV, S_NI_ACT, S_COUNT_MIXED,
+  S_ACN = S_COUNT_MIXED,
+  S_T181,  // T^1.81 at part 2's temperature
+  S_COUNT_FP64
 };
+// (The mixed form's 26 slots are what three blocks per CU leave room for.)
+template <class R> constexpr int kSlots = sizeof(R) == 8 ? S_COUNT_FP64 : S_COUNT_MIXED;
+// Dynamic viscosity from t and t^1.5 (P3I/p3_get_time_space_phys_variables_impl.hpp:20).
+template <class R> __device__ __forceinline__ R viscosity(R t, R t15) { return m_div(R(1.496e-6) * t15, t + R(120)); }
 struct Pt {
   double* b;
   __device__ __forceinline__ double& operator[](int slot) const { return b[slot * kTileThreads]; }
+  __device__ __forceinline__ float2& pair(int slot) const { return *reinterpret_cast<float2*>(b + slot * kTileThreads); }
 };
 // Keeps the compiler from carrying LDS values in registers across this point
 // (a thread reads only its own slots: no synchronisation is needed).
@@ -38,7 +47,7 @@ struct P2Out {
 // st is the state after part 2 (qc nc qr nr qi ni qm bm qv th); a bit of chg is
 // set for each of its fields that differs from the one after part 1.
 template <class R>
-__device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb, double dt, bool predictNc,
+__device__ __forceinline__ bool part2_level(const Runtime& rt, const RainGamma& rg, const Tables& tb, double dt, bool predictNc,
                                             bool prescribedCCN, double e_melt, const Pt s, double (&st)[10],
                                             unsigned& chg, P2Out& o, unsigned& err) {
   const double inv_dt = 1 / dt;
@@ -70,7 +79,7 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
   double rho_qm_cloud = 400;
   double evap_d = 0, nr_evap_d = 0;  // rain evaporation rates (finished in FP64)
   bool wetgrowth = false;
-  R mu_c = 0, lamc = 0, cdist = 0, cdist1 = 0, mu_r = 0, lamr = 0, cdistr = 0, logn0r = 0;
+  R mu_c = 0, lamc = 0, mu_r = 0, lamr = 0, cdistr = 0, logn0r = 0;
 
   const double T_atm = s[S_T];
   const bool skip_micro = !(qc_incld >= R(QSMALL) || qr_incld >= R(QSMALL) || qi_incld >= R(QSMALL));
@@ -78,9 +87,10 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
     const R Tr = R(T_atm), rhor = R(s[S_RHO]), rhofaci = R(s[S_RHOFACI]);
     const R dT_melt = R(T_atm - Tmelt);  // FP64 difference (exact in the FP64 form)
     // get_time_space_phys_variables, P3I/p3_get_time_space_phys_variables_impl.hpp:10-46
-    R T15, T181;  // T^1.5, T^1.81
-    pow_15_181(Tr, T15, T181);
-    const R mu = m_div(R(1.496e-6) * T15, Tr + R(120));
+    const R mu = sizeof(R) == 8 ? R(s[S_MU]) : R(s.pair(S_MU).x);
+    R T181;  // T^1.81
+    if constexpr (sizeof(R) == 8) T181 = s[S_T181];
+    else T181 = m_pow(Tr, R(1.81));
     const R dv = m_div(R(8.794e-5) * T181, R(s[S_PRES]));
     const R sc = m_div(mu, rhor * dv);
     const R dum_t = m_div(R(1), R(RV) * (Tr * Tr));
@@ -91,16 +101,16 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
     const R kap = R(1.414e+3) * mu;
     R eii;
     if (T_atm < 253.15) eii = R(0.001);
-    else if (T_atm < 273.15) eii = R(0.001) + R(T_atm - 253.15) * (R(0.3) - R(0.001)) / R(20);
+    else if (T_atm < 273.15) eii = R(0.001) + m_div(R(T_atm - 253.15) * (R(0.3) - R(0.001)), R(20));
     else eii = R(0.3);
 
-    get_cloud_dsd2<R>(qc_incld, nc_incld, mu_c, rhor, lamc, cdist, cdist1);
+    get_cloud_dsd2<R>(qc_incld, nc_incld, mu_c, rhor, lamc);
     put(S_NC, double(nc_incld) * s[S_CFL]);
 
     get_rain_dsd2<R>(rt, qr_incld, nr_incld, mu_r, lamr);
     // get_cdistr_logn0r, P3I/p3_dsd2_impl.hpp:128-148
     if (qr_incld >= R(QSMALL)) {
-      cdistr = m_div(nr_incld, m_tgamma(mu_r + R(1)));
+      cdistr = m_div(nr_incld, sizeof(R) == 8 || rg.mu == double(mu_r) ? R(rg.g1) : m_tgamma(mu_r + R(1)));
       logn0r = m_log10(cdistr) + (mu_r + R(1)) * m_log10(lamr);
     }
     put(S_NR, double(nr_incld) * s[S_CFR]);
@@ -155,10 +165,12 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
       ni_incld = vmin(ni_incld, tv_lammax * ni_incld);
       ni_incld = vmax(ni_incld, tv_lammin * ni_incld);
     }
+    // cbrt(sc) of the ventilation factors of ice and rain
+    const R cbrt_sc = qi_incld >= R(QSMALL) || qr_incld >= R(QSMALL) ? m_cbrt(sc) : R(0);
     // ventilation factor shared by melting, wet growth and the relaxation timescale
     // (every use below requires qi_incld >= QSMALL)
     const R vent = (qi_incld >= R(QSMALL))
-                       ? tv_qi2qr_melting + tv_vent_melt * m_cbrt(sc) * m_sqrt(m_div(rhofaci * rhor, mu))
+                       ? tv_qi2qr_melting + tv_vent_melt * cbrt_sc * m_sqrt(m_div(rhofaci * rhor, mu))
                        : R(0);
 
     if (rt.do_ice_production) {
@@ -181,12 +193,9 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
         const bool t_is_negative = T_atm <= Tmelt;
         const bool both = qi_incld >= R(QSMALL) && qr_incld >= R(QSMALL);
         const R f = R(rt.rain_to_ice_collection_factor);
-        if (both && t_is_negative) {
+        if (both && t_is_negative)
           qr2qi_collect_tend = m_pow(R(10.0), tv_qr2qi_collect + logn0r) * rhor * rhofaci * f * ni_incld;
-          nr_collect_tend = m_pow(R(10.0), tv_nr_collect + logn0r) * rhor * rhofaci * f * ni_incld;
-        }
-        if (both && !t_is_negative)
-          nr_collect_tend = m_pow(R(10.0), tv_nr_collect + logn0r) * rhor * rhofaci * f * ni_incld;
+        if (both) nr_collect_tend = m_pow(R(10.0), tv_nr_collect + logn0r) * rhor * rhofaci * f * ni_incld;
       }
       // ice_self_collection, P3I/p3_ice_collection_impl.hpp:108-151
       if (qi_incld >= R(QSMALL)) {
@@ -194,7 +203,7 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
         R tmp1 = R(0.0), Eii_fact = R(0.0);
         if (qm_pos) tmp1 = m_div(qm_incld, qi_incld);
         if (tmp1 < R(0.6) && qm_pos) Eii_fact = R(1);
-        if (tmp1 >= R(0.6) && tmp1 < R(0.9) && qm_pos) Eii_fact = R(1) - (tmp1 - R(0.6)) / R(0.3);
+        if (tmp1 >= R(0.6) && tmp1 < R(0.9) && qm_pos) Eii_fact = R(1) - m_div(tmp1 - R(0.6), R(0.3));
         if (tmp1 >= R(0.9) && qm_pos) Eii_fact = R(0);
         if (!qm_pos) Eii_fact = R(1);
         ni_selfcollect_tend = tv_ni_self_collect * rhor * eii * Eii_fact * rhofaci * ni_incld * ni_incld;
@@ -218,8 +227,8 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
       if (any_if) {
         const double qsat0 = p3m_div(ep_2 * e_melt, vmax(s[S_PRES], 1.e-3));  // qv_sat_dry(Tmelt, pres, liquid)
         const R dqs = R(qsat0 - s[S_QV]);
-        R qc_growth_rate = (vent * R(Pi * 2) * (rhor * R(latvap) * dv * dqs - dT_melt * kap) /
-                            (R(latice) + R(CpLiq) * dT_melt)) * ni_incld;
+        R qc_growth_rate = m_div(vent * R(Pi * 2) * (rhor * R(latvap) * dv * dqs - dT_melt * kap),
+                                 R(latice) + R(CpLiq) * dT_melt) * ni_incld;
         qc_growth_rate = vmax(qc_growth_rate, R(0.0));
         const R dum = vmax(R(0.0), (qc2qi_collect_tend + qr2qi_collect_tend) - qc_growth_rate);
         const bool dum_ge_small = dum >= R(1.0e-10);
@@ -247,7 +256,8 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
     if (qc2qi_collect_tend >= R(QSMALL) && T_atm < T_zerodegc) {
       const R vtrmi1 = tv_qi_fallspd * rhofaci;
       if (qc_incld >= R(QSMALL)) {
-        const R Vt_qc = m_div(R(s[S_ACN]) * m_tgamma(R(4 + bcn) + mu_c), m_pow(lamc, R(bcn)) * m_tgamma(R(4) + mu_c));
+        const R acn = sizeof(R) == 8 ? R(s[S_ACN]) : R(s.pair(S_MU).y);
+        const R Vt_qc = m_div(acn * m_tgamma(R(4 + bcn) + mu_c), m_pow(lamc, R(bcn)) * m_tgamma(R(4) + mu_c));
         const R D_c = m_div(R(4) + mu_c, lamc);
         const R V_impact = m_fabs(vtrmi1 - Vt_qc);
         const R inv_Tc = m_div(R(1), vmin(R(-0.001), R(T_atm - T_zerodegc)));
@@ -262,6 +272,8 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
       const R dT_frz = R(T_zerodegc - T_atm);
       // cldliq_immersion_freezing, P3I/p3_cldliq_imm_freezing_impl.hpp:15-52
       if (qc_incld >= R(QSMALL) && T_atm <= T_rainfrz) {
+        // (cdist1 of get_cloud_dsd2, P3I/p3_dsd2_impl.hpp:66, has no other use)
+        const R cdist1 = m_div(nc_incld, m_tgamma(mu_c + R(1)));
         const R expAimmDt = m_exp(aimm * dT_frz);
         const R x = m_div(R(1), lamc);
         const R inv_lamc3 = x * x * x;
@@ -275,9 +287,9 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
       }
       // rain_immersion_freezing, P3I/p3_rain_imm_freezing_impl.hpp:14-46
       if (qr_incld >= R(QSMALL) && T_atm <= T_rainfrz) {
-        qr2qi_immers_freeze_tend = R(CONS6) * m_exp(m_log(cdistr) + m_log(m_tgamma(R(7.) + mu_r)) - R(6.) * m_log(lamr)) *
+        qr2qi_immers_freeze_tend = R(CONS6) * m_exp(m_log(cdistr) + (sizeof(R) == 8 || rg.mu == double(mu_r) ? R(rg.log_g7) : m_log(m_tgamma(R(7.) + mu_r))) - R(6.) * m_log(lamr)) *
                                    m_exp(aimm * dT_frz);
-        nr2ni_immers_freeze_tend = R(CONS5) * m_exp(m_log(cdistr) + m_log(m_tgamma(R(4.) + mu_r)) - R(3.) * m_log(lamr)) *
+        nr2ni_immers_freeze_tend = R(CONS5) * m_exp(m_log(cdistr) + (sizeof(R) == 8 || rg.mu == double(mu_r) ? R(rg.log_g4) : m_log(m_tgamma(R(4.) + mu_r))) - R(3.) * m_log(lamr)) *
                                    m_exp(aimm * dT_frz);
       }
     }
@@ -287,7 +299,7 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const Tables& tb,
     if (qr_incld >= R(QSMALL)) {
       const Tab3<R> t3 = lookup3<R>(mu_r, lamr);
       epsr = R(2) * R(Pi) * cdistr * rhor * dv *
-             (m_div(R(f1r) * m_tgamma(mu_r + R(2)), lamr) + R(f2r) * m_sqrt(m_div(rhor, mu)) * m_cbrt(sc) * apply_table3<R>(TabOf<R>::get(tb).revap, t3));
+             (m_div(R(f1r) * (sizeof(R) == 8 || rg.mu == double(mu_r) ? R(rg.g2) : m_tgamma(mu_r + R(2))), lamr) + R(f2r) * m_sqrt(m_div(rhor, mu)) * cbrt_sc * apply_table3<R>(TabOf<R>::get(tb).revap, t3));
     }
 
     // evaporate_rain, P3I/p3_evaporate_rain_impl.hpp:83-201

@@ -51,17 +51,13 @@ __device__ __forceinline__ float m_fabs(float x) { return ::fabsf(x); }
 __device__ __forceinline__ double m_div(double a, double b) { return p3m_div(a, b); }
 __device__ __forceinline__ float m_div(float a, float b) { return a / b; }
 
-// t^1.5 and t^1.81 of a temperature (FP64: from one logarithm; NaN where t is
-// not positive and finite)
-__device__ __forceinline__ void pow_15_181(double t, double& a, double& b) {
-  double h, l;
+// t^y of a temperature whose logarithm is at hand (FP64: from it, h + l; NaN
+// where t is not positive and finite; the mixed form takes its own pow)
+__device__ __forceinline__ double pow_of_log(double, double h, double l, double y) { return p3m_pow_log(h, l, y); }
+__device__ __forceinline__ float pow_of_log(float t, double, double, float y) { return m_pow(t, y); }
+// The logarithm of a temperature as h + l (NaN where it is not positive and finite).
+__device__ __forceinline__ void log_temperature(double t, double& h, double& l) {
   p3m_log_core(p3m_positive(t) ? t : p3m_nan(), &h, &l);
-  a = p3m_pow_log(h, l, 1.5);
-  b = p3m_pow_log(h, l, 1.81);
-}
-__device__ __forceinline__ void pow_15_181(float t, float& a, float& b) {
-  a = m_pow(t, 1.5f);
-  b = m_pow(t, 1.81f);
 }
 
 // ekat::impl::min/max on scalars (ternary form, argument order preserved)
@@ -90,11 +86,12 @@ __device__ __forceinline__ double qv_sat_dry_liquid(double t, double p, unsigned
   check_temperature(t, err);
   return p3m_div(ep_2 * mk_svp_liquid(t, p3m_log(t), p3m_recip(t)), vmax(p, 1.e-3));
 }
-// qv_sat_dry over liquid and over ice (liquid again from Tmelt up) at one point:
-// log(t) and both reciprocals are formed once
-__device__ __forceinline__ void qv_sat_dry_both(double t, double p, double& liquid, double& ice, unsigned& err) {
+// qv_sat_dry over liquid and over ice (liquid again from Tmelt up) at one point,
+// from log(t); both reciprocals are formed once
+__device__ __forceinline__ void qv_sat_dry_both(double t, double logt, double p, double& liquid, double& ice,
+                                                unsigned& err) {
   check_temperature(t, err);
-  const double logt = p3m_log(t), rt = p3m_recip(t);
+  const double rt = p3m_recip(t);
   const double pm = vmax(p, 1.e-3), rp = p3m_recip(pm);
   liquid = p3m_div_y(ep_2 * mk_svp_liquid(t, logt, rt), pm, rp);
   ice = liquid;
@@ -130,6 +127,16 @@ template <class T> struct TableSet {
   const T* ice_p3;   // [5][4][50][4]: quantities 5,6,7,11 (part 3)
   const T* rain_v;   // [300][10][2]: vm, vn (rain sedimentation)
 };
+// Functions of the runtime's one rain shape parameter (constant_mu_rain), so that
+// they are not computed at every level with rain: in FP64 the host's values, from
+// the same portable functions; in the mixed form the device's own FP32 values for
+// the default parameter, formed once per context.  mu: the parameter they belong
+// to, as the form's arithmetic holds it (with another one the kernels compute them).
+struct RainGamma {
+  double mu;
+  double g1, g2;          // Gamma(mu + 1), Gamma(mu + 2)
+  double log_g7, log_g4;  // log Gamma(mu + 7), log Gamma(mu + 4)
+};
 struct Tables {
   TableSet<double> d;  // the drop-in FP64 form
   TableSet<float> f;   // the mixed-precision form (half the gather bytes, no conversions)
@@ -151,11 +158,15 @@ template <class R> struct TabIce { int dumi, dumii, dumjj; R dum1, dum4, dum5; }
 template <class R> struct TabRain { int dumj; R dum3; };
 template <class R> struct Tab3 { int dumii, dumjj; R rdumii, rdumjj; };
 
-// lookup_ice, P3I/p3_table_ice_impl.hpp:80-138
+// log10 of a ratio that is positive (FP64: without a branch)
+__device__ __forceinline__ double m_log10_pos(double x) { return p3m_log10_pos(x); }
+__device__ __forceinline__ float m_log10_pos(float x) { return m_log10(x); }
+
+// lookup_ice, P3I/p3_table_ice_impl.hpp:80-138 (qi and ni are positive)
 template <class R>
 __device__ __forceinline__ TabIce<R> lookup_ice(R qi, R ni, R qm, R rhop) {
   TabIce<R> t;
-  t.dum1 = (m_log10(m_div(qi, ni)) + R(18)) * R(lookup_table_1a_dum1_c) - R(10);
+  t.dum1 = (m_log10_pos(m_div(qi, ni)) + R(18)) * R(lookup_table_1a_dum1_c) - R(10);
   t.dumi = (int)t.dum1;
   t.dum1 = vmin(t.dum1, R(isize));
   t.dum1 = vmax(t.dum1, R(1.));
@@ -405,8 +416,8 @@ __device__ __forceinline__ void apply_table3_v(const R* __restrict__ table, cons
 // ---------------------------------------------------------------- size distributions
 // get_cloud_dsd2, P3I/p3_dsd2_impl.hpp:14-71 (iparam = 3, nu stays 0)
 template <class R>
-__device__ __forceinline__ void get_cloud_dsd2(R qc, R& nc, R& mu_c, R rho, R& lamc, R& cdist, R& cdist1) {
-  lamc = R(0); cdist = R(0); cdist1 = R(0); mu_c = R(0);
+__device__ __forceinline__ void get_cloud_dsd2(R qc, R& nc, R& mu_c, R rho, R& lamc) {
+  lamc = R(0); mu_c = R(0);
   if (qc >= R(QSMALL)) {
     nc = vmax(nc, R(NSMALL));
     R m = R(0.0005714) * (nc * R(1.e-6) * rho) + R(0.2714);
@@ -422,8 +433,6 @@ __device__ __forceinline__ void get_cloud_dsd2(R qc, R& nc, R& mu_c, R rho, R& l
     if (gt) lamc = lammax;
     if (lt || gt)
       nc = m_div(R(6) * (lamc * lamc * lamc) * qc, R(Pi) * R(RHO_H2O) * (m + R(3)) * (m + R(2)) * (m + R(1)));
-    cdist = m_div(nc * (m + R(1)), lamc);
-    cdist1 = m_div(nc, m_tgamma(m + R(1)));
   }
 }
 

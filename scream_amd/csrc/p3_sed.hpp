@@ -217,8 +217,8 @@ struct SedRun {
             nc_incld = incloud_div(nc, cfl, rcf[t]);
           }
           if (qc_incld > R(QSMALL)) {
-            R ncr = nc_incld, mu_c, lamc, cdist, cdist1;
-            get_cloud_dsd2<R>(qc_incld, ncr, mu_c, R(rho), lamc, cdist, cdist1);
+            R ncr = nc_incld, mu_c, lamc;
+            get_cloud_dsd2<R>(qc_incld, ncr, mu_c, R(rho), lamc);
             q[1][t] = double(ncr) * cf[t];
             const R dum = m_div(R(1), m_pow(lamc, R(bcn)));
             const R acn = R(coef[t]);
@@ -493,8 +493,8 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
     // cloud
     if (qc >= QSMALL) {
       const double rcfl = p3m_recip(cfl);
-      R ncr = R(p3m_div_y(nc, cfl, rcfl)), mu_c, lamc, cd, cd1;
-      get_cloud_dsd2<R>(R(p3m_div_y(qc, cfl, rcfl)), ncr, mu_c, R(rho), lamc, cd, cd1);
+      R ncr = R(p3m_div_y(nc, cfl, rcfl)), mu_c, lamc;
+      get_cloud_dsd2<R>(R(p3m_div_y(qc, cfl, rcfl)), ncr, mu_c, R(rho), lamc);
       nc = double(ncr) * cfl;
       reff_c = double(m_div(R(0.5) * (mu_c + R(3)), lamc));
     } else {

@@ -221,6 +221,9 @@ int fill_params(const p3x_context* c, const p3x_runtime* runtime, const p3x_prog
   k.tab.f = table_set(c->d_tab_f);
   static_assert(sizeof(p3d::Runtime) == sizeof(p3x_runtime), "runtime layouts differ");
   std::memcpy(&k.rt, runtime, sizeof(k.rt));
+  const double mu = runtime->constant_mu_rain;
+  k.rgf = c->rain_mixed;
+  k.rg = {mu, p3m_tgamma(mu + 1), p3m_tgamma(mu + 2), p3m_log(p3m_tgamma(7. + mu)), p3m_log(p3m_tgamma(4. + mu))};
   k.dt = infra->dt;
   k.predictNc = infra->predictNc ? 1 : 0;
   k.prescribedCCN = infra->prescribedCCN ? 1 : 0;
@@ -320,8 +323,12 @@ extern "C" int p3x_init(const p3x_table_data* t, p3x_context** out) {
   };
   up(&c->d_tab, pack_tables<double>(t));
   up(&c->d_tab_f, pack_tables<float>(t));
-  if (e == hipSuccess) e = hipMalloc((void**)&c->d_err, sizeof(unsigned));
+  // the error word, and room for four floats while the context is made
+  if (e == hipSuccess) e = hipMalloc((void**)&c->d_err, 8 * sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(c->d_err, 0, sizeof(unsigned));
+  p3x_runtime rt;
+  p3x_runtime_defaults(&rt);
+  if (e == hipSuccess) e = p3d::rain_gamma_mixed((float)rt.constant_mu_rain, (float*)(c->d_err + 4), &c->rain_mixed);
   if (e == hipSuccess) e = hipEventCreate(&c->ev0);
   if (e == hipSuccess) e = hipEventCreate(&c->ev1);
   if (e == hipSuccess) e = hipEventCreate(&c->ev_mid);

@@ -18,6 +18,7 @@ struct p3x_context {
   double* d_scratch = nullptr;
   size_t scratch_bytes = 0;
   unsigned* d_err = nullptr;
+  p3d::RainGamma rain_mixed{};  // of the mixed form, for the default constant_mu_rain
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t ev_mid = nullptr;  // between the part 1 + 2 and the sedimentation kernels
   // the liquid sedimentation kernel's stream (beside the ice kernel) and its

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kTileThreads, kFrontWaves<R>) void p3_front_batch(c
 // Part 3 one thread per (level, column), after the sedimentation launches;
 // first: the pointwise tile offsets.
 template <class R, bool PERSIST>
-__global__ __launch_bounds__(kTileThreads) void p3_part3_lvl_batch(const KParams* __restrict__ sets,
+__global__ __launch_bounds__(kTileThreads, kPart3Waves) void p3_part3_lvl_batch(const KParams* __restrict__ sets,
                                                                   const int* __restrict__ first, int nsets) {
   const auto sets4 = (const __attribute__((address_space(4))) KParams*)sets;
   for_virtual_blocks<PERSIST>(first[nsets], [&](int vb) {

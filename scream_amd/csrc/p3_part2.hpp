@@ -657,9 +657,11 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const RainGamma& 
     } else present = true;
 
     // P3I/p3_main_impl_part2.hpp:514-517
-    double ni_incld_d = p3m_div(u.ni, cld_frac_i);
-    impose_max_total_ni<double>(ni_incld_d, rt.max_total_ni, s[S_INV_RHO]);
-    u.ni = ni_incld_d * cld_frac_i;
+    if (u.ni != 0) {  // (0 stays 0, also where the cloud fraction is 0)
+      double ni_incld_d = p3m_div(u.ni, cld_frac_i);
+      impose_max_total_ni<double>(ni_incld_d, rt.max_total_ni, s[S_INV_RHO]);
+      u.ni = ni_incld_d * cld_frac_i;
+    }
     const double out[10] = {u.qc, u.nc, u.qr, u.nr, u.qi, u.ni, u.qm, u.bm, u.qv, u.th};
 #pragma unroll
     for (int q = 0; q < 10; ++q) {

@@ -362,8 +362,11 @@ struct SedRun {
       if (k < nlev) {
         const size_t x = p.at(i, k);
         if (k <= k_bot) {
+          // an empty level is empty in every field (part 3 would zero the others):
+          // part 3 then need not read them
+          const bool empty = q[0][t] == 0;
 #pragma unroll
-          for (int f = 0; f < NF; ++f) fld[f][x] = q[f][t];
+          for (int f = 0; f < NF; ++f) fld[f][x] = empty ? q[0][t] : q[f][t];
         }
         if (SP == 1) p.precip_liq_flux[p.atf(i, k + 1)] = pflux[t];  // rain_sed :140-153, interface k+1
       }
@@ -459,19 +462,42 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
   if (k == nlev - 1) p.precip_ice_flux[p.atf(i, nlev)] = 0;
   double reff_c = 10.e-6, reff_i = 25.e-6, reff_r = 500.e-6, rho_qi = 0;
   double qc = 0, nc = 0, qr = 0, nr = 0, qi = 0, ni = 0, qm = 0, bm = 0, qv = 0, th = 0;
+  // The kernel runs at the HBM rate, so a point reads what it needs: an absent
+  // species' other fields are zero (parts 1 and 2 and sedimentation leave them so),
+  // and th, qv and the liquid exchange change only where a remainder below QSMALL
+  // is given back to the vapour or liquid freezes.
+  const bool all = p.amble.on || p.dbg_check;
+  double T_part1 = 0, inv_exner = 0, vap_liq = 0, dp = 0, dz = 0, cfl = 0, cfr = 0, cfi = 0;
+  bool thermo = false;  // th, qv, inv_exner are loaded
+  auto load_thermo = [&] {
+    thermo = true;
+    qv = p.qv[x]; th = p.th[x];
+    inv_exner = p.inv_exner[x];
+  };
+  bool gives = false;  // cloud or rain gives back a remainder
   if (active || p.amble.on) {
-    qc = p.qc[x]; nc = p.nc[x]; qr = p.qr[x]; nr = p.nr[x]; qi = p.qi[x]; ni = p.ni[x];
-    qm = p.qm[x]; bm = p.bm[x]; qv = p.qv[x]; th = p.th[x];
+    qc = p.qc[x]; qr = p.qr[x]; qi = p.qi[x];
+    const bool cloud = qc >= QSMALL, rain = qr >= QSMALL;
+    gives = (qc != 0 && !cloud) || (qr != 0 && !rain);
+    if (all || qc != 0) nc = p.nc[x];
+    if (all || qr != 0) nr = p.nr[x];
+    if (all || qi != 0) { ni = p.ni[x]; qm = p.qm[x]; bm = p.bm[x]; }
+    if (all || gives || (qi != 0 && !(qi >= QSMALL))) load_thermo();
+    if (cloud || rain) T_part1 = p.sc(SC_T, i, k);
+    if (cloud) cfl = p.cld_frac_l[x];
+    if (rain) cfr = p.cld_frac_r[x];
+    if (cloud || rain || qi >= QSMALL) { dp = p.dpres[x]; dz = p.dz[x]; cfi = p.cld_frac_i[x]; }
+    if (gives) vap_liq = p.vap_liq_exchange[x];
   }
   // the state as it is in memory: without the post-amble, a field that part 3
   // leaves bit for bit unchanged is not stored again
   const double in[10] = {qc, nc, qr, nr, qi, ni, qm, bm, qv, th};
   if (active) {
-    const double inv_exner = p.inv_exner[x];
     if (rt.do_ice_production) {
-      const bool t_lt = p.sc(SC_T, i, k) < T_homogfrz;
+      const bool t_lt = T_part1 < T_homogfrz;  // (0 where there is no liquid)
       const bool qc_ge = t_lt && qc >= QSMALL;
       const bool qr_ge = t_lt && qr >= QSMALL;
+      if ((qc_ge || qr_ge) && !thermo) load_thermo();
       const double Qc_nuc = qc, Qr_nuc = qr;
       const double Nc_nuc = vmax(nc, NSMALL), Nr_nuc = vmax(nr, NSMALL);
       if (qc_ge) {
@@ -486,10 +512,7 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
       if (qr_ge) { qr = 0; nr = 0; }
     }
     // p3_main_part3, P3I/p3_main_impl_part3.hpp:60-199 (only the fields p3_main outputs)
-    const double rho = air_density(p.dpres[x], p.dz[x]);
-    const double inv_rho = p3m_div(1.0, rho);
-    const double cfl = p.cld_frac_l[x], cfr = p.cld_frac_r[x], cfi = p.cld_frac_i[x];
-    double vap_liq = p.vap_liq_exchange[x];
+    const double rho = air_density(dp, dz);
     // cloud
     if (qc >= QSMALL) {
       const double rcfl = p3m_recip(cfl);
@@ -517,45 +540,38 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
       qr = 0; nr = 0;
     }
     // ice
-    {
-      const bool qi_gt = qi >= QSMALL;
+    if (qi >= QSMALL) {
+      const double inv_rho = p3m_div(1.0, rho);
       ni = vmax(ni, NSMALL);
       const double rcfi = p3m_recip(cfi);
       const double qi_incld = p3m_div_y(qi, cfi, rcfi);
       double ni_incld = p3m_div_y(ni, cfi, rcfi);
       double qm_incld = p3m_div_y(qm, cfi, rcfi), bm_incld = p3m_div_y(bm, cfi, rcfi);
       R qmr = R(qm_incld), bmr = R(bm_incld);
-      R rhop = 0;
-      if (qi_gt) {
-        rhop = calc_bulk_rho_rime<R>(rt, R(qi_incld), qmr, bmr);
-        qm_incld = double(qmr); bm_incld = double(bmr);
-        qm = qm_incld * cfi;
-        bm = bm_incld * cfi;
-      }
+      const R rhop = calc_bulk_rho_rime<R>(rt, R(qi_incld), qmr, bmr);
+      qm_incld = double(qmr); bm_incld = double(bmr);
+      qm = qm_incld * cfi;
+      bm = bm_incld * cfi;
       impose_max_total_ni<double>(ni_incld, rt.max_total_ni, inv_rho);
-      if (qi_gt) {
-        const TabIce<R> ti = lookup_ice<R>(R(qi_incld), R(ni_incld), R(qm_incld), rhop);
-        if (p.dbg_ice_idx) p.dbg_ice_idx[x] = ti.dumjj * 10000 + ti.dumii * 100 + ti.dumi;
-        R v[4];  // quantities 5, 6, 7, 11
-        apply_table_ice_rec<4, 4, R>(TabOf<R>::get(p.tab).ice_p3, ti, v);
-        const R t_eff = v[0], t_lammax = v[1], t_lammin = v[2], t_rhomm = v[3];
-        ni_incld = vmin(ni_incld, double(t_lammax) * ni_incld);
-        ni_incld = vmax(ni_incld, double(t_lammin) * ni_incld);
-        reff_i = double(t_eff);
-        rho_qi = double(t_rhomm);
-      } else if (p.dbg_ice_idx) {
-        p.dbg_ice_idx[x] = -1;
-      }
+      const TabIce<R> ti = lookup_ice<R>(R(qi_incld), R(ni_incld), R(qm_incld), rhop);
+      if (p.dbg_ice_idx) p.dbg_ice_idx[x] = ti.dumjj * 10000 + ti.dumii * 100 + ti.dumi;
+      R v[4];  // quantities 5, 6, 7, 11
+      apply_table_ice_rec<4, 4, R>(TabOf<R>::get(p.tab).ice_p3, ti, v);
+      const R t_eff = v[0], t_lammax = v[1], t_lammin = v[2], t_rhomm = v[3];
+      ni_incld = vmin(ni_incld, double(t_lammax) * ni_incld);
+      ni_incld = vmax(ni_incld, double(t_lammin) * ni_incld);
+      reff_i = double(t_eff);
+      rho_qi = double(t_rhomm);
       ni = ni_incld * cfi;
-      if (qm < QSMALL && qi_gt) { qm = 0; bm = 0; }
-      if (!qi_gt) {
-        qv = qv + qi;
-        th = th - inv_exner * qi * (latvap + latice) * inv_cp;
-        qi = 0; ni = 0; qm = 0; bm = 0;
-      }
+      if (qm < QSMALL) { qm = 0; bm = 0; }
+    } else {
+      if (p.dbg_ice_idx) p.dbg_ice_idx[x] = -1;
+      qv = qv + qi;
+      th = th - inv_exner * qi * (latvap + latice) * inv_cp;
+      qi = 0; ni = 0; qm = 0; bm = 0;
     }
     if (qr < QSMALL) nr = 0;
-    p.vap_liq_exchange[x] = vap_liq;
+    if (gives) p.vap_liq_exchange[x] = vap_liq;
     if (p.dbg_check) {
       // check_values (P3I/p3_check_values_impl.hpp:25-79, called after part 3 at
       // P3I/p3_main_impl.hpp:316-324 in debug builds) on T = th exner and qv: T outside
@@ -693,6 +709,13 @@ __device__ __forceinline__ void sed_block(const KParams& p, int bid, const R* __
 
 // Part 3 as a kernel of its own, one thread per (level, column) on the
 // pointwise tiles, after the sedimentation kernel.
+//
+// Bound by HBM.  Reading all 18 fields at every point it took 70 us at 21600 x 72
+// FP64 and 82 us at 16384 x 128 mixed (4.4 TB/s); reading what a point needs
+// (part3_level), 54 and 62 us, and with registers for four wavefronts per SIMD
+// (128 VGPRs instead of 134), which hide the second round of loads, 51 and 56 us.
+// At five it spills (110 us in FP64).
+constexpr int kPart3Waves = 4;
 template <class R>
 __device__ __forceinline__ void part3_tile(const KParams& p, int tile) {
   int i, k;
@@ -723,7 +746,7 @@ __device__ __forceinline__ void part3_tile(const KParams& p, int tile) {
 }
 
 template <class R>
-__global__ __launch_bounds__(kTileThreads) void p3_part3_lvl_kernel(const KParams p) {
+__global__ __launch_bounds__(kTileThreads, kPart3Waves) void p3_part3_lvl_kernel(const KParams p) {
   part3_tile<R>(p, blockIdx.x);
 }
 

@@ -46,6 +46,25 @@ hipError_t noalloc_scratch_on(int dev, double** out) {
   *out = (double*)ptr;
   return hipSuccess;
 }
+
+// RainGamma of the mixed form for the default constant_mu_rain: the FP32 values of
+// this code on this architecture, formed by the process's first context.
+std::mutex g_rain_mu;
+p3d::RainGamma g_rain_mixed{};
+bool g_rain_known = false;
+
+hipError_t default_rain_gamma(float* d, p3d::RainGamma* out) {
+  std::lock_guard<std::mutex> lk(g_rain_mu);
+  if (!g_rain_known) {
+    p3x_runtime rt;
+    p3x_runtime_defaults(&rt);
+    const hipError_t e = p3d::rain_gamma_mixed((float)rt.constant_mu_rain, d, &g_rain_mixed);
+    if (e != hipSuccess) return e;
+    g_rain_known = true;
+  }
+  *out = g_rain_mixed;
+  return hipSuccess;
+}
 }  // namespace
 
 
@@ -323,12 +342,10 @@ extern "C" int p3x_init(const p3x_table_data* t, p3x_context** out) {
   };
   up(&c->d_tab, pack_tables<double>(t));
   up(&c->d_tab_f, pack_tables<float>(t));
-  // the error word, and room for four floats while the context is made
+  // the error word, and room for the four floats of default_rain_gamma
   if (e == hipSuccess) e = hipMalloc((void**)&c->d_err, 8 * sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(c->d_err, 0, sizeof(unsigned));
-  p3x_runtime rt;
-  p3x_runtime_defaults(&rt);
-  if (e == hipSuccess) e = p3d::rain_gamma_mixed((float)rt.constant_mu_rain, (float*)(c->d_err + 4), &c->rain_mixed);
+  if (e == hipSuccess) e = default_rain_gamma((float*)(c->d_err + 4), &c->rain_mixed);
   if (e == hipSuccess) e = hipEventCreate(&c->ev0);
   if (e == hipSuccess) e = hipEventCreate(&c->ev1);
   if (e == hipSuccess) e = hipEventCreate(&c->ev_mid);

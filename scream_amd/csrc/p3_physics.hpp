@@ -467,14 +467,15 @@ __device__ __forceinline__ R calc_bulk_rho_rime(const Runtime& rt, R qi_tot, R& 
   if (gt && lt_min) rho_rime = R(rt.min_rime_rho);
   if (gt && gt_max) rho_rime = R(rt.max_rime_rho);
   const bool clamped = gt && (gt_max || lt_min);
-  if (lt) { qi_rim = R(0); bi_rim = R(0); rho_rime = R(0); }
+  // The reference zeroes both fields here where `lt`; its later tests then fail, as
+  // they do with rho_rime = 0, so that one zeroing at the end serves.
   // The reference sets bi_rim = qi_rim / rho_rime for a clamped density, then
   // again with qi_rim = qi_tot when the rime exceeds the total; the second
   // overrides the first, and `lt` excludes both, so one division serves.
   const bool over = qi_rim > qi_tot && rho_rime > R(0);
   if (over || clamped) bi_rim = m_div(over ? qi_tot : qi_rim, rho_rime);
   if (over) qi_rim = qi_tot;
-  if (qi_rim < R(QSMALL)) { qi_rim = R(0); bi_rim = R(0); }
+  if (lt || qi_rim < R(QSMALL)) { qi_rim = R(0); bi_rim = R(0); }
   return rho_rime;
 }
 

@@ -101,14 +101,23 @@ template <class R, int G, int L> constexpr int sed_waves_per_simd() {
 // ice-sedimentation records.  Where the blocks the kernel's occupancy puts on
 // one CU (blocks of 4 wavefronts) can each hold it in the CU's 160 KB of LDS,
 // the copy is of the records that also carry each quantity's difference to
-// the next size cell (64 KB in FP64, 32 KB in FP32), which saves the four
+// the next size cell (80 KB in FP64, 32 KB in FP32), which saves the four
 // size-direction subtractions per quantity; elsewhere (the FP64 kernels at
-// three wavefronts per SIMD) it is of the plain records (32 KB).
+// three wavefronts per SIMD) it is of the plain records (48 KB).
 constexpr int kIceCells = densize * rimsize * isize;
 template <class R, int L> constexpr bool ice_rec_dif() {
-  return sed_waves_per_simd<R, SED_ICE, L>() * kIceCells * 8 * (int)sizeof(R) <= 160 * 1024;
+  return sed_waves_per_simd<R, SED_ICE, L>() * kIceCells * (sizeof(R) == 8 ? 10 : 8) * (int)sizeof(R) <= 160 * 1024;
 }
-template <class R, int L> constexpr int ice_lds_len() { return kIceCells * (ice_rec_dif<R, L>() ? 8 : 4); }
+// Values per cell in LDS.  All lanes read the same 16-byte part of their cells'
+// records at a time, so the records' stride decides which of the 16 bank groups
+// (16 bytes each) a read can fall on: FP64 records of 64 bytes would use 4 of them
+// and those of 32 bytes 8; one part more per record uses all 16 (before, conflicts
+// held the LDS 27 % of the kernel's time at 21600 x 72 FP64: sedimentation and part
+// 3 635 -> 608 us).  The mixed form's 32-byte records stay: a longer stride would
+// cost the fourth block per CU.
+template <class R, int L> constexpr int ice_rec_len() { return ice_rec_dif<R, L>() ? 8 : 4; }
+template <class R, int L> constexpr int ice_lds_stride() { return ice_rec_len<R, L>() + (sizeof(R) == 8 ? 2 : 0); }
+template <class R, int L> constexpr int ice_lds_len() { return kIceCells * ice_lds_stride<R, L>(); }
 
 // An in-cloud value q / cf after the first substep.  In FP64 the reciprocal
 // rcf = p3m_recip(cf) is formed once per level and run (cf does not change over
@@ -136,7 +145,7 @@ struct Geo {
 // the upwind flux are cross-lane operations inside the group).  DIF: the ice
 // records in ice_tab carry their size-direction differences (the layout the
 // kernel staged, chosen by its own levels per lane, not by this run's L).
-template <int SP, class R, int LPC, int L, bool DIF>
+template <int SP, class R, int LPC, int L, bool DIF, int STRIDE>
 struct SedRun {
   static constexpr int NF = SP == 2 ? 4 : 2;  // fields held (cloud always holds nc: its DSD rewrites it)
   Geo<L> g;
@@ -277,16 +286,16 @@ struct SedRun {
             // quantities 0, 1, 6, 7 of the records (in FP64 as two halves, which bounds the registers)
             R v[4];
             if constexpr (sizeof(R) == 4) {
-              if constexpr (DIF) apply_table_ice_dif<4, 8, 4, R>(ice_tab, ti, v, 0);
-              else apply_table_ice_rec<4, 4, R>(ice_tab, ti, v, 0);
+              if constexpr (DIF) apply_table_ice_dif<4, STRIDE, 4, R>(ice_tab, ti, v, 0);
+              else apply_table_ice_rec<4, STRIDE, R>(ice_tab, ti, v, 0);
             } else {
               R a[2], b[2];
               if constexpr (DIF) {
-                apply_table_ice_dif<2, 8, 4, R>(ice_tab, ti, a, 0);
-                apply_table_ice_dif<2, 8, 4, R>(ice_tab, ti, b, 2);
+                apply_table_ice_dif<2, STRIDE, 4, R>(ice_tab, ti, a, 0);
+                apply_table_ice_dif<2, STRIDE, 4, R>(ice_tab, ti, b, 2);
               } else {
-                apply_table_ice_rec<2, 4, R>(ice_tab, ti, a, 0);
-                apply_table_ice_rec<2, 4, R>(ice_tab, ti, b, 2);
+                apply_table_ice_rec<2, STRIDE, R>(ice_tab, ti, a, 0);
+                apply_table_ice_rec<2, STRIDE, R>(ice_tab, ti, b, 2);
               }
               v[0] = a[0]; v[1] = a[1]; v[2] = b[0]; v[3] = b[1];
             }
@@ -377,10 +386,10 @@ struct SedRun {
 // One species' run over the group's column, whole: load, the substeps (the
 // first peeled off the loop, so that neither carries the other's branch),
 // store.  prt (every lane) is the mass that left through the surface.
-template <int SP, class R, int LPC, int L, bool DIF>
+template <int SP, class R, int LPC, int L, bool DIF, int STRIDE>
 __device__ __forceinline__ void sediment_run(const KParams& p, int i, int j, int k_top, double& prt,
                                           int& nsub_out, unsigned& err, const R* __restrict__ ice_tab) {
-  SedRun<SP, R, LPC, L, DIF> r;
+  SedRun<SP, R, LPC, L, DIF, STRIDE> r;
   r.load(p, i, j, k_top);
   if (r.dt_left > dt_left_tol) r.substep(p, j, true, ice_tab);
 #pragma unroll 1
@@ -444,9 +453,10 @@ __device__ __forceinline__ void sediment(const KParams& p, int i, int j, int k_t
   if (k_top >= nlev) return;
   // the ice records' layout is the one the kernel staged for its own L
   constexpr bool dif = ice_rec_dif<R, L>();
-  if (lw <= 1) sediment_run<SP, R, LPC, 1, dif>(p, i, j, k_top, prt, nsub_out, err, ice_tab);
-  else if (L > 2 && lw <= 2) sediment_run<SP, R, LPC, (L > 2 ? 2 : L), dif>(p, i, j, k_top, prt, nsub_out, err, ice_tab);
-  else sediment_run<SP, R, LPC, L, dif>(p, i, j, k_top, prt, nsub_out, err, ice_tab);
+  constexpr int str = ice_lds_stride<R, L>();
+  if (lw <= 1) sediment_run<SP, R, LPC, 1, dif, str>(p, i, j, k_top, prt, nsub_out, err, ice_tab);
+  else if (L > 2 && lw <= 2) sediment_run<SP, R, LPC, (L > 2 ? 2 : L), dif, str>(p, i, j, k_top, prt, nsub_out, err, ice_tab);
+  else sediment_run<SP, R, LPC, L, dif, str>(p, i, j, k_top, prt, nsub_out, err, ice_tab);
 }
 
 // homogeneous_freezing (P3I/p3_ice_sed_impl.hpp:207-270) + p3_main_part3
@@ -762,12 +772,11 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
 
 // Copies the ice-sedimentation records into the block's LDS copy (16-byte
 // chunks), then waits for the whole block.
-template <class R, int LEN>
+template <class R, int L>
 __device__ __forceinline__ void stage_ice_table(const R* __restrict__ g, R* s) {
-  constexpr int n = LEN * (int)sizeof(R) / 16;
-  static_assert(LEN * sizeof(R) % 16 == 0, "16-byte chunks");
-  for (int c = threadIdx.x; c < n; c += blockDim.x)
-    reinterpret_cast<uint4*>(s)[c] = reinterpret_cast<const uint4*>(g)[c];
+  constexpr int per = ice_rec_len<R, L>() * (int)sizeof(R) / 16, str = ice_lds_stride<R, L>() * (int)sizeof(R) / 16;
+  for (int c = threadIdx.x; c < kIceCells * per; c += blockDim.x)
+    reinterpret_cast<uint4*>(s)[c / per * str + c % per] = reinterpret_cast<const uint4*>(g)[c];
   __syncthreads();
 }
 
@@ -786,7 +795,7 @@ __global__ __launch_bounds__(64 * WPB, (sed_waves_per_simd<R, G, L>())) void p3_
   if constexpr (G == SED_ICE) {
     static_assert(WPB == 4 || !ice_rec_dif<R, L>(), "the LDS budget assumes blocks of 4 wavefronts");
     __shared__ __align__(16) R s_tab[ice_lds_len<R, L>()];
-    stage_ice_table<R, ice_lds_len<R, L>()>(ice_lds_source<R, L>(p), s_tab);
+    stage_ice_table<R, L>(ice_lds_source<R, L>(p), s_tab);
     sed_block<R, LPC, L, WPB, G>(p, xcd_block(blockIdx.x, gridDim.x), s_tab);
   } else {
     sed_block<R, LPC, L, WPB, G>(p, xcd_block(blockIdx.x, gridDim.x), nullptr);
@@ -814,7 +823,7 @@ __global__ __launch_bounds__(64 * WPB, (sed_waves_per_simd<R, SED_ICE, L>())) vo
   __shared__ __align__(16) R s_tab[ice_lds_len<R, L>()];
   const int b = blockIdx.x;  // uniform over the block: the whole block takes one branch
   if (b < nb_ice) {
-    stage_ice_table<R, ice_lds_len<R, L>()>(ice_lds_source<R, L>(p), s_tab);
+    stage_ice_table<R, L>(ice_lds_source<R, L>(p), s_tab);
     sed_block<R, LPC, L, WPB, SED_ICE>(p, xcd_block(b, nb_ice), s_tab);
   } else {
     // block b runs on XCD b % 8; the liquid blocks' offset nb_ice only rotates

@@ -105,10 +105,10 @@ __global__ __launch_bounds__(64 * WPB, (sed_waves_per_simd<R, SED_ICE, L>())) vo
   const int s = find_set(first, nsets, vb);
   const KParams& p = *(const KParams*)(sets4 + s);
   if (b < nb) {
-    stage_ice_table<R, L>(ice_lds_source<R, L>(p), s_tab);
-    sed_block<R, LPC, L, WPB, SED_ICE>(p, vb - first[s], s_tab);
+    const IceTableStage<R, L, 64 * WPB> stage(ice_lds_source<R, L>(p), s_tab);
+    sed_block<R, LPC, L, WPB, SED_ICE>(p, vb - first[s], s_tab, stage);
   } else {
-    sed_block<R, LPC, L, WPB, SED_LIQ>(p, vb - first[s], nullptr);
+    sed_block<R, LPC, L, WPB, SED_LIQ>(p, vb - first[s], nullptr, NoStage{});
   }
 }
 
@@ -124,15 +124,16 @@ __global__ __launch_bounds__(64 * WPB, (sed_waves_per_simd<R, G, L>())) void p3_
     static_assert(WPB == 4 || !ice_rec_dif<R, L>(), "the LDS budget assumes blocks of 4 wavefronts");
     __shared__ __align__(16) R s_tab[ice_lds_len<R, L>()];
     if ((int)blockIdx.x >= total) return;  // the whole block leaves before the barrier
-    stage_ice_table<R, L>(ice_lds_source<R, L>(*(const KParams*)sets4), s_tab);
+    const IceTableStage<R, L, 64 * WPB> stage(ice_lds_source<R, L>(*(const KParams*)sets4), s_tab);
+    stage();
     for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {
       const int s = find_set(first, nsets, vb);
-      sed_block<R, LPC, L, WPB, G>(*(const KParams*)(sets4 + s), vb - first[s], s_tab);
+      sed_block<R, LPC, L, WPB, G>(*(const KParams*)(sets4 + s), vb - first[s], s_tab, NoStage{});
     }
   } else {
     for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {
       const int s = find_set(first, nsets, vb);
-      sed_block<R, LPC, L, WPB, G>(*(const KParams*)(sets4 + s), vb - first[s], nullptr);
+      sed_block<R, LPC, L, WPB, G>(*(const KParams*)(sets4 + s), vb - first[s], nullptr, NoStage{});
     }
   }
 }

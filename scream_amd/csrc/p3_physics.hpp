@@ -241,6 +241,17 @@ __device__ __forceinline__ void load_rec(const float* __restrict__ r, float (&v)
   }
 }
 
+// The record of the point's cell in a table of NR values per (density, rime,
+// size) cell.  The point's other corners lie at constant offsets from it, which
+// the load instructions take: one address, by a full-rate 24-bit multiplication
+// (a 32-bit one takes four times as long, and one per corner is what the
+// compiler makes of corner indices).
+template <int NR, class R>
+__device__ __forceinline__ const R* ice_record(const R* __restrict__ tab, const TabIce<R>& t) {
+  const unsigned cell = (t.dumjj * rimsize + t.dumii) * isize + t.dumi;
+  return reinterpret_cast<const R*>(reinterpret_cast<const char*>(tab) + __umul24(cell, NR * (unsigned)sizeof(R)));
+}
+
 // apply_table_ice, P3I/p3_table_ice_impl.hpp:175-217, for the NQ quantities of
 // a repacked record of NR values per (density, rime, size) cell; each value is
 // the reference's trilinear interpolation with its operation order.
@@ -251,17 +262,17 @@ __device__ __forceinline__ void apply_table_ice_rec(const R* __restrict__ tab, c
   const R w1 = (t.dum1 - R(i) - R(1));
   const R w4 = (t.dum4 - R(ii) - R(1));
   const R w5 = (t.dum5 - R(jj) - R(1));
-  // values q0 .. q0+NQ-1 of the record of cell (a, b, i)
-  auto rec = [&](int a, int b) { return tab + ((a * rimsize + b) * isize + i) * NR + q0; };
+  const R* const r = ice_record<NR>(tab, t) + q0;
+  constexpr int dr = isize * NR, dd = rimsize * isize * NR;  // the next rime fraction and density
   R c[8][NQ];
-  load_rec<NQ>(rec(jj, ii), c[0]);
-  load_rec<NQ>(rec(jj, ii) + NR, c[1]);
-  load_rec<NQ>(rec(jj, ii + 1), c[2]);
-  load_rec<NQ>(rec(jj, ii + 1) + NR, c[3]);
-  load_rec<NQ>(rec(jj + 1, ii), c[4]);
-  load_rec<NQ>(rec(jj + 1, ii) + NR, c[5]);
-  load_rec<NQ>(rec(jj + 1, ii + 1), c[6]);
-  load_rec<NQ>(rec(jj + 1, ii + 1) + NR, c[7]);
+  load_rec<NQ>(r, c[0]);
+  load_rec<NQ>(r + NR, c[1]);
+  load_rec<NQ>(r + dr, c[2]);
+  load_rec<NQ>(r + dr + NR, c[3]);
+  load_rec<NQ>(r + dd, c[4]);
+  load_rec<NQ>(r + dd + NR, c[5]);
+  load_rec<NQ>(r + dd + dr, c[6]);
+  load_rec<NQ>(r + dd + dr + NR, c[7]);
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
     R iproc1 = c[0][q] + w1 * (c[1][q] - c[0][q]);
@@ -287,16 +298,17 @@ __device__ __forceinline__ void apply_table_ice_dif(const R* __restrict__ tab, c
   const R w1 = (t.dum1 - R(i) - R(1));
   const R w4 = (t.dum4 - R(ii) - R(1));
   const R w5 = (t.dum5 - R(jj) - R(1));
-  auto rec = [&](int a, int b) { return tab + ((a * rimsize + b) * isize + i) * NR + q0; };
+  const R* const r = ice_record<NR>(tab, t) + q0;
+  constexpr int dr = isize * NR, dd = rimsize * isize * NR;  // the next rime fraction and density
   R c[4][NQ], d[4][NQ];
-  load_rec<NQ>(rec(jj, ii), c[0]);
-  load_rec<NQ>(rec(jj, ii) + DOFF, d[0]);
-  load_rec<NQ>(rec(jj, ii + 1), c[1]);
-  load_rec<NQ>(rec(jj, ii + 1) + DOFF, d[1]);
-  load_rec<NQ>(rec(jj + 1, ii), c[2]);
-  load_rec<NQ>(rec(jj + 1, ii) + DOFF, d[2]);
-  load_rec<NQ>(rec(jj + 1, ii + 1), c[3]);
-  load_rec<NQ>(rec(jj + 1, ii + 1) + DOFF, d[3]);
+  load_rec<NQ>(r, c[0]);
+  load_rec<NQ>(r + DOFF, d[0]);
+  load_rec<NQ>(r + dr, c[1]);
+  load_rec<NQ>(r + dr + DOFF, d[1]);
+  load_rec<NQ>(r + dd, c[2]);
+  load_rec<NQ>(r + dd + DOFF, d[2]);
+  load_rec<NQ>(r + dd + dr, c[3]);
+  load_rec<NQ>(r + dd + dr + DOFF, d[3]);
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
     R iproc1 = c[0][q] + w1 * d[0][q];

@@ -23,51 +23,61 @@
 
 namespace p3d {
 
-// Reductions over aligned groups of LPC lanes, all lanes getting the result.
-// Step o combines each lane with a lane of the other half of its 2o-lane
-// block; before the step both halves are uniform, so any pairing of the halves
-// does: inside a 16-lane row by DPP (o = 1, 2: quad permutes; 4, 8: the
-// half-row and row mirrors), across rows by ds_swizzle (o = 16, xor inside 32
-// lanes) and across the wavefront's halves by ds_bpermute (o = 32).  A lane
-// reads only lanes of its own group, and every lane of a group must be active
-// (a DPP read from an inactive lane returns the reader's own value): the
-// sedimentation code calls these with whole groups, never with part of one.
+// Reductions over aligned groups of LPC lanes, all lanes getting the result,
+// entirely in the VALU.  Step o combines each lane with a lane of the other half
+// of its 2o-lane block; before the step both halves are uniform, so any pairing of
+// the halves does: inside a 16-lane row by DPP (o = 1, 2: quad permutes; 4, 8: the
+// half-row and row mirrors), across rows and across the wavefront's halves by
+// v_permlane16_swap and v_permlane32_swap, which leave the two halves' values in
+// two registers.  A lane reads only lanes of its own group, and every lane of a
+// group must be active: the sedimentation code calls these with whole groups.
+// (ds_swizzle and ds_bpermute for the last two steps cost an LDS round trip each,
+// which a column on 32 or 64 lanes waits for in every substep.)
+struct Halves { int a, b; };
 template <int O>
-__device__ __forceinline__ int partner(int v) {
-  if constexpr (O == 1) return __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false);  // quad_perm 1,0,3,2
-  else if constexpr (O == 2) return __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false);  // quad_perm 2,3,0,1
-  else if constexpr (O == 4) return __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false);  // row_half_mirror
-  else if constexpr (O == 8) return __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false);  // row_mirror
-  else if constexpr (O == 16) return __builtin_amdgcn_ds_swizzle(v, 0x401F);  // lane ^ 16 within 32
-  else return __shfl_xor(v, 32, 64);
+__device__ __forceinline__ Halves halves(int v) {
+  if constexpr (O == 1) return {v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true)};       // quad_perm:[1,0,3,2]
+  else if constexpr (O == 2) return {v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true)};  // quad_perm:[2,3,0,1]
+  else if constexpr (O == 4) return {v, __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true)};  // row_half_mirror
+  else if constexpr (O == 8) return {v, __builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, true)};  // row_mirror
+  else if constexpr (O == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return {(int)r[0], (int)r[1]};
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return {(int)r[0], (int)r[1]};
+  }
 }
 template <int O>
-__device__ __forceinline__ double partner(double v) {
-  return __hiloint2double(partner<O>(__double2hiint(v)), partner<O>(__double2loint(v)));
+__device__ __forceinline__ void halves(double v, double& a, double& b) {
+  const Halves hi = halves<O>(__double2hiint(v)), lo = halves<O>(__double2loint(v));
+  a = __hiloint2double(hi.a, lo.a);
+  b = __hiloint2double(hi.b, lo.b);
 }
 
 template <int LPC>
 __device__ __forceinline__ int grp_min(int v) {
   if constexpr (LPC > 1) {
-    v = grp_min<LPC / 2>(v);
-    v = min(v, partner<LPC / 2>(v));
+    const Halves h = halves<LPC / 2>(grp_min<LPC / 2>(v));
+    v = min(h.a, h.b);
   }
   return v;
 }
 template <int LPC>
 __device__ __forceinline__ int grp_max(int v) {
   if constexpr (LPC > 1) {
-    v = grp_max<LPC / 2>(v);
-    v = max(v, partner<LPC / 2>(v));
+    const Halves h = halves<LPC / 2>(grp_max<LPC / 2>(v));
+    v = max(h.a, h.b);
   }
   return v;
 }
+// (of values that are not NaN)
 template <int LPC>
 __device__ __forceinline__ double grp_maxd(double v) {
   if constexpr (LPC > 1) {
-    v = grp_maxd<LPC / 2>(v);
-    const double w = partner<LPC / 2>(v);
-    v = w > v ? w : v;
+    double a, b;
+    halves<LPC / 2>(grp_maxd<LPC / 2>(v), a, b);
+    v = __builtin_fmax(a, b);
   }
   return v;
 }
@@ -76,10 +86,21 @@ __device__ __forceinline__ double grp_maxd(double v) {
 template <int LPC>
 __device__ __forceinline__ double grp_sumd(double v) {
   if constexpr (LPC > 1) {
-    v = grp_sumd<LPC / 2>(v);
-    v += partner<LPC / 2>(v);
+    double a, b;
+    halves<LPC / 2>(grp_sumd<LPC / 2>(v), a, b);
+    v = a + b;
   }
   return v;
+}
+// v of the lane below in the group, 0 in the group's first lane: a DPP shift of
+// the row (16 lanes) or of the wavefront.
+template <int LPC>
+__device__ __forceinline__ double grp_below(double v, int j) {
+  constexpr int ctrl = LPC == 16 ? 0x111 : 0x138;  // row_shr:1, wave_shr:1
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xF, 0xF, true);
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xF, 0xF, true);
+  const double w = __hiloint2double(hi, lo);
+  return LPC == 32 && j == 0 ? 0.0 : w;
 }
 
 // Sedimentation runs as two kernels over the same column blocks, one per
@@ -335,7 +356,7 @@ struct SedRun {
     // k_top, whose incoming flux is 0)
     double Fin[NF];
 #pragma unroll
-    for (int f = 0; f < NF; ++f) Fin[f] = __shfl_up(F[f][L - 1], 1, LPC);
+    for (int f = 0; f < NF; ++f) Fin[f] = grp_below<LPC>(F[f][L - 1], j);
 #pragma unroll
     for (int t = 0; t < L; ++t) {
       const int k = kbase + t;
@@ -343,8 +364,7 @@ struct SedRun {
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
           if (f < nfield) {
-            // level kbase + t is k_top exactly when t = 0 and j = 0
-            const double Fa = t == 0 ? (j == 0 ? 0.0 : Fin[f]) : F[f][t > 0 ? t - 1 : 0];
+            const double Fa = t == 0 ? Fin[f] : F[f][t > 0 ? t - 1 : 0];
             const double fluxdiv = (Fa - F[f][t]) * g.inv_dz[t];
             q[f][t] = q[f][t] + fluxdiv * dt_sub * g.inv_rho[t];
           }

@@ -66,6 +66,19 @@ __global__ __launch_bounds__(kTileThreads, kFrontWaves<R>) void p3_front_batch(c
   });
 }
 
+// The order of every set's columns: grid (nsets, y), the blocks of a column of
+// the grid sharing a set's blocks.
+template <class R>
+__global__ __launch_bounds__(kOrderThreads) void p3_order_batch(const KParams* __restrict__ sets) {
+  const auto sets4 = (const __attribute__((address_space(4))) KParams*)sets;
+  const KParams& p = *(const KParams*)(sets4 + blockIdx.x);
+  if (!p.ordered()) return;
+  for (int blk = blockIdx.y; blk * kOrderCols < p.ncol; blk += gridDim.y) {
+    order_block(p, blk);
+    __syncthreads();  // before the next block's counts
+  }
+}
+
 // Part 3 one thread per (level, column), after the sedimentation launches;
 // first: the pointwise tile offsets.
 template <class R, bool PERSIST>
@@ -76,20 +89,6 @@ __global__ __launch_bounds__(kTileThreads, kPart3Waves) void p3_part3_lvl_batch(
     const int s = find_set(first, nsets, vb);
     part3_tile<R>(*(const KParams*)(sets4 + s), vb - first[s]);
   });
-}
-
-// The virtual block that block b of nb runs, one block per virtual block: block
-// b is on XCD b % 8, so within each run of 8 * kXcdRun blocks an XCD takes
-// kXcdRun consecutive virtual blocks.  Neighbouring blocks hold parts of the same
-// 128-byte lines (4 to 16 columns each), while the runs keep the sets in order:
-// the longest steps start first (layout_batch).
-constexpr int kXcdRun = 16;
-__device__ __forceinline__ int run_block(int b, int nb) {
-  constexpr int chunk = kXcds * kXcdRun;
-  const int c0 = b / chunk * chunk;
-  if (c0 + chunk > nb) return b;
-  const int r = b - c0;
-  return c0 + r % kXcds * kXcdRun + r / kXcds;
 }
 
 // Both species groups of one class of sets in one launch, the ice blocks first

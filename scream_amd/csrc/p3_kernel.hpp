@@ -17,8 +17,9 @@ namespace p3d {
 // Scratch fields (ncol x nlev doubles each, in the layout of the column set):
 // per-level results of part 1 for sedimentation and part 3 (T, rhofacr,
 // rhofaci, acn), and the marks of part 2's pending levels (SC_PEND, only
-// without exch_zero).  Room for SC_COUNT fields is reserved.
-enum Scr { SC_T = 0, SC_RHOFACR, SC_RHOFACI, SC_ACN, SC_PEND, SC_COUNT = 7 };
+// without exch_zero).
+// SC_WET and SC_ORDER hold the words and the lists of p3_order_kernel.
+enum Scr { SC_T = 0, SC_RHOFACR, SC_RHOFACI, SC_ACN, SC_PEND, SC_WET, SC_ORDER, SC_COUNT };
 
 // The P3Microphysics pre- and post-amble (eamxx_p3_process_interface.hpp:63-261),
 // fused into part 1 and part 3 when `on`.  The prognostic pointers then hold the
@@ -68,6 +69,7 @@ struct KParams {
   int dbg_stride;       // species stride of dbg_substeps (>= ncol)
   double dt;
   int predictNc, prescribedCCN, exch_zero;
+  int keep_order;       // sedimentation takes the columns as they come (order())
   double e_melt;        // saturation vapour pressure over liquid at Tmelt (qv_sat_dry(Tmelt, p) numerator)
   Amble amble;
 
@@ -75,6 +77,25 @@ struct KParams {
   // check_values (fully stepped columns only), or for exchange fields that a
   // skipped column leaves as they were.
   __host__ __device__ __forceinline__ bool track() const { return dbg_status || dbg_check || !exch_zero; }
+  // Sedimentation with several columns per wavefront takes them in the order of
+  // p3_order_kernel.  Not with the status words (a skipped column may hold
+  // species), and only where the words and lists fit their scratch fields and the
+  // counts their 21 bits each.
+  __host__ __device__ __forceinline__ bool ordered() const {
+    return !keep_order && !track() && ncol >= 64 && ncol < 1 << 21 && nlev >= 16;
+  }
+  // The words: a bit per column, 8 bytes per 64 columns, a row per level, for
+  // cloud, rain and ice.
+  __host__ __device__ __forceinline__ int wet_words() const { return (ncol + 63) / 64; }
+  __device__ __forceinline__ unsigned long long* wet(int species) const {
+    return (unsigned long long*)(scratch + SC_WET * sfs) + (size_t)species * nlev * wet_words();
+  }
+  // The counts of the blocks that have appended so far (21 bits each: columns, of
+  // them with cloud or rain, with ice), and each group's list.
+  __device__ __forceinline__ unsigned long long* order_count() const {
+    return (unsigned long long*)(scratch + SC_ORDER * sfs);
+  }
+  __device__ __forceinline__ uint2* order(int group) const { return (uint2*)(order_count() + 1) + (size_t)group * ncol; }
   __host__ __device__ __forceinline__ size_t at(int i, int k) const { return (size_t)i * cs + (size_t)k * ks; }
   __host__ __device__ __forceinline__ size_t atf(int i, int k) const { return (size_t)i * fcs + (size_t)k * fks; }
   __host__ __device__ __forceinline__ double& sc(int f, int i, int k) const {
@@ -94,6 +115,10 @@ __device__ __forceinline__ double air_density(double dpres, double dz) {
 constexpr int kMaxSubsteps = 100000;
 // Column status bits: part 1 found work, part 2 left hydrometeors.
 constexpr int kStatusPart1 = 1, kStatusPart2 = 2, kStatusFull = 3;
+// What front_level leaves to sediment at its level: cloud, and the next bits rain and ice.
+constexpr int kWet = 4;
+// Species groups of the sedimentation and of its lists of columns.
+enum SedGroup { SED_LIQ = 0, SED_ICE = 1 };
 
 template <class R> struct RainOf {
   static __device__ __forceinline__ const RainGamma& get(const KParams& p) { return sizeof(R) == 8 ? p.rg : p.rgf; }
@@ -315,6 +340,9 @@ __device__ __forceinline__ void front_level(const KParams& p, int k, int i, cons
 #pragma unroll
   for (int q = 0; q < 10; ++q)
     if (chg >> q & 1) f[q][x] = st[q];
+#pragma unroll
+  for (int sp = 0; sp < 3; ++sp)
+    if (st[2 * sp] >= QSMALL) stat |= kWet << sp;
 }
 
 // Tiles of the pointwise kernels (part 1, part 2, part 3): 256 threads, one
@@ -398,6 +426,128 @@ __device__ __forceinline__ void colstat_or(const KParams& p, int i, int k, bool 
   if (set && !(m & run_below)) atomicOr(&p.colstat[i], bit);
 }
 
+// Stores where the points of pw_point<PW_BLOCKS> hold species sp, from the ballot
+// m of the wavefront's lanes; (i, k) is this lane's point.
+__device__ __forceinline__ void put_wet(const KParams& p, int sp, int i, int k, unsigned long long m) {
+  unsigned long long* const w = p.wet(sp);
+  const int lane = threadIdx.x & 63;
+  if (!p.colmajor) {
+    if (lane == 0) w[(size_t)k * p.wet_words() + i / 64] = m;
+    return;
+  }
+  // a byte per column, a bit per level: transposed, and a byte per level from the
+  // first column's lanes
+  unsigned long long t = (m ^ m >> 7) & 0x00aa00aa00aa00aaull;
+  m ^= t ^ t << 7;
+  t = (m ^ m >> 14) & 0x0000cccc0000ccccull;
+  m ^= t ^ t << 14;
+  t = (m ^ m >> 28) & 0x00000000f0f0f0f0ull;
+  m ^= t ^ t << 28;
+  if (lane < 8) ((unsigned char*)w)[(size_t)k * p.wet_words() * 8 + i / 8] = (unsigned char)(m >> 8 * lane);
+}
+
+// Orders the columns of a step for each sedimentation group, those with the
+// group's species first and the others behind them, and finds the top levels of
+// their species: entry {column, top levels of the group's first and second species
+// in 16 bits each (nlev: none)}.  A wavefront that sediments several columns lasts
+// as long as its longest; with clear columns spread among the wet ones nearly every
+// wavefront carries idle lanes.  The blocks append in the order in which they
+// arrive: the lists differ from run to run, the results do not.
+//
+// Bound by latency (one round of loads, one atomic): block blk of the set takes the
+// columns [blk * kOrderCols, + kOrderCols), stages kOrderRows levels of their words
+// in LDS at a time and searches them in groups of 8 levels, then within the group.
+// With a loop over the levels' words in global memory instead it took 16 and 26 us
+// at 21600 x 72 and 16384 x 128, now 6 and 6.  Sedimentation itself, which no longer
+// searches for the top levels: 21600 x 72 mixed dt 1800, a third of the columns clear,
+// 267 -> 208 us; 16384 x 128 mixed dt 100, none clear, 158 -> 138.
+constexpr int kOrderCols = 512, kOrderRows = 128, kOrderThreads = 1024;
+__device__ __forceinline__ void order_block(const KParams& p, int blk) {
+  constexpr int kWords = kOrderCols / 64, kGroups = kOrderRows / 8;
+  static_assert(kWords * kOrderRows == kOrderThreads && 3 * kGroups * kWords <= kOrderThreads, "one word per thread");
+  __shared__ unsigned long long s_row[3][kOrderRows][kWords], s_grp[3][kGroups][kWords];
+  __shared__ int s_n[2][kWords];
+  __shared__ unsigned long long s_at;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nw = p.wet_words(), nlev = p.nlev;
+  const bool lists = threadIdx.x < kOrderCols;  // whole wavefronts, one thread per column
+  const int i = blk * kOrderCols + threadIdx.x;
+  int top[3] = {nlev, nlev, nlev};
+  for (int k0 = 0; k0 < nlev; k0 += kOrderRows) {
+    const int row = threadIdx.x / kWords, q = threadIdx.x % kWords, w = blk * kWords + q, k = k0 + row;
+#pragma unroll
+    for (int sp = 0; sp < 3; ++sp) s_row[sp][row][q] = k < nlev && w < nw ? p.wet(sp)[(size_t)k * nw + w] : 0;
+    __syncthreads();
+    if (threadIdx.x < 3 * kGroups * kWords) {
+      const int sp = threadIdx.x / (kGroups * kWords), g = threadIdx.x / kWords % kGroups;
+      unsigned long long any = 0;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) any |= s_row[sp][g * 8 + r][q];
+      s_grp[sp][g][q] = any;
+    }
+    __syncthreads();
+    if (lists) {
+      const unsigned bit = 1u << (lane & 31);
+      const int h = wave * 2 + (lane >> 5);  // the 32-bit half word of this column
+#pragma unroll
+      for (int sp = 0; sp < 3; ++sp) {
+        int g = kGroups;
+#pragma unroll
+        for (int n = kGroups - 1; n >= 0; --n)
+          if (((const unsigned*)s_grp[sp][n])[h] & bit) g = n;
+        if (top[sp] == nlev && g < kGroups) {
+          int r = 0;
+#pragma unroll
+          for (int n = 7; n >= 0; --n)
+            if (((const unsigned*)s_row[sp][g * 8 + n])[h] & bit) r = n;
+          top[sp] = k0 + g * 8 + r;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  bool wet[2] = {false, false};
+  unsigned before[2] = {0, 0};
+  if (lists) {
+    // (past the last column the words may hold anything)
+    const bool col = i < p.ncol;
+    wet[SED_LIQ] = col && (top[0] < nlev || top[1] < nlev);
+    wet[SED_ICE] = col && top[2] < nlev;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const unsigned long long m = __ballot(wet[g]);
+      before[g] = (unsigned)__popcll(m & ((1ull << lane) - 1));
+      if (lane == 0) s_n[g][wave] = __popcll(m);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int left = p.ncol - blk * kOrderCols;
+    unsigned long long n = (unsigned long long)(left < kOrderCols ? left : kOrderCols);
+    for (int v = 0; v < kWords; ++v)
+      n += (unsigned long long)s_n[SED_LIQ][v] << 21 | (unsigned long long)s_n[SED_ICE][v] << 42;
+    s_at = atomicAdd(p.order_count(), n);
+  }
+  __syncthreads();
+  if (lists && i < p.ncol) {
+    const unsigned mask = (1u << 21) - 1;
+    const unsigned cols = (unsigned)s_at & mask;  // columns of the blocks before
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const unsigned base = (unsigned)(s_at >> 21 * (g + 1)) & mask;  // of them wet
+      for (int v = 0; v < wave; ++v) before[g] += (unsigned)s_n[g][v];
+      const unsigned at =
+          wet[g] ? base + before[g] : (unsigned)p.ncol - 1 - (cols - base + threadIdx.x - before[g]);
+      p.order(g)[at] = make_uint2((unsigned)i, g == SED_ICE ? (unsigned)top[2] : (unsigned)(top[0] | top[1] << 16));
+    }
+  }
+}
+
+template <class R>
+__global__ __launch_bounds__(kOrderThreads) void p3_order_kernel(const KParams p) {
+  order_block(p, blockIdx.x);
+}
+
 // Zeroes the column status words before p3_front_kernel (templated only so
 // that each precision's translation unit has its own copy).
 template <class R>
@@ -418,6 +568,11 @@ __device__ __forceinline__ void front_tile(const KParams& p, int tile, double* s
     colstat_or<PW_BLOCKS>(p, i, k, (stat & kStatusPart1) != 0, kStatusPart1);
     colstat_or<PW_BLOCKS>(p, i, k, (stat & kStatusPart2) != 0, kStatusPart2);
     if (k == 0 && p.dbg_check) p.dbg_check[i] = 0;  // part 3 ORs the column's check_values flags
+  }
+  if (p.ordered()) {
+#pragma unroll
+    for (int sp = 0; sp < 3; ++sp) put_wet(p, sp, i, k, __ballot((stat & kWet << sp) != 0));
+    if (tile == 0 && threadIdx.x == 0) *p.order_count() = 0;
   }
   if (err) atomicOr(p.err, err);
 }

@@ -76,6 +76,8 @@ struct BatchPlan {
   const KParams* sets;  // device array, all sets (pointwise launches)
   const int* first;     // device array, nsets + 1 entries: pointwise tiles (parts 1 to 3)
   int nsets;
+  int ordered;          // some set's sedimentation takes the columns in p3_order_batch's order
+  int order_blocks;     // blocks of p3_order_batch per set
   int track;            // some set keeps its column status words (KParams::track)
   int grid;             // blocks of the pointwise launches
   int total;            // pointwise virtual blocks (first[nsets]); grid >= total: one block each, no loop

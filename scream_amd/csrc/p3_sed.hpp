@@ -108,7 +108,6 @@ __device__ __forceinline__ double grp_below(double v, int j) {
 // the liquid surface precipitation) and the ice group.  The groups touch
 // disjoint state fields, so their order does not change a bit; apart, each
 // kernel holds only its own group's registers and field pointers.
-enum SedGroup { SED_LIQ = 0, SED_ICE = 1 };
 
 // Wavefronts per SIMD the sedimentation kernels are compiled for: up to 5
 // levels per lane two fit (256 registers); the FP64 ice group at up to 3
@@ -665,7 +664,13 @@ __device__ __forceinline__ void sed_wave(const KParams& p, int col0, const R* __
   static_assert(64 % LPC == 0, "a column group must divide the wavefront");
   const int lane = threadIdx.x & 63;
   const int j = lane % LPC;
-  const int i = col0 + lane / LPC;
+  // the column, in p3_order_kernel's order with its top levels; a position past the
+  // end is no column
+  int i = col0 + lane / LPC;
+  const bool ordered = LPC < 64 && p.ordered();
+  uint2 entry = make_uint2((unsigned)i, (unsigned)p.nlev << 16 | (unsigned)p.nlev);
+  if (ordered && i < p.ncol) entry = p.order(G)[i];
+  i = (int)entry.x;
   const int nlev = p.nlev, kbot = nlev - 1;
   const int kbase = j * L;
   unsigned err = 0;
@@ -683,7 +688,8 @@ __device__ __forceinline__ void sed_wave(const KParams& p, int col0, const R* __
   if constexpr (G == SED_LIQ) {
     double prt_c, prt_r;
     int ns_c, ns_r, top[2];
-    find_tops<LPC, L, 2>(p, i, j, run, {p.qc, p.qr}, top);
+    if (ordered) top[0] = (int)(entry.y & 0xffff), top[1] = (int)(entry.y >> 16);
+    else find_tops<LPC, L, 2>(p, i, j, run, {p.qc, p.qr}, top);
     const int top_c = top[0], top_r = top[1];
     sediment<0, R, LPC, L>(p, i, j, top_c, prt_c, ns_c, err);
     sediment<1, R, LPC, L>(p, i, j, top_r, prt_r, ns_r, err);
@@ -717,7 +723,8 @@ __device__ __forceinline__ void sed_wave(const KParams& p, int col0, const R* __
   } else {
     double prt_i;
     int ns_i, top[1];
-    find_tops<LPC, L, 1>(p, i, j, run, {p.qi}, top);
+    if (ordered) top[0] = (int)(entry.y & 0xffff);
+    else find_tops<LPC, L, 1>(p, i, j, run, {p.qi}, top);
     staged();
     const int top_i = top[0];
     sediment<2, R, LPC, L>(p, i, j, top_i, prt_i, ns_i, err, ice_tab);
@@ -793,6 +800,23 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
   return x * q + (x < r ? x : r) + n;
 }
 
+// The same in runs of kXcdRun blocks per XCD: within each 8 * kXcdRun blocks an
+// XCD takes kXcdRun consecutive ones.  For blocks whose work changes along the
+// grid: the longest steps first (layout_batch), or the clear columns last
+// (p3_order_kernel), which a contiguous range would give to the last XCDs alone.
+constexpr int kXcdRun = 16;
+__device__ __forceinline__ int run_block(int b, int nb) {
+  constexpr int chunk = kXcds * kXcdRun;
+  const int c0 = b / chunk * chunk;
+  if (c0 + chunk > nb) return b;
+  const int r = b - c0;
+  return c0 + r % kXcds * kXcdRun + r / kXcds;
+}
+template <int LPC>
+__device__ __forceinline__ int sed_order_block(const KParams& p, int b, int nb) {
+  return LPC < 64 && p.ordered() ? run_block(b, nb) : xcd_block(b, nb);
+}
+
 // Copies the ice-sedimentation records into the block's LDS copy, in 16-byte
 // chunks by the NT threads of the block: requested when the object is made, written
 // (and waited for by the whole block) by the call, so that the request travels
@@ -842,9 +866,9 @@ __global__ __launch_bounds__(64 * WPB, (sed_waves_per_simd<R, G, L>())) void p3_
     static_assert(WPB == 4 || !ice_rec_dif<R, L>(), "the LDS budget assumes blocks of 4 wavefronts");
     __shared__ __align__(16) R s_tab[ice_lds_len<R, L>()];
     const IceTableStage<R, L, 64 * WPB> stage(ice_lds_source<R, L>(p), s_tab);
-    sed_block<R, LPC, L, WPB, G>(p, xcd_block(blockIdx.x, gridDim.x), s_tab, stage);
+    sed_block<R, LPC, L, WPB, G>(p, sed_order_block<LPC>(p, blockIdx.x, gridDim.x), s_tab, stage);
   } else {
-    sed_block<R, LPC, L, WPB, G>(p, xcd_block(blockIdx.x, gridDim.x), nullptr, NoStage{});
+    sed_block<R, LPC, L, WPB, G>(p, sed_order_block<LPC>(p, blockIdx.x, gridDim.x), nullptr, NoStage{});
   }
 }
 
@@ -870,11 +894,11 @@ __global__ __launch_bounds__(64 * WPB, (sed_waves_per_simd<R, SED_ICE, L>())) vo
   const int b = blockIdx.x;  // uniform over the block: the whole block takes one branch
   if (b < nb_ice) {
     const IceTableStage<R, L, 64 * WPB> stage(ice_lds_source<R, L>(p), s_tab);
-    sed_block<R, LPC, L, WPB, SED_ICE>(p, xcd_block(b, nb_ice), s_tab, stage);
+    sed_block<R, LPC, L, WPB, SED_ICE>(p, sed_order_block<LPC>(p, b, nb_ice), s_tab, stage);
   } else {
     // block b runs on XCD b % 8; the liquid blocks' offset nb_ice only rotates
     // which XCD receives which contiguous range of column blocks
-    sed_block<R, LPC, L, WPB, SED_LIQ>(p, xcd_block(b - nb_ice, (int)gridDim.x - nb_ice), nullptr, NoStage{});
+    sed_block<R, LPC, L, WPB, SED_LIQ>(p, sed_order_block<LPC>(p, b - nb_ice, (int)gridDim.x - nb_ice), nullptr, NoStage{});
   }
 }
 

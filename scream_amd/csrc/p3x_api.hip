@@ -79,36 +79,43 @@ int status_of_err(unsigned err) {
   return err ? P3X_ERR_DEVICE : P3X_OK;
 }
 
-// Default sedimentation lanes per column of a step over ncol columns of nk levels.
+// Default sedimentation lanes per column of a step of dt seconds over ncol columns
+// of nk levels, by what was measured (us a step at 16 / 32 / 64 lanes, half of them
+// without and half with a third of the columns clear, which p3_order_kernel packs).
 //
-// Few columns (their wavefronts at 64 lanes, one per column, all fit the chip at
-// two per SIMD: 2048): a wavefront's time is its chain of level bodies per
-// substep, so the fewest levels per lane are the fastest.  Sedimentation and part
-// 3, us, at 16 / 32 / 64 lanes:
-//   FP64   72 levels, dt 1800: 256 columns 146 / 118 / 71, 2048 161 / 129 / 115,
-//                              3072 171 / 176 / 164, 4096 171 / 177 / 198
-//   FP64  128 levels, dt 100:  256 columns  62 /  38 / 27, 2048  81 /  56 /  57
-//   mixed  72 levels, dt 1800: 256 columns  99 /  67 / 52, 2048 108 /  76 /  75
-// More columns than that: the lanes that waste the fewest level slots and leave
-// two wavefronts per SIMD their registers (at most 5 levels per lane), per
-// species group (kernel trace, us):
-//                     liquid 16 / 32 / 64     ice 16 / 32 / 64
-//   FP64  21600 x 72     115 / 184 / 247     766 / 767 / 891
-//   FP64  16384 x 128    111 /  77 / 105     284 / 184 / 171
-//   mixed 21600 x 72      63 /  84 / 121     412 / 363 / 427
-//   mixed 16384 x 128     51 /  49 /  60     131 / 122 / 133
-// (FP64 ice at up to 80 levels: 16 lanes, 1143 against 1159 us a step at 32; the
-// mixed ice group up to 48 levels: 16 lanes, 20000 x 48 118 us against 140 with
-// ice on 32.)
-constexpr int kFewColumns = 2048;
-void default_shape(int precision, int nk, long long ncol, p3d::Shape* sh) {
-  if (ncol <= kFewColumns) {
-    sh->lpc = sh->lpc_ice = 64;
-    return;
-  }
-  sh->lpc = nk <= 80 ? 16 : (nk <= 32 * 5 ? 32 : 64);
-  if (precision == P3X_MIXED) sh->lpc_ice = nk <= 48 ? 16 : (nk <= 32 * 5 ? 32 : 64);
-  else sh->lpc_ice = nk <= 80 ? 16 : (nk <= 96 ? 32 : 64);
+// Few columns: one per wavefront and the fewest levels per lane, since a
+// wavefront's time is its chain of level bodies per substep.  Up to 2.5 wavefronts
+// per SIMD, and in the mixed form above 80 levels, where 32 lanes hold 4 levels, 4:
+//   FP64  2100 x 72 dt 300    111 / 123 / 106, clear 110 / 111 / 103
+//   FP64  3400 x 72 dt 300    122 / 138 / 132, clear 121 / 133 / 127
+//   mixed 2100 x 72 dt 1800   140 / 127 / 119, clear 143 / 113 / 116
+//   mixed 3400 x 72 dt 1800   153 / 145 / 152, clear 154 / 145 / 148
+//   mixed 2700 x 128 dt 300   152 / 137 / 122, clear 153 / 123 / 119
+// More: the lanes that waste the fewest level slots and leave two wavefronts per
+// SIMD their registers (at most 5 levels per lane):
+//   FP64  21600 x 72 dt 1800  815 / 984 / 1123, clear 661 / 771 / 1015
+//   FP64  12000 x 90 dt 300   465 / 388 / 422, clear 394 / 346 / 399
+//   FP64  12000 x 150 dt 300    - / 702 / 788, clear - / 608 / 729
+//   mixed 12000 x 50 dt 300   154 / 155 / 160, clear 144 / 145 / 154
+//   mixed 21600 x 72 dt 1800  528 / 572 / 707, clear 457 / 475 / 625
+//   mixed 16384 x 128 dt 300  574 / 533 / 545, clear 540 / 499 / 532
+// but between the two, while 16 lanes leave SIMDs without a wavefront, 32: in the
+// mixed form, and in FP64 where long steps give the groups many substeps:
+//   FP64  2700 x 72 dt 1800   196 / 198 / 190, clear 196 / 158 / 186
+//   FP64  2700 x 72 dt 300    114 / 126 / 116, clear 113 / 115 / 112
+//   mixed 5400 x 72 dt 1800   206 / 183 / 208, clear 173 / 165 / 192
+//   mixed 10000 x 72 dt 1800  291 / 291 / 345, clear 255 / 253 / 311
+// FP64 from 97 to 128 levels runs the groups apart, the ice on 64 lanes (2 levels,
+// three wavefronts per SIMD) and the liquid on 32: 16384 x 128 dt 300 734, against
+// 768 with both on 32 (712 and 682 with a third of the columns clear).
+constexpr int kFewColumns = 2560;
+void default_shape(int precision, int nk, long long ncol, double dt, p3d::Shape* sh) {
+  const bool mixed = precision == P3X_MIXED;
+  int l = nk <= 80 ? 16 : (nk <= 32 * 5 ? 32 : 64);
+  if (ncol <= (mixed && nk > 80 ? 4096 : kFewColumns)) l = 64;
+  else if (l == 16 && (mixed ? nk > 48 && ncol <= 8192 : ncol <= 3072 && dt * nk >= 600. * 72)) l = 32;
+  sh->lpc = sh->lpc_ice = l;
+  if (!mixed && l == 32 && nk > 96 && nk <= 128) sh->lpc_ice = 64;
 }
 
 // Offsets (in elements) of the tables in one device allocation; each is a
@@ -461,7 +468,7 @@ int p3x_detail::main_impl(p3x_context* c, const p3x_runtime* runtime, const p3x_
     const int st = check_options(nk, o.columns_per_block, o.threads_per_block, o.sed_lanes_per_column,
                                  o.part12_waves_per_simd);
     if (st != P3X_OK) return st;
-    default_shape(o.precision, nk, nj, &sh);
+    default_shape(o.precision, nk, nj, infra->dt, &sh);
     if (o.sed_lanes_per_column != 0) sh.lpc = sh.lpc_ice = o.sed_lanes_per_column;
   }
   hipStream_t s = (hipStream_t)o.stream;
@@ -543,9 +550,9 @@ int check_options(int nk_max, int cb, int nt, int lpc, int wpe) {
 
 // Lanes per column of one set of a batch of ncol columns altogether: both groups
 // on the lanes of the group that takes longer, the ice group.
-int batch_lanes(int precision, int nk, long long ncol) {
+int batch_lanes(int precision, int nk, long long ncol, double dt) {
   p3d::Shape sh;
-  default_shape(precision, nk, ncol, &sh);
+  default_shape(precision, nk, ncol, dt, &sh);
   return sh.lpc_ice;
 }
 
@@ -553,6 +560,8 @@ int layout_batch(const p3d::KParams* sets, int n, int precision, int lpc, Layout
   Layout& L = *out;
   L.first.assign(n + 1, 0);
   L.track = 0;
+  L.ordered = 0;
+  L.order_blocks = 1;
   long long ncol = 0;
   for (int i = 0; i < n; ++i) {
     L.first[i + 1] = L.first[i] + p3d::pw_tiles(sets[i]);
@@ -562,9 +571,13 @@ int layout_batch(const p3d::KParams* sets, int n, int precision, int lpc, Layout
   // class of a set: its lanes per column and levels per lane
   std::vector<std::pair<int, int>> cls_of(n);
   for (int i = 0; i < n; ++i) {
-    const int l = lpc != 0 ? lpc : batch_lanes(precision, sets[i].nlev, ncol);
+    const int l = lpc != 0 ? lpc : batch_lanes(precision, sets[i].nlev, ncol, sets[i].dt);
     cls_of[i] = {l, p3d::sed_levels_per_lane(sets[i].nlev, l)};
     if (cls_of[i].second == 0) return P3X_ERR_ARG;
+    if (l < 64 && sets[i].ordered()) {
+      L.ordered = 1;
+      L.order_blocks = std::min(64, std::max(L.order_blocks, (sets[i].ncol + p3d::kOrderCols - 1) / p3d::kOrderCols));
+    }
   }
   // the longest steps first: their blocks start first, and the class that holds
   // the longest one too, so that no long block starts when the others have ended
@@ -699,6 +712,8 @@ int build_plan(p3x_batch* b) {
   b->plan.first = b->d_first;
   b->plan.nsets = n;
   b->plan.track = lay.track;
+  b->plan.ordered = lay.ordered;
+  b->plan.order_blocks = lay.order_blocks;
   b->plan.nclass = (int)lay.cls.size();
   for (int ci = 0; ci < b->plan.nclass; ++ci) {
     const Layout::Cls& lc = lay.cls[ci];

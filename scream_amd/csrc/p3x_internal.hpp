@@ -41,8 +41,8 @@ namespace p3x_detail {
 int dev_fail(hipError_t e);
 // The P3X status of a nonzero device error word.
 int status_of_err(unsigned err);
-// Default launch shape of a step over ncol columns of nk levels.
-void default_shape(int precision, int nk, long long ncol, p3d::Shape* sh);
+// Default launch shape of a step of dt seconds over ncol columns of nk levels.
+void default_shape(int precision, int nk, long long ncol, double dt, p3d::Shape* sh);
 // Grows the context's scratch to at least need bytes (P3X_OK or an error status).
 int grow_scratch(p3x_context* c, size_t need);
 // Layout strides of a column set in k (P3X_ERR_ARG for an invalid layout or stride).
@@ -102,6 +102,8 @@ int check_options(int nk_max, int cb, int nt, int lpc, int wpe);
 struct Layout {
   std::vector<int> first;      // pointwise tile offsets, nsets + 1
   int track;                   // some set keeps its column status words
+  int ordered;                 // some set's sedimentation takes its columns in p3_order_batch's order
+  int order_blocks;            // blocks of p3_order_batch per set
   std::vector<int> sed_order;  // set indices grouped by sedimentation class, the longest steps first
   std::vector<int> sed_first;  // per class nsets_c + 1 offsets, classes concatenated
   struct Cls {

@@ -160,6 +160,8 @@ int launch_slot(p3x_server* srv, Slot& sl) {
   plan.grid = lay.first[n];
   plan.total = lay.first[n];
   plan.track = lay.track;
+  plan.ordered = lay.ordered;
+  plan.order_blocks = lay.order_blocks;
   plan.nclass = (int)lay.cls.size();
   for (int c = 0; c < plan.nclass; ++c) {
     const Layout::Cls& lc = lay.cls[c];

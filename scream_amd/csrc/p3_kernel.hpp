@@ -49,7 +49,7 @@ struct KParams {
   double *liq_ice_exchange, *vap_liq_exchange, *vap_ice_exchange;
   double* scratch;      // SC_COUNT fields of sfs doubles
   int* colstat;         // per column: 0 skipped after part 1, 1 after part 2, 3 full step (if track())
-  unsigned* err;        // device error word
+  unsigned* err;        // error word, in device or in pinned host memory
   int *dbg_status, *dbg_substeps, *dbg_ice_idx;
   int* dbg_check;       // per column: check_values flags (NULL = the check is off)
   Tables tab;
@@ -574,7 +574,7 @@ __device__ __forceinline__ void front_tile(const KParams& p, int tile, double* s
     for (int sp = 0; sp < 3; ++sp) put_wet(p, sp, i, k, __ballot((stat & kWet << sp) != 0));
     if (tile == 0 && threadIdx.x == 0) *p.order_count() = 0;
   }
-  if (err) atomicOr(p.err, err);
+  if (err) report_errors(p.err, err);
 }
 
 // Wavefronts per SIMD the front kernel is compiled for.  Two in FP64 (248

@@ -64,8 +64,15 @@ __device__ __forceinline__ void log_temperature(double t, double& h, double& l) 
 template <class T> __device__ __forceinline__ T vmin(T a, T b) { return a < b ? a : b; }
 template <class T> __device__ __forceinline__ T vmax(T a, T b) { return a > b ? a : b; }
 
-// Error bits reported through the device error word.
-enum : unsigned { ERR_BAD_TEMPERATURE = 1u, ERR_SUBSTEP_LIMIT = 2u, ERR_CHECK_VALUES = 4u };
+// Errors reported through the error word, one byte each: report_errors stores the
+// bytes, so the word can be in host memory, which takes no device atomic OR.
+enum : unsigned { ERR_BAD_TEMPERATURE = 1u, ERR_SUBSTEP_LIMIT = 1u << 8, ERR_CHECK_VALUES = 1u << 16 };
+__device__ __forceinline__ void report_errors(unsigned* word, unsigned err) {
+  volatile unsigned char* const b = (volatile unsigned char*)word;
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+    if (err >> 8 * q & 1) b[q] = 1;
+}
 
 // ---------------------------------------------------------------- saturation (FP64 always)
 // MurphyKoop_svp, PSH:38-77 (check_temperature, PSH:14-36, as a flag), from

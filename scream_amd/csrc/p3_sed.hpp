@@ -730,7 +730,7 @@ __device__ __forceinline__ void sed_wave(const KParams& p, int col0, const R* __
     sediment<2, R, LPC, L>(p, i, j, top_i, prt_i, ns_i, err, ice_tab);
     if (live && j == 0) ice_column_out(p, i, top_i < nlev, prt_i, ns_i);
   }
-  if (err) atomicOr(p.err, err);
+  if (err) report_errors(p.err, err);
 }
 
 // One block's work for group G: WPB wavefronts of 64/LPC columns each, the
@@ -782,7 +782,7 @@ __device__ __forceinline__ void part3_tile(const KParams& p, int tile) {
     a.ice_flux[i] = ice;
     a.heat_flux[i] = 0.0;
   }
-  if (err) atomicOr(p.err, err);
+  if (err) report_errors(p.err, err);
 }
 
 template <class R>

@@ -17,7 +17,8 @@ struct p3x_context {
   float* d_tab_f = nullptr;  // the same in FP32 for the mixed-precision form
   double* d_scratch = nullptr;
   size_t scratch_bytes = 0;
-  unsigned* d_err = nullptr;
+  unsigned* h_err = nullptr;  // the error word, in pinned host memory
+  unsigned* d_err = nullptr;  // its device address
   p3d::RainGamma rain_mixed{};  // of the mixed form, for the default constant_mu_rain
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t ev_mid = nullptr;  // between the part 1 + 2 and the sedimentation kernels
@@ -39,7 +40,7 @@ struct p3x_context {
 namespace p3x_detail {
 
 int dev_fail(hipError_t e);
-// The P3X status of a nonzero device error word.
+// The P3X status of a nonzero error word.
 int status_of_err(unsigned err);
 // Default launch shape of a step of dt seconds over ncol columns of nk levels.
 void default_shape(int precision, int nk, long long ncol, double dt, p3d::Shape* sh);

@@ -561,10 +561,11 @@ def summarize_pmc(fetch_dir, write_dir, out_path=None):
     scale_f = COPY_PROBE_BYTES / copy_f  # bytes per counter KiB, reads
     scale_w = COPY_PROBE_BYTES / copy_w  # bytes per counter KiB, writes
     kern = {}
-    # part 1 is p3_part1_lvl_kernel (one thread per level and column) or p3_part1_kernel;
-    # sedimentation is one launch of both species groups (p3_sed_fused_kernel) or two
-    # kernels (the ice group and the liquid group), summed
+    # parts 1 and 2 are one kernel, p3_front_kernel (builds that ran them apart:
+    # p3_part1*, p3_part2*); sedimentation is one launch of both species groups
+    # (p3_sed_fused_kernel) or two kernels (the ice group and the liquid group), summed
     for key, name in (("p3_part1", "p3_part1_kernel"), ("p3_part2", "p3_part2_kernel"),
+                      ("p3_front", "p3_front_kernel"), ("p3_order", "p3_order_kernel"),
                       ("p3_sed", "p3_sed_kernel"), ("p3_part3", "p3_part3_kernel")):
         f = pick(fetch, key)
         w = pick(write, key)

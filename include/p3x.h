@@ -190,7 +190,7 @@ typedef struct p3x_context p3x_context;
 
 /* Fill rt with the P3Runtime defaults (p3_functions.hpp:114-133). */
 void p3x_runtime_defaults(p3x_runtime* rt);
-/* Fill launch options with defaults (FP64, tuned block shape, synchronous). */
+/* Fill launch options with defaults (FP64, default lanes, synchronous). */
 void p3x_launch_defaults(p3x_launch* opts);
 
 /* Host: read the ice lookup table text (reader of p3_table_ice_impl.hpp:16-78,
@@ -246,7 +246,7 @@ int p3x_main_noalloc(p3x_context* ctx, const p3x_runtime* runtime,
 int p3x_sync(p3x_context* ctx);
 
 /* Device time of the context's last p3x_main (waits for it) in two intervals:
- * the part 1 and part 2 kernels, then the sedimentation and part 3 kernels.  No reference counterpart (the
+ * parts 1 and 2 with the columns' order, then sedimentation and part 3.  No reference counterpart (the
  * reference times the whole p3_main, p3_main_impl.hpp:328-330); it splits that
  * figure for profiling. */
 int p3x_last_kernel_times(p3x_context* ctx, double* part12_us, double* sed_us);
@@ -271,10 +271,10 @@ typedef struct p3x_column_set {
 
 typedef struct p3x_batch_options {
   int precision;             /* P3X_FP64 or P3X_MIXED                                     */
-  int columns_per_block;     /* part 1 shape, as in p3x_launch (0 = default)              */
+  int columns_per_block;     /* as in p3x_launch: accepted without effect                 */
   int threads_per_block;
   int sed_lanes_per_column;  /* 0 = default                                               */
-  int part12_waves_per_simd; /* 0 = default, 1 or 2, as in p3x_launch                    */
+  int part12_waves_per_simd; /* as in p3x_launch: accepted without effect                 */
   int blocks_per_cu;         /* persistent grid of each launch: this many blocks per CU;  */
                              /* 0 = as many as fit (occupancy); -1 = one block per unit   */
                              /* (the default: the kernels then run without their loop)   */
@@ -291,8 +291,8 @@ int p3x_batch_create(p3x_context* ctx, const p3x_runtime* runtime, const p3x_col
 /* Enqueue one step of every set on stream (NULL = default); returns after
  * enqueueing.  p3x_sync(ctx) waits and returns the status. */
 int p3x_batch_run(p3x_batch* batch, void* stream);
-/* Autotuner: times candidate shapes (part 1 + part 2 block shape, sedimentation
- * lanes per column, persistent blocks per CU) on the batch's own data, keeps the
+/* Autotuner: times candidate shapes (sedimentation lanes per column, persistent
+ * blocks per CU) on the batch's own data, keeps the
  * fastest, and leaves every set's state as it was.  reps timed steps per
  * candidate; chosen / best_us (optional) receive the result. */
 int p3x_batch_tune(p3x_batch* batch, void* stream, int reps, p3x_batch_options* chosen,
@@ -406,8 +406,8 @@ typedef struct p3x_server_options {
   int slots;                  /* batches in flight at once (one stream each); 0 = 4   */
   int max_batch;              /* requests per batch; 0 = 32                           */
   double scratch_budget_bytes;/* device scratch of all slots; 0 = 8 GiB               */
-  int columns_per_block, threads_per_block, sed_lanes_per_column;  /* 0 = default  */
-  int part12_waves_per_simd;                                        /* 0 = default  */
+  int columns_per_block, threads_per_block, sed_lanes_per_column;  /* as in p3x_launch */
+  int part12_waves_per_simd;                                       /* as in p3x_launch */
   double hbm_budget_bytes;    /* members' resident arrays + scratch; 0 = 200e9       */
 } p3x_server_options;
 

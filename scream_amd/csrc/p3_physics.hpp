@@ -137,7 +137,7 @@ template <class T> struct TableSet {
 // Functions of the runtime's one rain shape parameter (constant_mu_rain), so that
 // they are not computed at every level with rain: in FP64 the host's values, from
 // the same portable functions; in the mixed form the device's own FP32 values for
-// the default parameter, formed once per context.  mu: the parameter they belong
+// the default parameter, formed once per process.  mu: the parameter they belong
 // to, as the form's arithmetic holds it (with another one the kernels compute them).
 struct RainGamma {
   double mu;

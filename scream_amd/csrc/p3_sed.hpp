@@ -1,5 +1,5 @@
-// p3_sed.hpp -- second kernel of a P3 step: cloud, rain and ice sedimentation,
-// homogeneous freezing and p3_main_part3, with the surface precipitation.
+// p3_sed.hpp -- cloud, rain and ice sedimentation with the surface precipitation,
+// and homogeneous freezing with p3_main_part3.
 //
 // Work decomposition: one column per group of LPC lanes (LPC = 16, 32 or 64,
 // aligned inside the 64-lane wavefront); lane j of a group owns the L
@@ -8,7 +8,7 @@
 // substep needs from other levels goes through cross-lane operations inside
 // the group: the CFL maximum and find_top/find_bottom are butterfly
 // reductions, and the upwind flux entering a lane's first level is the last
-// level's flux of the lane above (one shuffle).  A column therefore runs
+// level's flux of the lane above (one lane shift).  A column therefore runs
 // exactly its own number of substeps, without block barriers, and reads its
 // state from HBM once per species.
 //
@@ -103,15 +103,15 @@ __device__ __forceinline__ double grp_below(double v, int j) {
   return LPC == 32 && j == 0 ? 0.0 : w;
 }
 
-// Sedimentation runs as two kernels over the same column blocks, one per
-// species group: the liquid group (cloud, then rain, with the rain flux and
+// Sedimentation runs as two kernels, or two halves of one launch, over the same
+// column blocks, one per species group: the liquid group (cloud, then rain, with the rain flux and
 // the liquid surface precipitation) and the ice group.  The groups touch
 // disjoint state fields, so their order does not change a bit; apart, each
-// kernel holds only its own group's registers and field pointers.
+// block holds only its own group's field pointers.
 
 // Wavefronts per SIMD the sedimentation kernels are compiled for: up to 5
 // levels per lane two fit (256 registers); the FP64 ice group at up to 3
-// levels per lane runs at three (168 registers and a 76-byte spill at 3 levels:
+// levels per lane runs at three (159 registers at 3 levels, 135 at 2; at three:
 // 736 -> 714 us at 21600 x 72; the FP32 ice group holds 127 registers anyway).
 template <class R, int G, int L> constexpr int sed_waves_per_simd() {
   return (G == SED_ICE && sizeof(R) == 8 && L <= 3) ? 3 : (L <= 5 ? 2 : 1);
@@ -426,7 +426,7 @@ __device__ __forceinline__ void sediment_run(const KParams& p, int i, int j, int
 // find_top (P3I/p3_find_impl.hpp:14-50) of NS species (mixing ratios f[s]) over
 // the group's column in the standard mapping (lane j: levels j*L .. j*L+L-1),
 // all loads in one pass; top[s] = nlev when species s is absent (or the column
-// does not run).
+// does not run).  For columns that p3_order_kernel has not listed.
 template <int LPC, int L, int NS>
 __device__ __forceinline__ void find_tops(const KParams& p, int i, int j, bool run,
                                           const double* const (&f)[NS], int (&top)[NS]) {

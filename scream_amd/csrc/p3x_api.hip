@@ -350,8 +350,8 @@ extern "C" int p3x_init(const p3x_table_data* t, p3x_context** out) {
   up(&c->d_tab, pack_tables<double>(t));
   up(&c->d_tab_f, pack_tables<float>(t));
   // The error word, in host memory (p3x_sync reads it without a copy: a waiting
-  // step of one column of 72 levels 57 -> 46 us, 93 -> 75 with the state copied), and room for the four floats of
-  // default_rain_gamma.
+  // step of one column of 72 levels 57 -> 46 us, 93 -> 75 with the state copied),
+  // and room for the four floats of default_rain_gamma.
   if (e == hipSuccess) e = hipHostMalloc((void**)&c->h_err, 8 * sizeof(unsigned), hipHostMallocCoherent);
   if (e == hipSuccess) std::memset(c->h_err, 0, 8 * sizeof(unsigned));
   if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&c->d_err, c->h_err, 0);
@@ -506,7 +506,8 @@ int p3x_detail::main_impl(p3x_context* c, const p3x_runtime* runtime, const p3x_
   }
   e = hipEventRecord(c->ev0, s);
   if (e != hipSuccess) return P3X_ERR_DEVICE;
-  // the liquid sedimentation kernel beside the ice kernel (21600 x 72 FP64: 1255 -> 1216 us per step)
+  // the liquid sedimentation kernel beside the ice kernel, where they are two
+  // (16384 x 128 FP64: 785 -> 752 us per step when it was added)
   const p3d::SedFork fork{c->side, c->ev_fork, c->ev_join};
   e = o.precision == P3X_FP64 ? p3d::launch_p3_fp64(k, sh, s, c->ev_mid, &fork)
                               : p3d::launch_p3_mixed(k, sh, s, c->ev_mid, &fork);

@@ -21,7 +21,7 @@ struct p3x_context {
   unsigned* d_err = nullptr;  // its device address
   p3d::RainGamma rain_mixed{};  // of the mixed form, for the default constant_mu_rain
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  hipEvent_t ev_mid = nullptr;  // between the part 1 + 2 and the sedimentation kernels
+  hipEvent_t ev_mid = nullptr;  // before the sedimentation kernels
   // the liquid sedimentation kernel's stream (beside the ice kernel) and its
   // fork and join events
   hipStream_t side = nullptr;

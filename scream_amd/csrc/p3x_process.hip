@@ -3,8 +3,8 @@
 // maximum-overlap rain fraction), p3_main, and post-amble (the rescaled
 // temperature change, dry -> wet, effective radii in microns, the accumulated
 // surface precipitation masses and the optional boundary fluxes).  The pre-amble
-// runs inside the part 1 kernel and the post-amble inside the sedimentation +
-// part 3 kernel (p3d::Amble), so a process step launches the p3_main kernels only.
+// runs inside the front kernel and the post-amble inside sedimentation and part 3
+// (p3d::Amble), so a process step launches the p3_main kernels only.
 //
 // Follows components/eamxx/src/physics/p3/eamxx_p3_process_interface.hpp:63-261,
 // eamxx_p3_process_interface.cpp:249-340 (which fields feed p3_main) and

@@ -402,8 +402,8 @@ class Context:
             raise P3Error(st, "p3x_reserve")
 
     def last_kernel_times(self) -> tuple[float, float]:
-        """Device microseconds of the last main() in two intervals: (the part 1 and part 2
-        kernels, the sedimentation and part 3 kernels)."""
+        """Device microseconds of the last main() in two intervals: (parts 1 and 2 with the
+        columns' order, sedimentation and part 3)."""
         a, b = C.c_double(), C.c_double()
         st = self._lib.p3x_last_kernel_times(self.handle, C.byref(a), C.byref(b))
         if st != P3X_OK:

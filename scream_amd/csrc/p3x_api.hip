@@ -105,17 +105,23 @@ int status_of_err(unsigned err) {
 //   FP64  2700 x 72 dt 300    114 / 126 / 116, clear 113 / 115 / 112
 //   mixed 5400 x 72 dt 1800   206 / 183 / 208, clear 173 / 165 / 192
 //   mixed 10000 x 72 dt 1800  291 / 291 / 345, clear 255 / 253 / 311
-// FP64 from 97 to 128 levels runs the groups apart, the ice on 64 lanes (2 levels,
-// three wavefronts per SIMD) and the liquid on 32: 16384 x 128 dt 300 734, against
-// 768 with both on 32 (712 and 682 with a third of the columns clear).
+// FP64 from 97 to 128 levels runs the groups of a short step apart, the ice on 64
+// lanes (2 levels, three wavefronts per SIMD) and the liquid on 32 (us apart / both
+// on 32): 16384 x 128 dt 100 594 / 602, clear 580 / 566; dt 300 735 / 762, clear 705 /
+// 669.  Of a long one, whose many substeps want the clear columns out of the way,
+// both on 32: dt 1800 1469 / 1483, clear 1350 / 1171; 6000 x 128 608 / 580, clear 568 /
+// 465; 12000 x 100 865 / 867, clear 798 / 683.  Not with few columns, where a batch
+// of short and long steps lasts as long as its longest (12 FP64 sets of 33 to 700
+// columns: 266 us with 128 levels on 64 lanes, 303 on 32).
 constexpr int kFewColumns = 2560;
 void default_shape(int precision, int nk, long long ncol, double dt, p3d::Shape* sh) {
   const bool mixed = precision == P3X_MIXED;
+  const bool long_step = dt * nk >= 600. * 72;  // 600 s on 72 levels
   int l = nk <= 80 ? 16 : (nk <= 32 * 5 ? 32 : 64);
   if (ncol <= (mixed && nk > 80 ? 4096 : kFewColumns)) l = 64;
-  else if (l == 16 && (mixed ? nk > 48 && ncol <= 8192 : ncol <= 3072 && dt * nk >= 600. * 72)) l = 32;
+  else if (l == 16 && (mixed ? nk > 48 && ncol <= 8192 : ncol <= 3072 && long_step)) l = 32;
   sh->lpc = sh->lpc_ice = l;
-  if (!mixed && l == 32 && nk > 96 && nk <= 128) sh->lpc_ice = 64;
+  if (!mixed && l == 32 && nk > 96 && nk <= 128 && !(long_step && ncol > 4096)) sh->lpc_ice = 64;
 }
 
 // Offsets (in elements) of the tables in one device allocation; each is a

@@ -77,53 +77,85 @@ struct BudgetParams {
   double *mass, *energy;
   int ncol, nlev;
   int cs, ks;  // element (i, k) at i*cs + k*ks
+  int levels_log2;  // levels a turn: nlev rounded up to a power of two, 64 at most
 };
 
-// Column sums of mass and energy, levels in order, so that they round like the
-// oracle's.  A block takes kBudCols columns: all its threads form the terms of
-// kBudLevels levels (a row of 16 columns is one 128-byte line level-major, a run
-// of 64 levels four of them column-major) and leave them in LDS, and one thread
-// per column and sum adds them up in order.  One thread per column doing both
-// waited out a memory round trip for every level: 59 us at 5400 x 72 and 57 us
-// at 867 x 128, against 8 us here.
-constexpr int kBudCols = 16, kBudLevels = 64, kBudStride = kBudCols + 1;
-__global__ __launch_bounds__(256) void p3_column_budget_kernel(const BudgetParams b) {
-  __shared__ double s_term[2][kBudLevels * kBudStride];
+// A point's terms of the column sums.
+__device__ __forceinline__ void budget_terms(const BudgetParams& b, int i, int k, double& m, double& e) {
   const p3x_budget_fields& f = b.f;
   const double g = p3c::gravit, cp = p3c::CP, lv = p3c::LatVap, lf = p3c::LatIce;
-  const int tid = threadIdx.x, i0 = blockIdx.x * kBudCols;
-  const int which = tid / kBudCols, ci = i0 + tid % kBudCols;  // of the summing threads
-  double sum = 0;
-  for (int k0 = 0; k0 < b.nlev; k0 += kBudLevels) {
+  const size_t x = (size_t)i * b.cs + (size_t)k * b.ks;
+  const double dp = f.pseudo_density[x];
+  const double qv = f.qv[x], qc = f.qc[x], qi = f.qi[x], qr = f.qr[x];
+  const double u2 = f.u ? f.u[x] * f.u[x] : 0.0;
+  const double v2 = f.v ? f.v[x] * f.v[x] : 0.0;
+  m = (qv + qc + qi + qr) * dp / g;
+  e = (f.T_mid[x] * cp + 0.5 * (u2 + v2) + (lv + lf) * qv + lf * (qc + qr)) * dp / g;
+}
+__device__ __forceinline__ double budget_surface(const BudgetParams& b, int i) {
+  return (b.f.phis ? b.f.phis[i] : 0.0) * (b.f.ps ? b.f.ps[i] : 0.0) / p3c::gravit;
+}
+
+// Column sums of mass and energy, levels in order, so that they round like the
+// oracle's.  All threads of a block form the terms of kBudPoints points in LDS, and
+// then one thread per column and sum adds them up in order.  One thread per column
+// doing both waited out a memory round trip for every level: 59 us at 5400 x 72 and
+// 57 us at 867 x 128, against 8 us here.  A turn takes the column's levels rounded up
+// to a power of two, 64 at most, and as many columns as that leaves: with 64 levels a
+// row of 16 columns is one 128-byte line level-major and a run of levels four of them
+// column-major; with 16 columns per block at any depth, columns of few levels left
+// most threads without a point (level-major / column-major at 400000 x 4 21.6 / 68.2
+// us, here 16.9 / 14.6; at 200000 x 16 41.0 / 36.8, here 23.8 / 23.7).
+constexpr int kBudPoints = 1024, kBudLevelsLog2 = 6;
+constexpr int kBudTerms = kBudPoints + (1 << kBudLevelsLog2);  // rows of columns + 1
+__global__ __launch_bounds__(256) void p3_column_budget_kernel(const BudgetParams b) {
+  __shared__ double s_term[2][kBudTerms];
+  const int levels = 1 << b.levels_log2, cols_log2 = 10 - b.levels_log2, cols = kBudPoints >> b.levels_log2;
+  static_assert(kBudPoints == 1 << 10, "cols_log2");
+  const int tid = threadIdx.x, i0 = blockIdx.x * cols;
+  double sum = 0;  // of the levels before (several turns: at most one column and sum per thread)
+  for (int k0 = 0; k0 < b.nlev; k0 += levels) {
 #pragma unroll
-    for (int t = 0; t < kBudCols * kBudLevels / 256; ++t) {
+    for (int t = 0; t < kBudPoints / 256; ++t) {
       const int e = tid + t * 256;
-      const int c = b.ks == 1 ? e / kBudLevels : e % kBudCols;
-      const int kk = b.ks == 1 ? e % kBudLevels : e / kBudCols;
-      const int i = i0 + c, k = k0 + kk;
-      if (i < b.ncol && k < b.nlev) {
-        const size_t x = (size_t)i * b.cs + (size_t)k * b.ks;
-        const double dp = f.pseudo_density[x];
-        const double qv = f.qv[x], qc = f.qc[x], qi = f.qi[x], qr = f.qr[x];
-        const double u2 = f.u ? f.u[x] * f.u[x] : 0.0;
-        const double v2 = f.v ? f.v[x] * f.v[x] : 0.0;
-        s_term[0][kk * kBudStride + c] = (qv + qc + qi + qr) * dp / g;
-        s_term[1][kk * kBudStride + c] =
-            (f.T_mid[x] * cp + 0.5 * (u2 + v2) + (lv + lf) * qv + lf * (qc + qr)) * dp / g;
-      }
+      const int c = b.ks == 1 ? e >> b.levels_log2 : e & (cols - 1);
+      const int kk = b.ks == 1 ? e & (levels - 1) : e >> cols_log2;
+      const int i = i0 + c, k = k0 + kk, at = kk * (cols + 1) + c;
+      if (i < b.ncol && k < b.nlev) budget_terms(b, i, k, s_term[0][at], s_term[1][at]);
     }
     __syncthreads();
-    if (which < 2 && ci < b.ncol) {
-      const int n = b.nlev - k0 < kBudLevels ? b.nlev - k0 : kBudLevels;
-      const double* const s = s_term[which] + tid % kBudCols;
+    const int n = b.nlev - k0 < levels ? b.nlev - k0 : levels;
+    for (int w = tid; w < 2 * cols; w += 256) {
+      const int which = w >> cols_log2, c = w & (cols - 1), i = i0 + c;
+      if (i >= b.ncol) continue;
+      const double* const s = s_term[which] + c;
 #pragma unroll 8
-      for (int kk = 0; kk < n; ++kk) sum += s[kk * kBudStride];
+      for (int kk = 0; kk < n; ++kk) sum += s[kk * (cols + 1)];
+      if (k0 + levels < b.nlev) continue;  // the next turn goes on
+      if (which == 0) b.mass[i] = sum;
+      else b.energy[i] = sum + budget_surface(b, i);
+      sum = 0;
     }
     __syncthreads();
   }
-  if (which == 0 && ci < b.ncol) b.mass[ci] = sum;
-  if (which == 1 && ci < b.ncol)
-    b.energy[ci] = sum + (f.phis ? f.phis[ci] : 0.0) * (f.ps ? f.ps[ci] : 0.0) / g;
+}
+
+// One thread per column: with one or two levels there is nothing to wait for in
+// turn, and the way through LDS costs 10.5 -> 13.0 us at 1000000 x 1, 5.5 -> 6.6 at
+// 300000 x 2 (400000 x 4: 16.2 / 27.1 us in the two layouts against 16.9 / 14.6).
+constexpr int kBudFewLevels = 2;
+__global__ __launch_bounds__(256) void p3_column_budget_few_kernel(const BudgetParams b) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= b.ncol) return;
+  double m = 0, e = 0;
+  for (int k = 0; k < b.nlev; ++k) {
+    double mk, ek;
+    budget_terms(b, i, k, mk, ek);
+    m += mk;
+    e += ek;
+  }
+  b.mass[i] = m;
+  b.energy[i] = e + budget_surface(b, i);
 }
 
 struct ErrParams {
@@ -153,8 +185,12 @@ extern "C" int p3x_column_budget(p3x_context* c, const p3x_budget_fields* f, int
   p3d::KParams g;
   if (set_geometry(ncol, nlev, f->layout, f->ld, 0, &g) != P3X_OK) return P3X_ERR_ARG;
   if (ncol == 0) return P3X_OK;
-  const BudgetParams b{*f, mass, energy, ncol, nlev, g.cs, g.ks};
-  hipLaunchKernelGGL(p3_column_budget_kernel, dim3((ncol + kBudCols - 1) / kBudCols), dim3(256), 0, (hipStream_t)stream, b);
+  BudgetParams b{*f, mass, energy, ncol, nlev, g.cs, g.ks, 0};
+  while (b.levels_log2 < kBudLevelsLog2 && 1 << b.levels_log2 < nlev) ++b.levels_log2;
+  const bool few = nlev <= kBudFewLevels;
+  const int cols = few ? 256 : kBudPoints >> b.levels_log2;
+  hipLaunchKernelGGL(few ? p3_column_budget_few_kernel : p3_column_budget_kernel,
+                     dim3((unsigned)(((long long)ncol + cols - 1) / cols)), dim3(256), 0, (hipStream_t)stream, b);
   return hipGetLastError() == hipSuccess ? P3X_OK : P3X_ERR_DEVICE;
 }
 

@@ -47,6 +47,58 @@ hipError_t noalloc_scratch_on(int dev, double** out) {
   return hipSuccess;
 }
 
+// The contexts' error words, in pages of pinned host memory.  A context takes a slot,
+// a cache line of its own, for its lifetime; a page whose slots are all back is freed
+// unless it is the only one.  (With an allocation of its own each of 24 contexts alive
+// together took 232-278 us to create and 580 to close, here 194-230 and 345.)
+constexpr int kPageBytes = 4096, kSlotBytes = 64;
+struct WordPage {
+  char* h;
+  unsigned long long used;  // a bit per slot
+};
+static_assert(kPageBytes / kSlotBytes == 64, "one bit per slot");
+std::mutex g_words_mu;
+std::vector<WordPage>& word_pages() {  // (never destroyed: a context may be finalized during exit)
+  static auto* const pages = new std::vector<WordPage>;
+  return *pages;
+}
+
+// A zeroed slot, reachable from every device.
+hipError_t take_words(unsigned** h) {
+  std::lock_guard<std::mutex> lk(g_words_mu);
+  std::vector<WordPage>& pages = word_pages();
+  size_t n = 0;
+  while (n < pages.size() && ~pages[n].used == 0) ++n;
+  if (n == pages.size()) {
+    void* p = nullptr;
+    const hipError_t e = hipHostMalloc(&p, kPageBytes, hipHostMallocCoherent | hipHostMallocPortable);
+    if (e != hipSuccess) return e;
+    pages.push_back({(char*)p, 0});
+  }
+  const int slot = __builtin_ctzll(~pages[n].used);
+  pages[n].used |= 1ull << slot;
+  char* const w = pages[n].h + slot * kSlotBytes;
+  std::memset(w, 0, kSlotBytes);
+  *h = (unsigned*)w;
+  return hipSuccess;
+}
+
+// (once no kernel that may write the slot is left)
+void give_words(unsigned* h) {
+  std::lock_guard<std::mutex> lk(g_words_mu);
+  std::vector<WordPage>& pages = word_pages();
+  for (size_t n = 0; n < pages.size(); ++n) {
+    const long off = (char*)h - pages[n].h;
+    if (off < 0 || off >= kPageBytes) continue;
+    pages[n].used &= ~(1ull << off / kSlotBytes);
+    if (pages[n].used == 0 && pages.size() > 1) {
+      (void)hipHostFree(pages[n].h);
+      pages.erase(pages.begin() + n);
+    }
+    return;
+  }
+}
+
 // RainGamma of the mixed form for the default constant_mu_rain: the FP32 values of
 // this code on this architecture, formed by the process's first context.
 std::mutex g_rain_mu;
@@ -358,8 +410,7 @@ extern "C" int p3x_init(const p3x_table_data* t, p3x_context** out) {
   // The error word, in host memory (p3x_sync reads it without a copy: a waiting
   // step of one column of 72 levels 57 -> 46 us, 93 -> 75 with the state copied),
   // and room for the four floats of default_rain_gamma.
-  if (e == hipSuccess) e = hipHostMalloc((void**)&c->h_err, 8 * sizeof(unsigned), hipHostMallocCoherent);
-  if (e == hipSuccess) std::memset(c->h_err, 0, 8 * sizeof(unsigned));
+  if (e == hipSuccess) e = take_words(&c->h_err);
   if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&c->d_err, c->h_err, 0);
   if (e == hipSuccess) e = default_rain_gamma((float*)(c->d_err + 4), &c->rain_mixed);
   // The three events order and time work on this device alone; what the host reads
@@ -389,12 +440,18 @@ extern "C" int p3x_init(const p3x_table_data* t, p3x_context** out) {
 
 extern "C" void p3x_finalize(p3x_context* c) {
   if (!c) return;
+  // no kernel of the context is left on its device, whichever is current: its error
+  // word goes to another context
+  int current = c->device;
+  (void)hipGetDevice(&current);
+  if (current != c->device) (void)hipSetDevice(c->device);
   (void)hipDeviceSynchronize();
+  if (current != c->device) (void)hipSetDevice(current);
   // teardown: nothing useful can be done with a failure here
   (void)hipFree(c->d_tab);
   (void)hipFree(c->d_tab_f);
   (void)hipFree(c->d_scratch);
-  if (c->h_err) (void)hipHostFree(c->h_err);
+  if (c->h_err) give_words(c->h_err);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->ev_mid) (void)hipEventDestroy(c->ev_mid);

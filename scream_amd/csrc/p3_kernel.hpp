@@ -109,8 +109,21 @@ __host__ __device__ __forceinline__ double exner_function(double pres) {  // Phy
 
 // Air density of a layer (dpres / dz / g), as every kernel forms it.
 __device__ __forceinline__ double air_density(double dpres, double dz) {
-  return p3m_div(p3m_div(dpres, dz), gravit);
+  return p3m_div(p3m_div_inf(dpres, dz), gravit);
 }
+
+// q * num / den of several q, with one reciprocal; both factors are scaled by a power
+// of two where den is too small for that, which changes no bit of a quotient.
+struct Ratio {
+  double num, den, rden;
+  __device__ __forceinline__ Ratio(double n, double d) {
+    const double s = m_fabs(d) < 0x1p-1000 ? 0x1p100 : 1.0;
+    num = n * s;
+    den = d * s;
+    rden = p3m_recip(den);
+  }
+  __device__ __forceinline__ double of(double q) const { return p3m_div_y_inf(q * num, den, rden); }
+};
 
 constexpr int kMaxSubsteps = 100000;
 // Column status bits: part 1 found work, part 2 left hydrometeors.
@@ -168,11 +181,11 @@ __device__ __forceinline__ void front_level(const KParams& p, int k, int i, cons
     const double dp = a.dp_wet[x], dp_dry = p.dpres[x];
     const double c1 = -1.0 + 1.0 / ep_2;  // calculate_dz with the wet qv's virtual temperature
     const double T_virtual = T * (1.0 + c1 * p.qv[x]);
-    dz = p3m_div((Rair / gravit) * dp * T_virtual, pmid);
+    dz = p3m_div_inf((Rair / gravit) * dp * T_virtual, pmid);
     a.dz[x] = dz;
     // wet -> dry mixing ratios (calculate_drymmr_from_wetmmr_dp_based)
-    const double rdry = p3m_recip(dp_dry);
-    auto to_dry = [&](double q) { return p3m_div_y(q * dp, dp_dry, rdry); };
+    const Ratio dry(dp, dp_dry);
+    auto to_dry = [&](double q) { return dry.of(q); };
     qc = to_dry(p.qc[x]); nc = to_dry(p.nc[x]); qr = to_dry(p.qr[x]);
     nr = to_dry(p.nr[x]); qi = to_dry(p.qi[x]); ni = to_dry(p.ni[x]);
     qm = to_dry(p.qm[x]); bm = to_dry(p.bm[x]);
@@ -223,16 +236,16 @@ __device__ __forceinline__ void front_level(const KParams& p, int k, int i, cons
   // stored again (with the pre-amble every field changes to dry)
   const double in[10] = {qc, nc, qr, nr, qi, ni, qm, bm, qv, th};
   qv = vmax(qv, 0.0);
-  const double exner = p3m_div(1.0, inv_exner);
+  const double exner = p3m_div_inf(1.0, inv_exner);
   double T_atm = th * exner;
   const double rho = air_density(dpres, dz);
-  const double inv_rho = p3m_div(1.0, rho);
+  const double inv_rho = p3m_div_inf(1.0, rho);
   const double T_first = T_atm;
   double lh, ll;
   log_temperature(T_atm, lh, ll);
   double qv_sat_l, qv_sat_i;
   qv_sat_dry_both(T_atm, lh + ll, pres, qv_sat_l, qv_sat_i, err);
-  const double qv_supersat_i = p3m_div(qv, qv_sat_i) - 1;
+  const double qv_supersat_i = p3m_div_inf(qv, qv_sat_i) - 1;
   double rhofacr, rhofaci, acn;
   R mu;
   {

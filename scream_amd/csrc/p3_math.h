@@ -51,13 +51,19 @@ P3M_FN double p3m_nan(void) { return p3m_from_bits(0x7ff8000000000000ULL); }
  * (v_div_scale) and the condition code they leave only serve operands near the
  * ends of the exponent range.  Without that scaling the same steps -- v_rcp,
  * two Newton steps y <- y + y (1 - b y), q = a y, q + y (a - b q) -- give the
- * same bits whenever b, a / b and 1 / b are normal, |a| >= 2^-969 and
- * |a / b| < 2^768: the scaling is then the identity.  A quarter-rate v_rcp
- * included, a division measured 65 cycles per wavefront on MI355X against 52
- * here and 20 for one more division by the same b (p3m_div_y).
+ * same bits whenever b, a / b and 1 / b are normal and |a| >= 2^-969.  A
+ * quarter-rate v_rcp included, a division measured 65 cycles per wavefront on
+ * MI355X against 52 here and 20 for one more division by the same b (p3m_div_y).
  * v_div_fixup keeps the results for zero, infinite and NaN operands; the _n form
- * leaves it out where the operands are finite and b is not zero.  On the CPU
- * all of these are a / b. */
+ * leaves it out where the operands are finite and b is not zero.  For |a| < 2^-969
+ * the result is within one unit in the last place.  Not covered, and so to be kept
+ * away by a guard on the operands or by their form:
+ *  - a quotient beyond the largest number (the last step leaves inf - inf).
+ *    p3m_div_inf is infinite there: the minimum with infinity drops the NaN;
+ *  - b so small that 1 / b overflows, |b| <= 2^-1024.  p3m_div_inf is right there
+ *    for |a| >= 1, p3m_div_any for every a.
+ * A caller's field as the divisor takes p3m_div_any.  On the CPU all of these are
+ * a / b. */
 #if P3M_DEVICE
 P3M_FN double p3m_recip(double b) { /* the refined 1/b of the division, for p3m_div_y */
   double y = __builtin_amdgcn_rcp(b);
@@ -71,13 +77,29 @@ P3M_FN double p3m_div_yn(double a, double b, double y) {
 P3M_FN double p3m_div_y(double a, double b, double y) {
   return __builtin_amdgcn_div_fixup(p3m_div_yn(a, b, y), b, a);
 }
+P3M_FN double p3m_div_y_inf(double a, double b, double y) {
+  return __builtin_amdgcn_div_fixup(__builtin_fmin(p3m_div_yn(a, b, y), p3m_inf()), b, a);
+}
+/* a / b for any operands: the same steps on scaled ones (written out, since the
+ * mixed form's flags allow the compiler an a / b without scaling and fixup) */
+P3M_FN double p3m_div_any(double a, double b) {
+  bool unused, scaled;
+  const double d = __builtin_amdgcn_div_scale(a, b, false, &unused);
+  const double n = __builtin_amdgcn_div_scale(a, b, true, &scaled);
+  const double y = p3m_recip(d);
+  const double q = n * y;
+  return __builtin_amdgcn_div_fixup(__builtin_amdgcn_div_fmas(fma(-d, q, n), y, q, scaled), b, a);
+}
 #else
 P3M_FN double p3m_recip(double b) { return 1.0 / b; }
 P3M_FN double p3m_div_yn(double a, double b, double y) { (void)y; return a / b; }
 P3M_FN double p3m_div_y(double a, double b, double y) { (void)y; return a / b; }
+P3M_FN double p3m_div_y_inf(double a, double b, double y) { (void)y; return a / b; }
+P3M_FN double p3m_div_any(double a, double b) { return a / b; }
 #endif
 P3M_FN double p3m_div(double a, double b) { return p3m_div_y(a, b, p3m_recip(b)); }
 P3M_FN double p3m_div_n(double a, double b) { return p3m_div_yn(a, b, p3m_recip(b)); }
+P3M_FN double p3m_div_inf(double a, double b) { return p3m_div_y_inf(a, b, p3m_recip(b)); }
 
 /* a * b + c for a constant c.  hipcc forms v_fmac, which overwrites c, and so
  * moves every polynomial coefficient into vector registers first (three

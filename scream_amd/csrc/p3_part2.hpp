@@ -63,7 +63,7 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const RainGamma& 
   double qr_incld_d;
   {
     const Incld in0 = incloud(s[S_QC], s[S_QR], s[S_QI], s[S_QM], s[S_NC], s[S_NR], s[S_NI], s[S_BM],
-                              p3m_div(1.0, s[S_CFL]), p3m_div(1.0, s[S_CFI]), p3m_div(1.0, s[S_CFR]));
+                              p3m_div_inf(1.0, s[S_CFL]), p3m_div_inf(1.0, s[S_CFI]), p3m_div_inf(1.0, s[S_CFR]));
     qc_incld = R(in0.qc); qr_incld = R(in0.qr); qi_incld = R(in0.qi); qm_incld = R(in0.qm);
     nc_incld = R(in0.nc); nr_incld = R(in0.nr); ni_incld = R(in0.ni); bm_incld = R(in0.bm);
     qr_incld_d = in0.qr;
@@ -91,9 +91,9 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const RainGamma& 
     R T181;  // T^1.81
     if constexpr (sizeof(R) == 8) T181 = s[S_T181];
     else T181 = m_pow(Tr, R(1.81));
-    const R dv = m_div(R(8.794e-5) * T181, R(s[S_PRES]));
-    const R sc = m_div(mu, rhor * dv);
-    const R dum_t = m_div(R(1), R(RV) * (Tr * Tr));
+    const R dv = m_div<DIV_INF>(R(8.794e-5) * T181, R(s[S_PRES]));
+    const R sc = m_div<DIV_INF>(mu, rhor * dv);
+    const R dum_t = m_div<DIV_INF>(R(1), R(RV) * (Tr * Tr));
     const R dqsdt = R(latvap) * R(s[S_QVSL]) * dum_t;
     const R dqsidt = R(latvap + latice) * R(s[S_QVSI]) * dum_t;
     const R ab = R(1) + dqsdt * R(latvap) * R(INV_CP);
@@ -310,7 +310,7 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const RainGamma& 
       const R cfr = R(s[S_CFR]);
       if (qr_incld >= R(QSMALL) && ssat_r_d < 0 && cfr > cld_frac) {
         const R inv_dt_r = R(1 / dt);
-        const R tau_r = m_div(R(1), epsr);
+        const R tau_r = m_div<DIV_INF>(R(1), epsr);
         const R dqv_dt = R((s[S_QV] - s[S_QV_PREV]) * (1 / dt));
         const R dT = R(T_atm - s[S_T_PREV]);
         R eps_eff, A_c;
@@ -343,7 +343,7 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const RainGamma& 
         if (ev > ev_max) ev = ev_max;
         if (ev < 0) ev = 0;
         if (ev > qr_incld_d * inv_dt_d) ev = qr_incld_d * inv_dt_d;
-        ev = p3m_div(ev * (s[S_CFR] - cfd), s[S_CFR]);
+        ev = p3m_div_any(ev * (s[S_CFR] - cfd), s[S_CFR]);
         evap_d = ev;
         nr_evap_d = ev * p3m_div(double(nr_incld), qr_incld_d);
       }
@@ -563,7 +563,7 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const RainGamma& 
   }
   // ice_supersat_conservation, P3I/p3_ice_supersat_conservation_impl.hpp:14-43
   {
-    const double t_atm = p3m_div(u.th, s[S_INV_EXNER]);
+    const double t_atm = p3m_div_inf(u.th, s[S_INV_EXNER]);
     const double latsublim2 = (latvap + latice) * (latvap + latice);
     const double qv_sink = t_qv2qi_vapdep + t_qv2qi_nucleat;
     if (qv_sink > QSMALL && cld_frac_i > 1e-20) {
@@ -658,7 +658,7 @@ __device__ __forceinline__ bool part2_level(const Runtime& rt, const RainGamma& 
 
     // P3I/p3_main_impl_part2.hpp:514-517
     if (u.ni != 0) {  // (0 stays 0, also where the cloud fraction is 0)
-      double ni_incld_d = p3m_div(u.ni, cld_frac_i);
+      double ni_incld_d = p3m_div_any(u.ni, cld_frac_i);
       impose_max_total_ni<double>(ni_incld_d, rt.max_total_ni, s[S_INV_RHO]);
       u.ni = ni_incld_d * cld_frac_i;
     }

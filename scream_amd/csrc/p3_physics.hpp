@@ -46,10 +46,13 @@ __device__ __forceinline__ float m_expm1(float x) { return ::expm1f(x); }
 __device__ __forceinline__ double m_fabs(double x) { return ::fabs(x); }
 __device__ __forceinline__ float m_fabs(float x) { return ::fabsf(x); }
 
-// Division whose operands and quotient stay inside the exponent range that
-// needs no scaling (p3_math.h); the mixed form divides as it always did.
-__device__ __forceinline__ double m_div(double a, double b) { return p3m_div(a, b); }
-__device__ __forceinline__ float m_div(float a, float b) { return a / b; }
+// Division whose quotient does not overflow, and where it may (p3_math.h); the mixed
+// form divides as it always did.
+enum Div { DIV, DIV_INF };
+template <Div D = DIV> __device__ __forceinline__ double m_div(double a, double b) {
+  return D == DIV_INF ? p3m_div_inf(a, b) : p3m_div(a, b);
+}
+template <Div D = DIV> __device__ __forceinline__ float m_div(float a, float b) { return a / b; }
 
 // t^y of a temperature whose logarithm is at hand (FP64: from it, h + l; NaN
 // where t is not positive and finite; the mixed form takes its own pow)
@@ -78,12 +81,12 @@ __device__ __forceinline__ void report_errors(unsigned* word, unsigned err) {
 // MurphyKoop_svp, PSH:38-77 (check_temperature, PSH:14-36, as a flag), from
 // log(t) and the reciprocal of t that its divisions by t share
 __host__ __device__ __forceinline__ double mk_svp_ice(double t, double logt, double rt) {
-  return p3m_exp(9.550426 - p3m_div_y(5723.265, t, rt) + (3.53068 * logt) - (0.00728332 * t));
+  return p3m_exp(9.550426 - p3m_div_y_inf(5723.265, t, rt) + (3.53068 * logt) - (0.00728332 * t));
 }
 __host__ __device__ __forceinline__ double mk_svp_liquid(double t, double logt, double rt) {
-  return p3m_exp(54.842763 - p3m_div_y(6763.22, t, rt) - (4.210 * logt) + (0.000367 * t) +
+  return p3m_exp(54.842763 - p3m_div_y_inf(6763.22, t, rt) - (4.210 * logt) + (0.000367 * t) +
                (p3m_tanh(0.0415 * (t - 218.8)) *
-                (53.878 - p3m_div_y(1331.22, t, rt) - (9.44523 * logt) + 0.014025 * t)));
+                (53.878 - p3m_div_y_inf(1331.22, t, rt) - (9.44523 * logt) + 0.014025 * t)));
 }
 __host__ __device__ __forceinline__ void check_temperature(double t, unsigned& err) {
   if (t <= 0 || t != t) err |= ERR_BAD_TEMPERATURE;  // t != t: NaN
@@ -170,16 +173,16 @@ __device__ __forceinline__ double m_log10_pos(double x) { return p3m_log10_pos(x
 __device__ __forceinline__ float m_log10_pos(float x) { return m_log10(x); }
 
 // lookup_ice, P3I/p3_table_ice_impl.hpp:80-138 (qi and ni are positive)
-template <class R>
+template <class R, Div D = DIV_INF>
 __device__ __forceinline__ TabIce<R> lookup_ice(R qi, R ni, R qm, R rhop) {
   TabIce<R> t;
-  t.dum1 = (m_log10_pos(m_div(qi, ni)) + R(18)) * R(lookup_table_1a_dum1_c) - R(10);
+  t.dum1 = (m_log10_pos(m_div<D>(qi, ni)) + R(18)) * R(lookup_table_1a_dum1_c) - R(10);
   t.dumi = (int)t.dum1;
   t.dum1 = vmin(t.dum1, R(isize));
   t.dum1 = vmax(t.dum1, R(1.));
   t.dumi = vmax(1, t.dumi);
   t.dumi = vmin(isize - 1, t.dumi);
-  t.dum4 = m_div(qm, qi) * R(3) + R(1);
+  t.dum4 = m_div<D>(qm, qi) * R(3) + R(1);
   t.dumii = (int)t.dum4;
   t.dum4 = vmin(t.dum4, R(rimsize));
   t.dum4 = vmax(t.dum4, R(1.));
@@ -434,7 +437,7 @@ __device__ __forceinline__ void apply_table3_v(const R* __restrict__ table, cons
 
 // ---------------------------------------------------------------- size distributions
 // get_cloud_dsd2, P3I/p3_dsd2_impl.hpp:14-71 (iparam = 3, nu stays 0)
-template <class R>
+template <class R, Div D = DIV_INF>
 __device__ __forceinline__ void get_cloud_dsd2(R qc, R& nc, R& mu_c, R rho, R& lamc) {
   lamc = R(0); mu_c = R(0);
   if (qc >= R(QSMALL)) {
@@ -444,26 +447,26 @@ __device__ __forceinline__ void get_cloud_dsd2(R qc, R& nc, R& mu_c, R rho, R& l
     m = vmax(m, R(2));
     m = vmin(m, R(15));
     mu_c = m;
-    lamc = m_cbrt(m_div(R(CONS1) * nc * (m + R(3)) * (m + R(2)) * (m + R(1)), qc));
+    lamc = m_cbrt(m_div<D>(R(CONS1) * nc * (m + R(3)) * (m + R(2)) * (m + R(1)), qc));
     const R lammin = (m + R(1)) * R(2.5e+4);
     const R lammax = (m + R(1)) * R(1.e+6);
     const bool lt = lamc < lammin, gt = lamc > lammax;
     if (lt) lamc = lammin;
     if (gt) lamc = lammax;
     if (lt || gt)
-      nc = m_div(R(6) * (lamc * lamc * lamc) * qc, R(Pi) * R(RHO_H2O) * (m + R(3)) * (m + R(2)) * (m + R(1)));
+      nc = m_div<D>(R(6) * (lamc * lamc * lamc) * qc, R(Pi) * R(RHO_H2O) * (m + R(3)) * (m + R(2)) * (m + R(1)));
   }
 }
 
 // get_rain_dsd2, P3I/p3_dsd2_impl.hpp:73-126
-template <class R>
+template <class R, Div D = DIV_INF>
 __device__ __forceinline__ void get_rain_dsd2(const Runtime& rt, R qr, R& nr, R& mu_r, R& lamr) {
   lamr = R(0);
   if (qr >= R(QSMALL)) {
     const R nr_lim = vmax(nr, R(NSMALL));
     mu_r = R(rt.constant_mu_rain);
     const R f = R(CONS1) * (mu_r + R(3)) * (mu_r + R(2)) * (mu_r + R(1));
-    lamr = m_cbrt(m_div(f * nr_lim, qr));
+    lamr = m_cbrt(m_div<D>(f * nr_lim, qr));
     const R lammax = (mu_r + R(1.)) * R(1.e+5);
     const R lammin = (mu_r + R(1.)) * R(500);
     const bool lt = lamr < lammin, gt = lamr > lammax;
@@ -471,17 +474,17 @@ __device__ __forceinline__ void get_rain_dsd2(const Runtime& rt, R qr, R& nr, R&
     if (lt || gt) {
       if (lt) lamr = lammin;
       if (gt) lamr = lammax;
-      nr = m_div(lamr * lamr * lamr * qr, f);
+      nr = m_div<D>(lamr * lamr * lamr * qr, f);
     }
   }
 }
 
 // calc_bulk_rho_rime, P3I/p3_ice_sed_impl.hpp:14-64
-template <class R>
+template <class R, Div D = DIV_INF>
 __device__ __forceinline__ R calc_bulk_rho_rime(const Runtime& rt, R qi_tot, R& qi_rim, R& bi_rim) {
   R rho_rime = R(0);
   const bool gt = bi_rim >= R(BSMALL), lt = bi_rim < R(BSMALL);
-  if (gt) rho_rime = m_div(qi_rim, bi_rim);
+  if (gt) rho_rime = m_div<D>(qi_rim, bi_rim);
   const bool lt_min = rho_rime < R(rt.min_rime_rho), gt_max = rho_rime > R(rt.max_rime_rho);
   if (gt && lt_min) rho_rime = R(rt.min_rime_rho);
   if (gt && gt_max) rho_rime = R(rt.max_rime_rho);
@@ -492,7 +495,7 @@ __device__ __forceinline__ R calc_bulk_rho_rime(const Runtime& rt, R qi_tot, R& 
   // again with qi_rim = qi_tot when the rime exceeds the total; the second
   // overrides the first, and `lt` excludes both, so one division serves.
   const bool over = qi_rim > qi_tot && rho_rime > R(0);
-  if (over || clamped) bi_rim = m_div(over ? qi_tot : qi_rim, rho_rime);
+  if (over || clamped) bi_rim = m_div<D>(over ? qi_tot : qi_rim, rho_rime);
   if (over) qi_rim = qi_tot;
   if (lt || qi_rim < R(QSMALL)) { qi_rim = R(0); bi_rim = R(0); }
   return rho_rime;
@@ -519,7 +522,7 @@ __device__ __forceinline__ Incld incloud(double qc, double qr, double qi, double
 // impose_max_total_ni, P3I/p3_impose_max_total_ni_impl.hpp:9-26
 template <class R>
 __device__ __forceinline__ void impose_max_total_ni(R& ni, R max_total_ni, R inv_rho) {
-  if (ni >= R(1e-20)) ni = ni * vmin(m_div(max_total_ni * inv_rho, ni), R(1));
+  if (ni >= R(1e-20)) ni = ni * vmin(m_div<DIV_INF>(max_total_ni * inv_rho, ni), R(1));
 }
 
 }  // namespace p3d

@@ -139,12 +139,29 @@ template <class R, int L> constexpr int ice_rec_len() { return ice_rec_dif<R, L>
 template <class R, int L> constexpr int ice_lds_stride() { return ice_rec_len<R, L>() + (sizeof(R) == 8 ? 2 : 0); }
 template <class R, int L> constexpr int ice_lds_len() { return kIceCells * ice_lds_stride<R, L>(); }
 
-// An in-cloud value q / cf after the first substep.  In FP64 the reciprocal
+// In-cloud values q / cf of a level after the first substep.  In FP64 the reciprocal
 // rcf = p3m_recip(cf) is formed once per level and run (cf does not change over
 // the substeps): four instructions instead of a division's thirteen issue
-// slots, for up to four fields per level and substep.
-__device__ __forceinline__ double incloud_div(double q, double cf, double rcf) { return p3m_div_y(q, cf, rcf); }
-__device__ __forceinline__ float incloud_div(float q, float cf, float) { return q / cf; }
+// slots, for up to four fields per level and substep.  A run with cloud fractions too
+// small for that (below kTinyFrac) takes a uniform branch to general divisions: 2 % of
+// sedimentation at 2700 x 72, 1 % at 16384 x 128.  (A second substep loop for such runs
+// spilled, 92 -> 130 us at 2700 x 72; out of line it took the stack with it.)
+constexpr double kTinyFrac = 0x1p-900;
+template <int N>
+__device__ __forceinline__ void incloud_div(const double (&q)[N], double cf, double rcf, bool tiny, double (&v)[N]) {
+  if (__builtin_expect(tiny, 0)) {
+#pragma unroll
+    for (int f = 0; f < N; ++f) v[f] = p3m_div_any(q[f], cf);
+  } else {
+#pragma unroll
+    for (int f = 0; f < N; ++f) v[f] = p3m_div_y(q[f], cf, rcf);
+  }
+}
+template <int N>
+__device__ __forceinline__ void incloud_div(const float (&q)[N], float cf, float, bool, float (&v)[N]) {
+#pragma unroll
+  for (int f = 0; f < N; ++f) v[f] = q[f] / cf;
+}
 
 // Per-lane geometry of the owned levels.
 template <int L>
@@ -171,6 +188,7 @@ struct SedRun {
   Geo<L> g;
   double q[NF][L], cf[L], coef[L], cfl_ice[L], pflux[L];
   R rcf[L];  // FP64: p3m_recip(cf)
+  bool tiny;   // FP64: a cloud fraction of the wavefront's columns is below kTinyFrac
   int kbase, k_top, k_bot;
   double dt_left, prt_accum;  // prt_accum: mass through the surface, on the lane owning the lowest level
   int nsub;
@@ -190,6 +208,7 @@ struct SedRun {
     k_top = top;
     kbase = k_top + j * L;
     int my_bot = -1;
+    bool my_tiny = false;
 #pragma unroll
     for (int t = 0; t < L; ++t) {
       const int k = kbase + t;
@@ -198,27 +217,33 @@ struct SedRun {
       const double dz = ok ? p.dz[x] : 1.0;
       const double dp = ok ? p.dpres[x] : 1.0;
       g.rho[t] = air_density(dp, dz);
-      g.inv_rho[t] = p3m_div(1.0, g.rho[t]);
-      g.inv_dz[t] = p3m_div(1.0, dz);
+      g.inv_rho[t] = p3m_div_inf(1.0, g.rho[t]);
+      g.inv_dz[t] = p3m_div_inf(1.0, dz);
 #pragma unroll
       for (int f = 0; f < NF; ++f) q[f][t] = ok ? fld[f][x] : 0.0;
       cf[t] = ok ? cfp[x] : 1.0;
       rcf[t] = sizeof(R) == 8 ? R(p3m_recip(cf[t])) : R(0);
       coef[t] = ok ? p.sc(coef_f, i, ok ? k : 0) : 0.0;
       cfl_ice[t] = (SP == 2 && ok) ? p.cld_frac_l[x] : 1.0;
+      my_tiny |= m_fabs(cf[t]) < kTinyFrac && cf[t] != 0;  // (0 is the fixup's)
       pflux[t] = 0;
       // find_bottom, P3I/p3_find_impl.hpp:52-92 (find_top gave k_top)
       if (ok && q[0][t] >= QSMALL) my_bot = k;
     }
     k_bot = grp_max<LPC>(my_bot);
+    tiny = sizeof(R) == 8 && __any(my_tiny);
     dt_left = p.dt;
     prt_accum = 0;
     nsub = 0;
   }
 
-  // One substep; `first` (the first substep: in-cloud values limited) is a
-  // constant after inlining wherever the caller knows it.
-  __device__ __forceinline__ void substep(const KParams& p, int j, bool first, const R* __restrict__ ice_tab) {
+  // One substep.  FIRST: the first one, which limits the in-cloud mixing ratios (a
+  // template parameter, so that neither kind carries the other's branches) but not the
+  // numbers, so that its quotients may overflow.
+  template <bool FIRST>
+  __device__ __forceinline__ void substep(const KParams& p, int j, const R* __restrict__ ice_tab) {
+    constexpr bool first = FIRST;
+    constexpr Div D = FIRST ? DIV_INF : DIV;
     const int nlev = p.nlev, kbot = nlev - 1;
     const Runtime& rt = p.rt;
     const int nfield = SP == 2 ? 4 : (SP == 1 ? 2 : (p.predictNc ? 2 : 1));
@@ -238,16 +263,18 @@ struct SedRun {
           const R qc = R(q[0][t]), nc = R(q[1][t]);
           R qc_incld, nc_incld;
           if (first) {
-            const R icfl = m_div(R(1), cfl);
+            const R icfl = m_div<D>(R(1), cfl);
             if (q[0][t] >= QSMALL) { qc_incld = vmin(qc * icfl, R(incloud_limit)); nc_incld = vmax(nc * icfl, R(0)); }
             else { qc_incld = 0; nc_incld = 0; }
           } else {
-            qc_incld = incloud_div(qc, cfl, rcf[t]);
-            nc_incld = incloud_div(nc, cfl, rcf[t]);
+            const R in[2] = {qc, nc};
+            R v[2];
+            incloud_div(in, cfl, rcf[t], tiny, v);
+            qc_incld = v[0]; nc_incld = v[1];
           }
           if (qc_incld > R(QSMALL)) {
             R ncr = nc_incld, mu_c, lamc;
-            get_cloud_dsd2<R>(qc_incld, ncr, mu_c, R(rho), lamc);
+            get_cloud_dsd2<R, D>(qc_incld, ncr, mu_c, R(rho), lamc);
             q[1][t] = double(ncr) * cf[t];
             const R dum = m_div(R(1), m_pow(lamc, R(bcn)));
             const R acn = R(coef[t]);
@@ -260,16 +287,18 @@ struct SedRun {
           const R qr = R(q[0][t]), nr = R(q[1][t]);
           R qr_incld, nr_incld;
           if (first) {
-            const R icfr = m_div(R(1), cfr);
+            const R icfr = m_div<D>(R(1), cfr);
             if (q[0][t] >= QSMALL) { qr_incld = vmin(qr * icfr, R(precip_limit)); nr_incld = vmax(nr * icfr, R(0)); }
             else { qr_incld = 0; nr_incld = 0; }
           } else {
-            qr_incld = incloud_div(qr, cfr, rcf[t]);
-            nr_incld = incloud_div(nr, cfr, rcf[t]);
+            const R in[2] = {qr, nr};
+            R v[2];
+            incloud_div(in, cfr, rcf[t], tiny, v);
+            qr_incld = v[0]; nr_incld = v[1];
           }
           if (qr_incld > R(QSMALL)) {
             R nrr = nr_incld, mu_r = 0, lamr;
-            get_rain_dsd2<R>(rt, qr_incld, nrr, mu_r, lamr);
+            get_rain_dsd2<R, D>(rt, qr_incld, nrr, mu_r, lamr);
             const Tab3<R> t3 = lookup3<R>(mu_r, lamr);
             const R rhofacr = R(coef[t]);
             R v[2];  // vm, vn
@@ -284,25 +313,25 @@ struct SedRun {
           const R qi = R(q[0][t]), ni = R(q[1][t]), qm = R(q[2][t]), bm = R(q[3][t]);
           R qi_incld, ni_incld, qm_incld, bm_incld;
           if (first) {
-            const R icfi = m_div(R(1), cfi), icfl = m_div(R(1), R(cfl_ice[t]));
+            const R icfi = m_div<D>(R(1), cfi), icfl = m_div<D>(R(1), R(cfl_ice[t]));
             if (q[0][t] >= QSMALL) { qi_incld = vmin(qi * icfi, R(incloud_limit)); ni_incld = vmax(ni * icfi, R(0)); }
             else { qi_incld = 0; ni_incld = 0; }
             if (q[0][t] >= QSMALL && q[2][t] >= QSMALL) { qm_incld = qm * icfi; bm_incld = vmin(vmax(bm * icfl, R(0)), R(incloud_limit)); }
             else { qm_incld = 0; bm_incld = 0; }
           } else {
-            qi_incld = incloud_div(qi, cfi, rcf[t]);
-            ni_incld = incloud_div(ni, cfi, rcf[t]);
-            qm_incld = incloud_div(qm, cfi, rcf[t]);
-            bm_incld = incloud_div(bm, cfi, rcf[t]);
+            const R in[4] = {qi, ni, qm, bm};
+            R v[4];
+            incloud_div(in, cfi, rcf[t], tiny, v);
+            qi_incld = v[0]; ni_incld = v[1]; qm_incld = v[2]; bm_incld = v[3];
           }
           if (qi_incld > R(QSMALL)) {
             R nir = vmax(ni_incld, R(NSMALL));
             R qmr = qm_incld, bmr = bm_incld;
             const R qir = qi_incld;
-            const R rhop = calc_bulk_rho_rime<R>(rt, qir, qmr, bmr);
+            const R rhop = calc_bulk_rho_rime<R, D>(rt, qir, qmr, bmr);
             q[2][t] = double(qmr) * cf[t];
             q[3][t] = double(bmr) * cf[t];
-            const TabIce<R> ti = lookup_ice<R>(qir, nir, qmr, rhop);
+            const TabIce<R> ti = lookup_ice<R, D>(qir, nir, qmr, rhop);
             // quantities 0, 1, 6, 7 of the records (in FP64 as two halves, which bounds the registers)
             R v[4];
             if constexpr (sizeof(R) == 4) {
@@ -410,13 +439,13 @@ __device__ __forceinline__ void sediment_run(const KParams& p, int i, int j, int
                                           int& nsub_out, unsigned& err, const R* __restrict__ ice_tab) {
   SedRun<SP, R, LPC, L, DIF, STRIDE> r;
   r.load(p, i, j, k_top);
-  if (r.dt_left > dt_left_tol) r.substep(p, j, true, ice_tab);
+  if (r.dt_left > dt_left_tol) r.template substep<true>(p, j, ice_tab);
 #pragma unroll 1
   while (r.dt_left > dt_left_tol) {
     // The substep count is bounded by the CFL number (a few hundred at most for
     // physical inputs); the cap only guarantees termination for corrupt inputs.
     if (r.nsub >= kMaxSubsteps) { err |= ERR_SUBSTEP_LIMIT; break; }
-    r.substep(p, j, false, ice_tab);
+    r.template substep<false>(p, j, ice_tab);
   }
   r.store(p, i);
   prt = grp_sumd<LPC>(r.prt_accum);  // only the lane owning kbot accumulated
@@ -544,11 +573,10 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
     const double rho = air_density(dp, dz);
     // cloud
     if (qc >= QSMALL) {
-      const double rcfl = p3m_recip(cfl);
-      R ncr = R(p3m_div_y(nc, cfl, rcfl)), mu_c, lamc;
-      get_cloud_dsd2<R>(R(p3m_div_y(qc, cfl, rcfl)), ncr, mu_c, R(rho), lamc);
+      R ncr = R(p3m_div_any(nc, cfl)), mu_c, lamc;
+      get_cloud_dsd2<R>(R(p3m_div_any(qc, cfl)), ncr, mu_c, R(rho), lamc);
       nc = double(ncr) * cfl;
-      reff_c = double(m_div(R(0.5) * (mu_c + R(3)), lamc));
+      reff_c = double(m_div<DIV_INF>(R(0.5) * (mu_c + R(3)), lamc));
     } else {
       qv = qv + qc;
       th = th - inv_exner * qc * latvap * inv_cp;
@@ -557,9 +585,8 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
     }
     // rain
     if (qr >= QSMALL) {
-      const double rcfr = p3m_recip(cfr);
-      R nrr = R(p3m_div_y(nr, cfr, rcfr)), mu_r = 0, lamr;
-      get_rain_dsd2<R>(rt, R(p3m_div_y(qr, cfr, rcfr)), nrr, mu_r, lamr);
+      R nrr = R(p3m_div_any(nr, cfr)), mu_r = 0, lamr;
+      get_rain_dsd2<R>(rt, R(p3m_div_any(qr, cfr)), nrr, mu_r, lamr);
       nr = double(nrr) * cfr;
       reff_r = double(m_div(R(1.5), lamr));
     } else {
@@ -570,12 +597,11 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
     }
     // ice
     if (qi >= QSMALL) {
-      const double inv_rho = p3m_div(1.0, rho);
+      const double inv_rho = p3m_div_inf(1.0, rho);
       ni = vmax(ni, NSMALL);
-      const double rcfi = p3m_recip(cfi);
-      const double qi_incld = p3m_div_y(qi, cfi, rcfi);
-      double ni_incld = p3m_div_y(ni, cfi, rcfi);
-      double qm_incld = p3m_div_y(qm, cfi, rcfi), bm_incld = p3m_div_y(bm, cfi, rcfi);
+      const double qi_incld = p3m_div_any(qi, cfi);
+      double ni_incld = p3m_div_any(ni, cfi);
+      double qm_incld = p3m_div_any(qm, cfi), bm_incld = p3m_div_any(bm, cfi);
       R qmr = R(qm_incld), bmr = R(bm_incld);
       const R rhop = calc_bulk_rho_rime<R>(rt, R(qi_incld), qmr, bmr);
       qm_incld = double(qmr); bm_incld = double(bmr);
@@ -619,8 +645,8 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
     const Amble& a = p.amble;
     const double dp = a.dp_wet[x], dp_dry = p.dpres[x];
     const double T_before = a.T_mid[x];
-    const double rdp = p3m_recip(dp);
-    auto to_wet = [&](double q) { return p3m_div_y(q * dp_dry, dp, rdp); };
+    const Ratio wet(dp_dry, dp);
+    auto to_wet = [&](double q) { return wet.of(q); };
     double T = to_wet(th * exner_function(a.p_mid[x]) - T_before);
     T += T_before;
     a.T_mid[x] = T;

@@ -238,6 +238,9 @@ __device__ __forceinline__ void front_level(const KParams& p, int k, int i, cons
   qv = vmax(qv, 0.0);
   const double exner = p3m_div_inf(1.0, inv_exner);
   double T_atm = th * exner;
+  // The mixed form refuses an inverse Exner function of 0 (an array never filled), as it
+  // did when its divisions made T NaN of it; in FP64 T is infinite, which passes.
+  if (sizeof(R) == 4 && !(m_fabs(exner) < p3m_inf())) err |= ERR_BAD_TEMPERATURE;
   const double rho = air_density(dpres, dz);
   const double inv_rho = p3m_div_inf(1.0, rho);
   const double T_first = T_atm;

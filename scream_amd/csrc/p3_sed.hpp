@@ -139,29 +139,28 @@ template <class R, int L> constexpr int ice_rec_len() { return ice_rec_dif<R, L>
 template <class R, int L> constexpr int ice_lds_stride() { return ice_rec_len<R, L>() + (sizeof(R) == 8 ? 2 : 0); }
 template <class R, int L> constexpr int ice_lds_len() { return kIceCells * ice_lds_stride<R, L>(); }
 
-// In-cloud values q / cf of a level after the first substep.  In FP64 the reciprocal
-// rcf = p3m_recip(cf) is formed once per level and run (cf does not change over
-// the substeps): four instructions instead of a division's thirteen issue
-// slots, for up to four fields per level and substep.  A run with cloud fractions too
-// small for that (below kTinyFrac) takes a uniform branch to general divisions: 2 % of
-// sedimentation at 2700 x 72, 1 % at 16384 x 128.  (A second substep loop for such runs
-// spilled, 92 -> 130 us at 2700 x 72; out of line it took the stack with it.)
+// An in-cloud value q / cf after the first substep.  In FP64 the reciprocal is formed
+// once per level and run (cf does not change over the substeps): five instructions
+// instead of a division's thirteen issue slots, for up to four fields per level and
+// substep.  So that any cf divides as it should, den is cf times 2^up, up > 0 where cf
+// is tiny, and the quotient is scaled back, exactly or to infinity.  (Without the last
+// step sedimentation and part 3 take 92.5 us at 2700 x 72 and 266 at 16384 x 128, with it
+// 93.3 and 270; with a uniform branch to general divisions instead 95.5 and 270.  A
+// second substep loop for such runs spilled: 130 us at 2700 x 72.)
 constexpr double kTinyFrac = 0x1p-900;
-template <int N>
-__device__ __forceinline__ void incloud_div(const double (&q)[N], double cf, double rcf, bool tiny, double (&v)[N]) {
-  if (__builtin_expect(tiny, 0)) {
-#pragma unroll
-    for (int f = 0; f < N; ++f) v[f] = p3m_div_any(q[f], cf);
-  } else {
-#pragma unroll
-    for (int f = 0; f < N; ++f) v[f] = p3m_div_y(q[f], cf, rcf);
+struct Frac {
+  double den, rden;  // rden: p3m_recip(den)
+  int up;
+  __device__ __forceinline__ void set(double cf) {
+    up = m_fabs(cf) < kTinyFrac ? 300 : 0;
+    den = __builtin_amdgcn_ldexp(cf, up);
+    rden = p3m_recip(den);
   }
+};
+__device__ __forceinline__ double incloud_div(double q, double, const Frac& f) {
+  return __builtin_amdgcn_ldexp(p3m_div_y(q, f.den, f.rden), f.up);
 }
-template <int N>
-__device__ __forceinline__ void incloud_div(const float (&q)[N], float cf, float, bool, float (&v)[N]) {
-#pragma unroll
-  for (int f = 0; f < N; ++f) v[f] = q[f] / cf;
-}
+__device__ __forceinline__ float incloud_div(float q, float cf, const Frac&) { return q / cf; }
 
 // Per-lane geometry of the owned levels.
 template <int L>
@@ -187,8 +186,7 @@ struct SedRun {
   static constexpr int NF = SP == 2 ? 4 : 2;  // fields held (cloud always holds nc: its DSD rewrites it)
   Geo<L> g;
   double q[NF][L], cf[L], coef[L], cfl_ice[L], pflux[L];
-  R rcf[L];  // FP64: p3m_recip(cf)
-  bool tiny;   // FP64: a cloud fraction of the wavefront's columns is below kTinyFrac
+  Frac frac[L];  // FP64
   int kbase, k_top, k_bot;
   double dt_left, prt_accum;  // prt_accum: mass through the surface, on the lane owning the lowest level
   int nsub;
@@ -208,7 +206,6 @@ struct SedRun {
     k_top = top;
     kbase = k_top + j * L;
     int my_bot = -1;
-    bool my_tiny = false;
 #pragma unroll
     for (int t = 0; t < L; ++t) {
       const int k = kbase + t;
@@ -222,16 +219,14 @@ struct SedRun {
 #pragma unroll
       for (int f = 0; f < NF; ++f) q[f][t] = ok ? fld[f][x] : 0.0;
       cf[t] = ok ? cfp[x] : 1.0;
-      rcf[t] = sizeof(R) == 8 ? R(p3m_recip(cf[t])) : R(0);
+      if (sizeof(R) == 8) frac[t].set(cf[t]);
       coef[t] = ok ? p.sc(coef_f, i, ok ? k : 0) : 0.0;
       cfl_ice[t] = (SP == 2 && ok) ? p.cld_frac_l[x] : 1.0;
-      my_tiny |= m_fabs(cf[t]) < kTinyFrac && cf[t] != 0;  // (0 is the fixup's)
       pflux[t] = 0;
       // find_bottom, P3I/p3_find_impl.hpp:52-92 (find_top gave k_top)
       if (ok && q[0][t] >= QSMALL) my_bot = k;
     }
     k_bot = grp_max<LPC>(my_bot);
-    tiny = sizeof(R) == 8 && __any(my_tiny);
     dt_left = p.dt;
     prt_accum = 0;
     nsub = 0;
@@ -267,10 +262,8 @@ struct SedRun {
             if (q[0][t] >= QSMALL) { qc_incld = vmin(qc * icfl, R(incloud_limit)); nc_incld = vmax(nc * icfl, R(0)); }
             else { qc_incld = 0; nc_incld = 0; }
           } else {
-            const R in[2] = {qc, nc};
-            R v[2];
-            incloud_div(in, cfl, rcf[t], tiny, v);
-            qc_incld = v[0]; nc_incld = v[1];
+            qc_incld = incloud_div(qc, cfl, frac[t]);
+            nc_incld = incloud_div(nc, cfl, frac[t]);
           }
           if (qc_incld > R(QSMALL)) {
             R ncr = nc_incld, mu_c, lamc;
@@ -291,10 +284,8 @@ struct SedRun {
             if (q[0][t] >= QSMALL) { qr_incld = vmin(qr * icfr, R(precip_limit)); nr_incld = vmax(nr * icfr, R(0)); }
             else { qr_incld = 0; nr_incld = 0; }
           } else {
-            const R in[2] = {qr, nr};
-            R v[2];
-            incloud_div(in, cfr, rcf[t], tiny, v);
-            qr_incld = v[0]; nr_incld = v[1];
+            qr_incld = incloud_div(qr, cfr, frac[t]);
+            nr_incld = incloud_div(nr, cfr, frac[t]);
           }
           if (qr_incld > R(QSMALL)) {
             R nrr = nr_incld, mu_r = 0, lamr;
@@ -319,10 +310,10 @@ struct SedRun {
             if (q[0][t] >= QSMALL && q[2][t] >= QSMALL) { qm_incld = qm * icfi; bm_incld = vmin(vmax(bm * icfl, R(0)), R(incloud_limit)); }
             else { qm_incld = 0; bm_incld = 0; }
           } else {
-            const R in[4] = {qi, ni, qm, bm};
-            R v[4];
-            incloud_div(in, cfi, rcf[t], tiny, v);
-            qi_incld = v[0]; ni_incld = v[1]; qm_incld = v[2]; bm_incld = v[3];
+            qi_incld = incloud_div(qi, cfi, frac[t]);
+            ni_incld = incloud_div(ni, cfi, frac[t]);
+            qm_incld = incloud_div(qm, cfi, frac[t]);
+            bm_incld = incloud_div(bm, cfi, frac[t]);
           }
           if (qi_incld > R(QSMALL)) {
             R nir = vmax(ni_incld, R(NSMALL));

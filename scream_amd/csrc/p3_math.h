@@ -128,12 +128,25 @@ P3M_FN double p3m_scale2(double x, int k) {
 #endif
 }
 
+/* The integer part of x.  On the device any x, saturating, and 0 for NaN, as v_cvt_i32
+ * converts (in C++ a cast of what int does not hold is undefined); on the CPU the
+ * callers keep x in range. */
+P3M_FN int p3m_int(double x) {
+#if P3M_DEVICE
+  int k;
+  asm("v_cvt_i32_f64 %0, %1" : "=v"(k) : "v"(x));
+  return k;
+#else
+  return (int)x;
+#endif
+}
+
 /* exp of a finite x in about [-746, 710] (NaN gives NaN): Cody-Waite reduction
  * x = k ln2 + r, |r| <= ln2/2, then the Taylor series of e^r to r^13
  * (truncation < 1e-17), evaluated with fma. */
 P3M_FN double p3m_exp_core(double x) {
   const double t = x * P3M_INVLN2;
-  const int k = (int)(t + (t >= 0 ? 0.5 : -0.5));
+  const int k = p3m_int(t + (t >= 0 ? 0.5 : -0.5));
   const double kd = (double)k;
   double r = fma(-kd, P3M_LN2_HI, x);
   r = fma(-kd, P3M_LN2_LO, r);
@@ -157,7 +170,7 @@ P3M_FN double p3m_exp_core(double x) {
 P3M_FN double p3m_exp(double x) {
 #if P3M_DEVICE
   /* the range ends by selects: branches would end the basic blocks that the
-   * compiler schedules across (the float to int conversion saturates) */
+   * compiler schedules across */
   double e = p3m_exp_core(x);
   e = x > 709.782712893384 ? p3m_inf() : e;
   return x < -745.1332191019412 ? 0.0 : e;

@@ -418,28 +418,19 @@ __device__ __forceinline__ bool pw_point(const KParams& p, int tile, int& i, int
 }
 
 // ORs `bit` into the status word of column i for every lane whose `set` is
-// true, one atomic per column and wavefront.  Level-major lanes hold distinct
-// columns.  Column-major lanes hold runs of one column's consecutive levels:
-// under PW_RUNS lane l's run starts min(l, k) lanes below it, under PW_BLOCKS
-// the runs are the aligned groups of 8 lanes; the lowest lane of a run with
-// `set` makes the atomic.  Every lane of the wavefront that is still running
-// must call this.
-template <int MAP>
-__device__ __forceinline__ void colstat_or(const KParams& p, int i, int k, bool set, int bit) {
+// true, one atomic per column and wavefront, on the points of pw_point<PW_BLOCKS>.
+// Level-major lanes hold distinct columns; column-major the aligned groups of 8
+// lanes hold one column's levels, and the lowest lane of a group with `set` makes
+// the atomic.  Every lane of the wavefront that is still running must call this.
+__device__ __forceinline__ void colstat_or(const KParams& p, int i, bool set, int bit) {
   if (!p.colmajor) {
     if (set) atomicOr(&p.colstat[i], bit);
     return;
   }
   const unsigned long long m = __ballot(set);
   const int l = threadIdx.x & 63;
-  unsigned long long run_below;
-  if constexpr (MAP == PW_RUNS) {
-    const int below = k < l ? k : l;
-    run_below = ((1ull << l) - 1) ^ ((1ull << (l - below)) - 1);
-  } else {
-    run_below = (0xFFull << (l & ~7)) & ((1ull << l) - 1);
-  }
-  if (set && !(m & run_below)) atomicOr(&p.colstat[i], bit);
+  const unsigned long long below = (0xFFull << (l & ~7)) & ((1ull << l) - 1);
+  if (set && !(m & below)) atomicOr(&p.colstat[i], bit);
 }
 
 // Stores where the points of pw_point<PW_BLOCKS> hold species sp, from the ballot
@@ -581,8 +572,8 @@ __device__ __forceinline__ void front_tile(const KParams& p, int tile, double* s
   int stat = 0;
   front_level<R>(p, k, i, Pt{s_lds + threadIdx.x}, stat, err);
   if (p.track()) {
-    colstat_or<PW_BLOCKS>(p, i, k, (stat & kStatusPart1) != 0, kStatusPart1);
-    colstat_or<PW_BLOCKS>(p, i, k, (stat & kStatusPart2) != 0, kStatusPart2);
+    colstat_or(p, i, (stat & kStatusPart1) != 0, kStatusPart1);
+    colstat_or(p, i, (stat & kStatusPart2) != 0, kStatusPart2);
     if (k == 0 && p.dbg_check) p.dbg_check[i] = 0;  // part 3 ORs the column's check_values flags
   }
   if (p.ordered()) {

@@ -172,11 +172,14 @@ template <class R> struct Tab3 { int dumii, dumjj; R rdumii, rdumjj; };
 __device__ __forceinline__ double m_log10_pos(double x) { return p3m_log10_pos(x); }
 __device__ __forceinline__ float m_log10_pos(float x) { return m_log10(x); }
 
-// lookup_ice, P3I/p3_table_ice_impl.hpp:80-138 (qi and ni are positive)
-template <class R, Div D = DIV_INF>
+// lookup_ice, P3I/p3_table_ice_impl.hpp:80-138.  POSITIVE: qi and ni are, by the
+// caller's limits; part 3's ni, limited by the air density, is not in a layer of
+// negative thickness.
+template <class R, Div D = DIV_INF, bool POSITIVE = true>
 __device__ __forceinline__ TabIce<R> lookup_ice(R qi, R ni, R qm, R rhop) {
   TabIce<R> t;
-  t.dum1 = (m_log10_pos(m_div<D>(qi, ni)) + R(18)) * R(lookup_table_1a_dum1_c) - R(10);
+  const R size = m_div<D>(qi, ni);
+  t.dum1 = ((POSITIVE ? m_log10_pos(size) : m_log10(size)) + R(18)) * R(lookup_table_1a_dum1_c) - R(10);
   t.dumi = (int)t.dum1;
   t.dum1 = vmin(t.dum1, R(isize));
   t.dum1 = vmax(t.dum1, R(1.));

@@ -599,7 +599,7 @@ __device__ __forceinline__ void part3_level(const KParams& p, int k, int i, bool
       qm = qm_incld * cfi;
       bm = bm_incld * cfi;
       impose_max_total_ni<double>(ni_incld, rt.max_total_ni, inv_rho);
-      const TabIce<R> ti = lookup_ice<R>(R(qi_incld), R(ni_incld), R(qm_incld), rhop);
+      const TabIce<R> ti = lookup_ice<R, DIV_INF, false>(R(qi_incld), R(ni_incld), R(qm_incld), rhop);
       if (p.dbg_ice_idx) p.dbg_ice_idx[x] = ti.dumjj * 10000 + ti.dumii * 100 + ti.dumi;
       R v[4];  // quantities 5, 6, 7, 11
       apply_table_ice_rec<4, 4, R>(TabOf<R>::get(p.tab).ice_p3, ti, v);

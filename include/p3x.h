@@ -56,7 +56,8 @@ enum {
   P3X_ERR_TABLE_VERSION = 3,/* table header is not "VERSION 4.1.1"                 */
   P3X_ERR_DEVICE = 4,       /* a HIP runtime call failed                           */
   P3X_ERR_TEMPERATURE = 5,  /* T <= 0 or NaN reached the saturation functions;     */
-                            /* the reference aborts here (physics_saturation_impl.hpp:14-36) */
+                            /* the reference aborts here (physics_saturation_impl.hpp:14-36); */
+                            /* mixed form: also 1 / inv_exner infinite            */
   P3X_ERR_NO_MEMORY = 6,    /* device allocation failed                            */
   P3X_ERR_SUBSTEPS = 7,     /* a sedimentation loop hit the 100000-substep cap     */
   P3X_ERR_BUDGET = 8,       /* served form: a member does not fit the HBM budget   */

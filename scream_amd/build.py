@@ -31,8 +31,9 @@ SOURCES = [(f"p3_kernel_{prec}.hip", lpc) for prec in ("fp64", "mixed") for lpc 
 
 # Extra flags per translation unit.  The mixed-precision form may use the
 # hardware-backed FP32 division, square root and transcendental sequences
-# (a few ulp instead of correctly rounded); FP64 arithmetic is not affected by
-# these flags, and the FP64 form is a translation unit of its own.
+# (a few ulp instead of correctly rounded).  Of its FP64 arithmetic they change a plain
+# a / b, which loses its scaling and fixup (p3_math.h writes its divisions out); the
+# FP64 form is a translation unit of its own.
 FILE_FLAGS: dict[str, list[str]] = {
     "p3_kernel_mixed.hip": ["-fno-hip-fp32-correctly-rounded-divide-sqrt", "-fapprox-func"],
 }

@@ -78,9 +78,10 @@ struct KParams {
   // skipped column leaves as they were.
   __host__ __device__ __forceinline__ bool track() const { return dbg_status || dbg_check || !exch_zero; }
   // Sedimentation with several columns per wavefront takes them in the order of
-  // p3_order_kernel.  Not with the status words (a skipped column may hold
-  // species), and only where the words and lists fit their scratch fields and the
-  // counts their 21 bits each.
+  // p3_order_kernel.  Not with the status words: the lists would hold there too (a
+  // column that the reference skips has none of the species), but the gain is measured
+  // without them.  And only where the words and lists fit their scratch fields and
+  // the counts their 21 bits each.
   __host__ __device__ __forceinline__ bool ordered() const {
     return !keep_order && !track() && ncol >= 64 && ncol < 1 << 21 && nlev >= 16;
   }
@@ -154,10 +155,12 @@ template <class R> struct RainOf {
 //    hydrometeors after part 2 makes its column run.
 //
 // What part 2 needs later than it is computed stays in LDS (s), not in
-// registers: 26 doubles per point.  Without that part 2 alone spilled at two
-// wavefronts per SIMD in FP64 and could not run at three in the mixed form.
+// registers: 28 doubles per point in FP64, 26 in the mixed form.  Without that part 2
+// alone spilled at two wavefronts per SIMD in FP64 and could not run at three in the
+// mixed form.
 //
-// Bound by VALU issue: 66 % busy in FP64, 91 % in the mixed form.  As kernels of
+// Bound by the latency of its loads and table gathers at two and three wavefronts per
+// SIMD: the VALU is busy 52 % of the time in FP64, 74 % in the mixed form.  As kernels of
 // their own, part 1 (at the HBM rate) wrote seven scratch fields and part 2
 // (43 % busy, waiting on loads) read them and the state again.  Together, at
 // 21600 x 72 FP64 48 + 187 -> 225 us, at 16384 x 128 mixed 67 + 189 -> 195 us,
@@ -584,10 +587,10 @@ __device__ __forceinline__ void front_tile(const KParams& p, int tile, double* s
   if (err) report_errors(p.err, err);
 }
 
-// Wavefronts per SIMD the front kernel is compiled for.  Two in FP64 (248
+// Wavefronts per SIMD the front kernel is compiled for.  Two in FP64 (246
 // VGPRs; at three it spilled 89 of them: 276 against 225 us at 21600 x 72), three
-// in the mixed form (165 VGPRs).  The LDS slots are 52 KB per block of four
-// wavefronts, so three blocks fit a CU.
+// in the mixed form (164 VGPRs).  A block of four wavefronts holds 52 KB of LDS slots
+// in the mixed form, of which three blocks fit a CU, and 56 KB in FP64, of which two.
 template <class R> constexpr int kFrontWaves = sizeof(R) == 8 ? 2 : 3;
 
 template <class R>

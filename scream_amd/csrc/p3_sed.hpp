@@ -111,8 +111,8 @@ __device__ __forceinline__ double grp_below(double v, int j) {
 
 // Wavefronts per SIMD the sedimentation kernels are compiled for: up to 5
 // levels per lane two fit (256 registers); the FP64 ice group at up to 3
-// levels per lane runs at three (159 registers at 3 levels, 135 at 2; at three:
-// 736 -> 714 us at 21600 x 72; the FP32 ice group holds 127 registers anyway).
+// levels per lane runs at three (167 registers at 3 levels, 138 at 2; at three:
+// 736 -> 714 us at 21600 x 72).
 template <class R, int G, int L> constexpr int sed_waves_per_simd() {
   return (G == SED_ICE && sizeof(R) == 8 && L <= 3) ? 3 : (L <= 5 ? 2 : 1);
 }
@@ -901,8 +901,8 @@ __global__ __launch_bounds__(64 * WPB, (sed_waves_per_simd<R, G, L>())) void p3_
 // are the same bits.  The kernel is compiled for the ice group's wavefronts
 // per SIMD; the shapes it is launched at are those where the liquid group's
 // code also fits that register budget without a spill (in FP64 not at 3
-// levels per lane, where the ice group runs three wavefronts and the liquid
-// group needs 173 VGPRs).
+// levels per lane, where the ice group runs three wavefronts: the liquid group needed
+// 173 VGPRs of 168 when the line was drawn; a kernel of its own now takes 139 to 143).
 template <class R, int LPC, int L, int WPB>
 __global__ __launch_bounds__(64 * WPB, (sed_waves_per_simd<R, SED_ICE, L>())) void p3_sed_fused_kernel(
     const KParams p, int nb_ice) {

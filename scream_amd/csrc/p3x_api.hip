@@ -151,8 +151,12 @@ int status_of_err(unsigned err) {
 //   mixed 12000 x 50 dt 300   154 / 155 / 160, clear 144 / 145 / 154
 //   mixed 21600 x 72 dt 1800  528 / 572 / 707, clear 457 / 475 / 625
 //   mixed 16384 x 128 dt 300  574 / 533 / 545, clear 540 / 499 / 532
-// but between the two, while 16 lanes leave SIMDs without a wavefront, 32: in the
-// mixed form, and in FP64 where long steps give the groups many substeps:
+// but between the two 32: in the mixed form, until 16 lanes fill two wavefronts per
+// SIMD (8192 columns), and in FP64 where
+// long steps give the groups many substeps and the clear columns are packed, which
+// 32 lanes do from 2050 columns on and 16 from 4100 (p3_kernel_variants.inc).  The
+// FP64 line at 3072 rests on 2700 columns; the sizes measured around it, 2100 and
+// 3400, are ties without clear columns:
 //   FP64  2700 x 72 dt 1800   196 / 198 / 190, clear 196 / 158 / 186
 //   FP64  2700 x 72 dt 300    114 / 126 / 116, clear 113 / 115 / 112
 //   mixed 5400 x 72 dt 1800   206 / 183 / 208, clear 173 / 165 / 192
